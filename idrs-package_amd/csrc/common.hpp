@@ -222,6 +222,13 @@ __device__ inline cplx<R> ldnt(const cplx<R> *p) {
     const R *q = reinterpret_cast<const R *>(p);
     return {__builtin_nontemporal_load(q), __builtin_nontemporal_load(q + 1)};
 }
+// A stream's load under the launch's cache policy: KEEP leaves the lines in
+// L2 and the 256 MB Infinity Cache for the next kernel that reads them.
+template <bool KEEP, class V>
+__device__ inline V ldp(const V *p) {
+    if constexpr (KEEP) return *p;
+    else return ldnt(p);
+}
 // non-temporal stores, for outputs no later kernel reads soon
 template <class V>
 __device__ inline void stnt(V *p, V v) { __builtin_nontemporal_store(v, p); }

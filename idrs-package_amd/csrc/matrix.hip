@@ -352,7 +352,28 @@ static SpmvArgs<VT, T> base_args(const DevMatrix &K, const VT *val) {
     A.sl_ptr = nullptr;
     A.sl_col = nullptr;
     A.pair32 = 0;
+    A.keep = 0;
     return A;
+}
+
+// Cache policy of a product's matrix and P streams.  A matrix that fits the
+// 256 MB Infinity Cache together with the vectors a product touches is read
+// with ordinary loads, so that the next product finds it there (7.2 TB/s, and
+// 12 TB/s out of the L2s when it fits those; HBM gives 6.5 TB/s); a larger one
+// is read non-temporally, so that it does not push out the gathered vector.
+// A chain of DIA products per step, cached against non-temporal: 100^3
+// 11.6 / 14.8 us, 128^3 21.1 / 26.5, 160^3 (295 MB) 45.6 / 49.6, 200^3
+// (576 MB) 116 / 96.
+constexpr size_t KEEP_BYTES = size_t(240) << 20;
+template <class VT, class T>
+static void set_keep(const Operator &op, SpmvArgs<VT, T> &A, int epi, const EpiArgs<T> &E) {
+    const DevMatrix &K = *op.K;
+    size_t b = 0;
+    if (K.fmt != DevFmt::CRS) b = sizeof(VT) * (size_t)op.stored_values();
+    else if (A.pair32) b = 8 * (size_t)K.sell->nent;
+    else b = (sizeof(VT) + sizeof(int)) * (size_t)(A.sl_ptr ? K.sell->nent : K.nnz);
+    const size_t vecs = 4 + (epi == EPI_PDOT ? (size_t)E.prow : 0);
+    A.keep = b + vecs * sizeof(T) * (size_t)K.nrows <= KEEP_BYTES;
 }
 
 // group 1: point the product at the sliced copy of the values it reads
@@ -429,6 +450,7 @@ void op_spmv(const Operator &op, const T *x, T xs, const T *z, T a, T *y, int ep
     const DevMatrix &K = *op.K;
     with_args<T>(op, [&](auto &A) {
         A.x = x; A.xs = xs; A.z = z; A.a = a; A.y = y;
+        set_keep(op, A, epi, E);
         if (tc) dispatch_epi_tiles(K, A, E, epi, *tc, st);
         else dispatch_epi(K, A, E, epi, info, st);
     });
@@ -444,6 +466,7 @@ void op_spmv_cols(const Operator &op, int nc, long ld, const T *x, T xs, const T
         bool done = false;
         with_args<T>(op, [&](auto &A) {
             A.xs = xs;
+            set_keep(op, A, EPI_NONE, none);
             ColArgs<T> C{};
             C.nc = m;
             C.ld = ld;

@@ -48,6 +48,7 @@ struct SpmvArgs {
     const VT *sdiag;
     T seed;
     T *y;
+    int keep;          // cache policy of the matrix and P streams (set_keep)
 };
 
 // y(row) = xs*(acc - seed*x(row)/sdiag(row)) + a*z(row) for the vectors x
@@ -80,7 +81,7 @@ struct ColArgs {
 
 // Operands of one row's epilogue: PC components of its P row (PDOT: this
 // lane's components c, c+step, ...), or r(row) (OMEGA).
-template <class T, int EPI, int PC>
+template <class T, int EPI, int PC, bool KEEP = false>
 __device__ inline void epi_load(T (&pe)[PC], const EpiArgs<T> &E, long row, int c, int step) {
     if constexpr (EPI == EPI_PDOT) {
         const T *p = E.P + row * E.prow;
@@ -90,7 +91,7 @@ __device__ inline void epi_load(T (&pe)[PC], const EpiArgs<T> &E, long row, int 
             if (step == 1 && c == 0 && E.prow == PC) {
 #pragma unroll
                 for (int k = 0; k < PC; k += 2) {
-                    const dbl2_nt v = __builtin_nontemporal_load((const dbl2_nt *)(p + k));
+                    const dbl2_nt v = ldp<KEEP>((const dbl2_nt *)(p + k));
                     pe[k] = v.x;
                     pe[k + 1] = v.y;
                 }
@@ -99,20 +100,20 @@ __device__ inline void epi_load(T (&pe)[PC], const EpiArgs<T> &E, long row, int 
         }
         const int last = E.prow - 1;
 #pragma unroll
-        for (int k = 0; k < PC; k++) pe[k] = ldnt(p + min(c + k * step, last));
+        for (int k = 0; k < PC; k++) pe[k] = ldp<KEEP>(p + min(c + k * step, last));
     } else if constexpr (EPI == EPI_OMEGA) {
         pe[0] = E.r[row];
     }
 }
 
 // The whole P row at p (PDOT with step 1 from component 0): as epi_load.
-template <class T, int PC>
+template <class T, int PC, bool KEEP = false>
 __device__ inline void epi_load_row(T (&pe)[PC], const EpiArgs<T> &E, const T *p) {
     if constexpr (std::is_same<T, double>::value && PC % 2 == 0) {
         if (E.prow == PC) {
 #pragma unroll
             for (int k = 0; k < PC; k += 2) {
-                const dbl2_nt v = __builtin_nontemporal_load((const dbl2_nt *)(p + k));
+                const dbl2_nt v = ldp<KEEP>((const dbl2_nt *)(p + k));
                 pe[k] = v.x;
                 pe[k + 1] = v.y;
             }
@@ -121,7 +122,7 @@ __device__ inline void epi_load_row(T (&pe)[PC], const EpiArgs<T> &E, const T *p
     }
     const int last = E.prow - 1;
 #pragma unroll
-    for (int k = 0; k < PC; k++) pe[k] = ldnt(p + min(k, last));
+    for (int k = 0; k < PC; k++) pe[k] = ldp<KEEP>(p + min(k, last));
 }
 
 // Accumulates a row into the epilogue sums: PDOT adds P components

@@ -14,6 +14,14 @@
 
 namespace idrs {
 
+// the launch under the cache policy A.keep
+#define SPMV_TARGS(...) __VA_ARGS__
+#define SPMV_LAUNCH(KER, TARGS, ...)                                                                \
+    do {                                                                                            \
+        if (A.keep) hipLaunchKernelGGL((KER<SPMV_TARGS TARGS, true>), gd, bd, 0, st, __VA_ARGS__);  \
+        else hipLaunchKernelGGL((KER<SPMV_TARGS TARGS, false>), gd, bd, 0, st, __VA_ARGS__);        \
+    } while (0)
+
 // CRS: a group of G lanes per row (G >= the typical row length), so a
 // wavefront covers 64/G consecutive rows whose entries are one contiguous,
 // coalesced stretch of values and column indices.  The block's row pointers
@@ -26,7 +34,7 @@ namespace idrs {
 // for P^T y lane g takes the P components g, g+G, ... of its rows.
 constexpr int CRS_CHUNK = 2048;   // rows whose row pointers sit in LDS at once
 
-template <class VT, class T, int EPI, int NV, int G>
+template <class VT, class T, int EPI, int NV, int G, bool KEEP>
 __global__ __launch_bounds__(SPMV_THREADS) void k_spmv_crs(SpmvArgs<VT, T> A, EpiArgs<T> E, const int *info) {
     if (info && *info >= 0) return;
     constexpr int GPB = SPMV_THREADS / G;
@@ -67,8 +75,8 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_spmv_crs(SpmvArgs<VT, T> A, Ep
             for (int u = 0; u < U; u++) {
                 const int j = a[u] + g;
                 const bool ok = j < b[u];
-                vv[u] = ok ? ldnt(&val[j]) : VT(0);
-                cc[u] = ok ? ldnt(&col[j]) : -1;
+                vv[u] = ok ? ldp<KEEP>(&val[j]) : VT(0);
+                cc[u] = ok ? ldp<KEEP>(&col[j]) : -1;
             }
             // P components of the rows (P^T y) are issued with the matrix
             // loads; z and r are loaded at the finish, where the register
@@ -76,14 +84,14 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_spmv_crs(SpmvArgs<VT, T> A, Ep
             T pe[U][PC];
             if constexpr (EPI == EPI_PDOT) {
 #pragma unroll
-                for (int u = 0; u < U; u++) epi_load<T, EPI, PC>(pe[u], E, rq[u], g, G);
+                for (int u = 0; u < U; u++) epi_load<T, EPI, PC, KEEP>(pe[u], E, rq[u], g, G);
             }
             T acc[U];
 #pragma unroll
             for (int u = 0; u < U; u++) acc[u] = cc[u] >= 0 ? mulv(vv[u], x[cc[u]]) : T(0);
 #pragma unroll
             for (int u = 0; u < U; u++)
-                for (int j = a[u] + g + G; j < b[u]; j += G) acc[u] = fmav(ldnt(&val[j]), x[ldnt(&col[j])], acc[u]);
+                for (int j = a[u] + g + G; j < b[u]; j += G) acc[u] = fmav(ldp<KEEP>(&val[j]), x[ldp<KEEP>(&col[j])], acc[u]);
 #pragma unroll
             for (int u = 0; u < U; u++)
 #pragma unroll
@@ -97,7 +105,7 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_spmv_crs(SpmvArgs<VT, T> A, Ep
                     if constexpr (EPI == EPI_PDOT) {
                         epi_accum<T, EPI, PC, PC>(e, pe[u], E, yv, g, G);
                     } else if (g == 0) {
-                        epi_load<T, EPI, PC>(pe[u], E, row[u], 0, 1);
+                        epi_load<T, EPI, PC, KEEP>(pe[u], E, row[u], 0, 1);
                         epi_accum<T, EPI, NV, PC>(e, pe[u], E, yv, 0, 1);
                     }
                 }
@@ -109,7 +117,7 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_spmv_crs(SpmvArgs<VT, T> A, Ep
 
 // DIA: one thread per row over a contiguous row range; every diagonal is a
 // coalesced stream.  ND > 0 unrolls a known diagonal count.
-template <class VT, class T, int EPI, int NV, int ND>
+template <class VT, class T, int EPI, int NV, int ND, bool KEEP>
 __global__ __launch_bounds__(SPMV_THREADS) void k_spmv_dia(SpmvArgs<VT, T> A, EpiArgs<T> E, const int *info) {
     if (info && *info >= 0) return;
     constexpr int PC = EPI == EPI_PDOT ? NV : 1;
@@ -161,7 +169,7 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_spmv_dia(SpmvArgs<VT, T> A, Ep
             zq = zp ? *(const T *)((const char *)zp + bo) : T(0);
             if constexpr (EPI == EPI_PDOT) {
                 const T *p = (const T *)((const char *)E.P + (unsigned)row * (unsigned)(E.prow * sizeof(T)));
-                epi_load_row<T, PC>(pe, E, p);
+                epi_load_row<T, PC, KEEP>(pe, E, p);
             }
             VT vv[ND];
             T xx[ND];
@@ -175,7 +183,7 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_spmv_dia(SpmvArgs<VT, T> A, Ep
                 const bool ok = cc >= 0 && cc < ncols;
                 if constexpr (std::is_same<VT, T>::value) {
                     const unsigned xo = (unsigned)(ok ? cc : row) * (unsigned)sizeof(T);
-                    const VT v = d == ud ? VT(1) : ldnt((const VT *)((const char *)vb[d] + vbo));
+                    const VT v = d == ud ? VT(1) : ldp<KEEP>((const VT *)((const char *)vb[d] + vbo));
                     const T xv = *(const T *)((const char *)x + xo);
                     vv[d] = ok ? v : VT(0);
                     xx[d] = ok ? xv : T(0);
@@ -183,7 +191,7 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_spmv_dia(SpmvArgs<VT, T> A, Ep
                     // values of another type: loads under the column test, so
                     // that the conversion is not placed next to each load
                     // (which would wait for it before the next is issued)
-                    vv[d] = !ok ? VT(0) : (d == ud ? VT(1) : ldnt((const VT *)((const char *)vb[d] + vbo)));
+                    vv[d] = !ok ? VT(0) : (d == ud ? VT(1) : ldp<KEEP>((const VT *)((const char *)vb[d] + vbo)));
                     xx[d] = ok ? *(const T *)((const char *)x + (unsigned)cc * (unsigned)sizeof(T)) : T(0);
                 }
             }
@@ -191,21 +199,21 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_spmv_dia(SpmvArgs<VT, T> A, Ep
             for (int d = 0; d < ND; d++) acc = fmav(vv[d], xx[d], acc);
             const T yv = finish_value(A, row, acc, zq);
             *(T *)((char *)A.y + bo) = yv;
-            if constexpr (EPI != EPI_PDOT) epi_load<T, EPI, PC>(pe, E, row, 0, 1);
+            if constexpr (EPI != EPI_PDOT) epi_load<T, EPI, PC, KEEP>(pe, E, row, 0, 1);
             epi_accum<T, EPI, NV, PC>(e, pe, E, yv, 0, 1);
             continue;
         } else {
             zq = zp ? zp[row] : T(0);
-            if constexpr (EPI == EPI_PDOT) epi_load<T, EPI, PC>(pe, E, row, 0, 1);
+            if constexpr (EPI == EPI_PDOT) epi_load<T, EPI, PC, KEEP>(pe, E, row, 0, 1);
             for (int d = 0; d < ndiag; d++) {
                 const long cc = row + s_off[d];
                 const long sd = d - (d > ud ? 1 : 0);
-                if (cc >= 0 && cc < ncols) acc = fmav(d == ud ? VT(1) : ldnt(&val[sd * n + row]), x[cc], acc);
+                if (cc >= 0 && cc < ncols) acc = fmav(d == ud ? VT(1) : ldp<KEEP>(&val[sd * n + row]), x[cc], acc);
             }
         }
         const T yv = finish_value(A, row, acc, zq);
         A.y[row] = yv;
-        if constexpr (EPI != EPI_PDOT) epi_load<T, EPI, PC>(pe, E, row, 0, 1);
+        if constexpr (EPI != EPI_PDOT) epi_load<T, EPI, PC, KEEP>(pe, E, row, 0, 1);
         epi_accum<T, EPI, NV, PC>(e, pe, E, yv, 0, 1);
     }
     epi_store<T, EPI, NV>(e, E, s_red);
@@ -216,7 +224,7 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_spmv_dia(SpmvArgs<VT, T> A, Ep
 // SELL_C consecutive values (or column indices).  Entries go in chunks of 8:
 // all value and index loads of a chunk, then all its x gathers; the row sum
 // runs over k in CRS order (the reference's sequential row sum).
-template <class VT, class T>
+template <bool KEEP, class VT, class T>
 __device__ inline T sell_row(const SpmvArgs<VT, T> &A, long row, long p0, int w) {
     const VT *__restrict__ val = A.val;
     const int *__restrict__ scol = A.sl_col;
@@ -235,7 +243,7 @@ __device__ inline T sell_row(const SpmvArgs<VT, T> &A, long row, long p0, int w)
 #pragma unroll
                 for (int k = 0; k < 8; k++) {
                     const bool ok = k0 + k < len;
-                    const unsigned long long e = ok ? __builtin_nontemporal_load(&pr[p0 + (long)SELL_C * (k0 + k)]) : 0ull;
+                    const unsigned long long e = ok ? ldp<KEEP>(&pr[p0 + (long)SELL_C * (k0 + k)]) : 0ull;
                     vv[k] = __uint_as_float((unsigned)(e & 0xffffffffull));
                     cc[k] = (int)(e >> 32);
                 }
@@ -257,8 +265,8 @@ __device__ inline T sell_row(const SpmvArgs<VT, T> &A, long row, long p0, int w)
 #pragma unroll
         for (int k = 0; k < 8; k++) {
             const bool ok = k0 + k < len;
-            vv[k] = ok ? ldnt(&val[p0 + (long)SELL_C * (k0 + k)]) : VT(0);
-            cc[k] = ok ? ldnt(&scol[p0 + (long)SELL_C * (k0 + k)]) : 0;
+            vv[k] = ok ? ldp<KEEP>(&val[p0 + (long)SELL_C * (k0 + k)]) : VT(0);
+            cc[k] = ok ? ldp<KEEP>(&scol[p0 + (long)SELL_C * (k0 + k)]) : 0;
         }
         T xx[8];
 #pragma unroll
@@ -270,7 +278,7 @@ __device__ inline T sell_row(const SpmvArgs<VT, T> &A, long row, long p0, int w)
     return acc;
 }
 
-template <class VT, class T, int EPI, int NV>
+template <class VT, class T, int EPI, int NV, bool KEEP>
 __global__ __launch_bounds__(SPMV_THREADS) void k_spmv_sell(SpmvArgs<VT, T> A, EpiArgs<T> E, const int *info) {
     static_assert(SPMV_THREADS % SELL_C == 0 && SELL_C == WAVE, "one slice per wavefront");
     if (info && *info >= 0) return;
@@ -294,11 +302,11 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_spmv_sell(SpmvArgs<VT, T> A, E
         const int w = (int)((A.sl_ptr[slice + 1] - sp) / SELL_C);
         const T zq = zp ? zp[row] : T(0);
         T pe[PC];
-        if constexpr (EPI == EPI_PDOT) epi_load<T, EPI, PC>(pe, E, row, 0, 1);
-        const T acc = sell_row(A, row, sp + (row % SELL_C), w);
+        if constexpr (EPI == EPI_PDOT) epi_load<T, EPI, PC, KEEP>(pe, E, row, 0, 1);
+        const T acc = sell_row<KEEP>(A, row, sp + (row % SELL_C), w);
         const T yv = finish_value(A, row, acc, zq);
         A.y[row] = yv;
-        if constexpr (EPI != EPI_PDOT) epi_load<T, EPI, PC>(pe, E, row, 0, 1);
+        if constexpr (EPI != EPI_PDOT) epi_load<T, EPI, PC, KEEP>(pe, E, row, 0, 1);
         epi_accum<T, EPI, NV, PC>(e, pe, E, yv, 0, 1);
     }
     epi_store<T, EPI, NV>(e, E, s_red);
@@ -311,17 +319,17 @@ static void launch_spmv(const DevMatrix &K, const SpmvArgs<VT, T> &A, EpiArgs<T>
     E.nparts = grid;
     dim3 gd(grid), bd(SPMV_THREADS);
     if (K.fmt == DevFmt::CRS && A.sl_ptr) {
-        hipLaunchKernelGGL((k_spmv_sell<VT, T, EPI, NV>), gd, bd, 0, st, A, E, info);
+        SPMV_LAUNCH(k_spmv_sell, (VT, T, EPI, NV), A, E, info);
     } else if (K.fmt == DevFmt::CRS) {
         // group 1 without sliced values (e.g. the FP32 copy): 2 lanes per row
         switch (K.group) {
         case 1:
-        case 2: hipLaunchKernelGGL((k_spmv_crs<VT, T, EPI, NV, 2>), gd, bd, 0, st, A, E, info); break;
-        case 4: hipLaunchKernelGGL((k_spmv_crs<VT, T, EPI, NV, 4>), gd, bd, 0, st, A, E, info); break;
-        case 8: hipLaunchKernelGGL((k_spmv_crs<VT, T, EPI, NV, 8>), gd, bd, 0, st, A, E, info); break;
-        case 16: hipLaunchKernelGGL((k_spmv_crs<VT, T, EPI, NV, 16>), gd, bd, 0, st, A, E, info); break;
-        case 32: hipLaunchKernelGGL((k_spmv_crs<VT, T, EPI, NV, 32>), gd, bd, 0, st, A, E, info); break;
-        default: hipLaunchKernelGGL((k_spmv_crs<VT, T, EPI, NV, 64>), gd, bd, 0, st, A, E, info); break;
+        case 2: SPMV_LAUNCH(k_spmv_crs, (VT, T, EPI, NV, 2), A, E, info); break;
+        case 4: SPMV_LAUNCH(k_spmv_crs, (VT, T, EPI, NV, 4), A, E, info); break;
+        case 8: SPMV_LAUNCH(k_spmv_crs, (VT, T, EPI, NV, 8), A, E, info); break;
+        case 16: SPMV_LAUNCH(k_spmv_crs, (VT, T, EPI, NV, 16), A, E, info); break;
+        case 32: SPMV_LAUNCH(k_spmv_crs, (VT, T, EPI, NV, 32), A, E, info); break;
+        default: SPMV_LAUNCH(k_spmv_crs, (VT, T, EPI, NV, 64), A, E, info); break;
         }
     } else {
         // the unrolled kernels address rows by 32-bit byte offsets
@@ -329,10 +337,10 @@ static void launch_spmv(const DevMatrix &K, const SpmvArgs<VT, T> &A, EpiArgs<T>
         const int nd =
             K.nrows <= K.ncols && (unsigned long long)K.ncols * rowb < (1ull << 32) ? K.ndiag : 0;
         switch (nd) {
-        case 3: hipLaunchKernelGGL((k_spmv_dia<VT, T, EPI, NV, 3>), gd, bd, 0, st, A, E, info); break;
-        case 5: hipLaunchKernelGGL((k_spmv_dia<VT, T, EPI, NV, 5>), gd, bd, 0, st, A, E, info); break;
-        case 7: hipLaunchKernelGGL((k_spmv_dia<VT, T, EPI, NV, 7>), gd, bd, 0, st, A, E, info); break;
-        default: hipLaunchKernelGGL((k_spmv_dia<VT, T, EPI, NV, 0>), gd, bd, 0, st, A, E, info); break;
+        case 3: SPMV_LAUNCH(k_spmv_dia, (VT, T, EPI, NV, 3), A, E, info); break;
+        case 5: SPMV_LAUNCH(k_spmv_dia, (VT, T, EPI, NV, 5), A, E, info); break;
+        case 7: SPMV_LAUNCH(k_spmv_dia, (VT, T, EPI, NV, 7), A, E, info); break;
+        default: SPMV_LAUNCH(k_spmv_dia, (VT, T, EPI, NV, 0), A, E, info); break;
         }
     }
     LAUNCH_CHECK();
@@ -364,7 +372,7 @@ void dispatch_epi(const DevMatrix &K, const SpmvArgs<VT, T> &A, const EpiArgs<T>
 // launch; each column's row sum and finish are those of k_spmv_dia /
 // k_spmv_sell, so column j equals the one-column product of x_j bit for bit.
 // ---------------------------------------------------------------------------
-template <class VT, class T, int ND>
+template <class VT, class T, int ND, bool KEEP>
 __global__ __launch_bounds__(SPMV_THREADS) void k_spmv_dia_cols(SpmvArgs<VT, T> A, ColArgs<T> C) {
     static_assert(ND > 0 && ND <= 8, "known diagonal counts only");
     const int lb = xcd_block(blockIdx.x, gridDim.x);
@@ -382,7 +390,7 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_spmv_dia_cols(SpmvArgs<VT, T> 
             const long cc = row + A.off8[d];
             ok[d] = cc >= 0 && cc < ncols;
             const long sd = d - (d > ud ? 1 : 0);
-            vv[d] = !ok[d] ? VT(0) : (d == ud ? VT(1) : ldnt(A.val + sd * n + row));
+            vv[d] = !ok[d] ? VT(0) : (d == ud ? VT(1) : ldp<KEEP>(A.val + sd * n + row));
         }
 #pragma unroll
         for (int j = 0; j < SPMV_COLS; j++) {
@@ -402,7 +410,7 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_spmv_dia_cols(SpmvArgs<VT, T> 
     }
 }
 
-template <class VT, class T>
+template <class VT, class T, bool KEEP>
 __global__ __launch_bounds__(SPMV_THREADS) void k_spmv_sell_cols(SpmvArgs<VT, T> A, ColArgs<T> C) {
     const int lb = xcd_block(blockIdx.x, gridDim.x);
     const long n = A.nrows;
@@ -429,8 +437,8 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_spmv_sell_cols(SpmvArgs<VT, T>
 #pragma unroll
             for (int k = 0; k < 8; k++) {
                 const bool ok = k0 + k < len;
-                vv[k] = ok ? ldnt(&val[p0 + (long)SELL_C * (k0 + k)]) : VT(0);
-                cc[k] = ok ? ldnt(&scol[p0 + (long)SELL_C * (k0 + k)]) : 0;
+                vv[k] = ok ? ldp<KEEP>(&val[p0 + (long)SELL_C * (k0 + k)]) : VT(0);
+                cc[k] = ok ? ldp<KEEP>(&scol[p0 + (long)SELL_C * (k0 + k)]) : 0;
             }
 #pragma unroll
             for (int j = 0; j < SPMV_COLS; j++) {
@@ -463,12 +471,12 @@ bool launch_cols(const DevMatrix &K, const SpmvArgs<VT, T> &A, const ColArgs<T> 
     dim3 gd(spmv_grid(K)), bd(SPMV_THREADS);
     if (K.fmt == DevFmt::CRS) {
         if (!A.sl_ptr || A.pair32) return false;
-        hipLaunchKernelGGL((k_spmv_sell_cols<VT, T>), gd, bd, 0, st, A, C);
+        SPMV_LAUNCH(k_spmv_sell_cols, (VT, T), A, C);
     } else {
         switch (K.ndiag) {
-        case 3: hipLaunchKernelGGL((k_spmv_dia_cols<VT, T, 3>), gd, bd, 0, st, A, C); break;
-        case 5: hipLaunchKernelGGL((k_spmv_dia_cols<VT, T, 5>), gd, bd, 0, st, A, C); break;
-        case 7: hipLaunchKernelGGL((k_spmv_dia_cols<VT, T, 7>), gd, bd, 0, st, A, C); break;
+        case 3: SPMV_LAUNCH(k_spmv_dia_cols, (VT, T, 3), A, C); break;
+        case 5: SPMV_LAUNCH(k_spmv_dia_cols, (VT, T, 5), A, C); break;
+        case 7: SPMV_LAUNCH(k_spmv_dia_cols, (VT, T, 7), A, C); break;
         default: return false;
         }
     }
@@ -489,7 +497,7 @@ struct TileArgs {
     int stride;
 };
 
-template <class VT, class T, int EPI, int NV, int G>
+template <class VT, class T, int EPI, int NV, int G, bool KEEP>
 __global__ __launch_bounds__(SPMV_THREADS) void k_bspmv_crs(SpmvArgs<VT, T> A, EpiArgs<T> E, TileArgs ta) {
     const int tile = blockIdx.x;
     if (ta.info && ta.info[(long)ta.tile_sys[tile] * ta.stride] >= 0) return;
@@ -525,20 +533,20 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_bspmv_crs(SpmvArgs<VT, T> A, E
         for (int u = 0; u < U; u++) {
             const int j = a[u] + g;
             const bool ok = j < b[u];
-            vv[u] = ok ? ldnt(&val[j]) : VT(0);
-            cc[u] = ok ? ldnt(&col[j]) : -1;
+            vv[u] = ok ? ldp<KEEP>(&val[j]) : VT(0);
+            cc[u] = ok ? ldp<KEEP>(&col[j]) : -1;
         }
         T pe[U][PC];
         if constexpr (EPI == EPI_PDOT) {
 #pragma unroll
-            for (int u = 0; u < U; u++) epi_load<T, EPI, PC>(pe[u], E, rq[u], g, G);
+            for (int u = 0; u < U; u++) epi_load<T, EPI, PC, KEEP>(pe[u], E, rq[u], g, G);
         }
         T acc[U];
 #pragma unroll
         for (int u = 0; u < U; u++) acc[u] = cc[u] >= 0 ? mulv(vv[u], x[cc[u]]) : T(0);
 #pragma unroll
         for (int u = 0; u < U; u++)
-            for (int j = a[u] + g + G; j < b[u]; j += G) acc[u] = fmav(ldnt(&val[j]), x[ldnt(&col[j])], acc[u]);
+            for (int j = a[u] + g + G; j < b[u]; j += G) acc[u] = fmav(ldp<KEEP>(&val[j]), x[ldp<KEEP>(&col[j])], acc[u]);
 #pragma unroll
         for (int u = 0; u < U; u++)
 #pragma unroll
@@ -552,7 +560,7 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_bspmv_crs(SpmvArgs<VT, T> A, E
                 if constexpr (EPI == EPI_PDOT) {
                     epi_accum<T, EPI, PC, PC>(e, pe[u], E, yv, g, G);
                 } else if (g == 0) {
-                    epi_load<T, EPI, PC>(pe[u], E, row[u], 0, 1);
+                    epi_load<T, EPI, PC, KEEP>(pe[u], E, row[u], 0, 1);
                     epi_accum<T, EPI, NV, PC>(e, pe[u], E, yv, 0, 1);
                 }
             }
@@ -563,7 +571,7 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_bspmv_crs(SpmvArgs<VT, T> A, E
 
 // tile form of k_spmv_sell: a tile starts at any row; each wavefront walks
 // whole slices and masks the rows outside the tile
-template <class VT, class T, int EPI, int NV>
+template <class VT, class T, int EPI, int NV, bool KEEP>
 __global__ __launch_bounds__(SPMV_THREADS) void k_bspmv_sell(SpmvArgs<VT, T> A, EpiArgs<T> E, TileArgs ta) {
     const int tile = blockIdx.x;
     if (ta.info && ta.info[(long)ta.tile_sys[tile] * ta.stride] >= 0) return;
@@ -587,11 +595,11 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_bspmv_sell(SpmvArgs<VT, T> A, 
         const int w = (int)((A.sl_ptr[slice + 1] - sp) / SELL_C);
         const T zq = zp ? zp[row] : T(0);
         T pe[PC];
-        if constexpr (EPI == EPI_PDOT) epi_load<T, EPI, PC>(pe, E, row, 0, 1);
-        const T acc = sell_row(A, row, sp + (row % SELL_C), w);
+        if constexpr (EPI == EPI_PDOT) epi_load<T, EPI, PC, KEEP>(pe, E, row, 0, 1);
+        const T acc = sell_row<KEEP>(A, row, sp + (row % SELL_C), w);
         const T yv = finish_value(A, row, acc, zq);
         A.y[row] = yv;
-        if constexpr (EPI != EPI_PDOT) epi_load<T, EPI, PC>(pe, E, row, 0, 1);
+        if constexpr (EPI != EPI_PDOT) epi_load<T, EPI, PC, KEEP>(pe, E, row, 0, 1);
         epi_accum<T, EPI, NV, PC>(e, pe, E, yv, 0, 1);
     }
     epi_store<T, EPI, NV>(e, E, s_red);
@@ -609,18 +617,18 @@ static void launch_bspmv(const DevMatrix &K, const SpmvArgs<VT, T> &A, EpiArgs<T
     E.nparts = nt;
     dim3 gd(nt), bd(SPMV_THREADS);
     if (A.sl_ptr) {
-        hipLaunchKernelGGL((k_bspmv_sell<VT, T, EPI, NV>), gd, bd, 0, st, A, E, ta);
+        SPMV_LAUNCH(k_bspmv_sell, (VT, T, EPI, NV), A, E, ta);
         LAUNCH_CHECK();
         return;
     }
     switch (K.group) {
     case 1:
-    case 2: hipLaunchKernelGGL((k_bspmv_crs<VT, T, EPI, NV, 2>), gd, bd, 0, st, A, E, ta); break;
-    case 4: hipLaunchKernelGGL((k_bspmv_crs<VT, T, EPI, NV, 4>), gd, bd, 0, st, A, E, ta); break;
-    case 8: hipLaunchKernelGGL((k_bspmv_crs<VT, T, EPI, NV, 8>), gd, bd, 0, st, A, E, ta); break;
-    case 16: hipLaunchKernelGGL((k_bspmv_crs<VT, T, EPI, NV, 16>), gd, bd, 0, st, A, E, ta); break;
-    case 32: hipLaunchKernelGGL((k_bspmv_crs<VT, T, EPI, NV, 32>), gd, bd, 0, st, A, E, ta); break;
-    default: hipLaunchKernelGGL((k_bspmv_crs<VT, T, EPI, NV, 64>), gd, bd, 0, st, A, E, ta); break;
+    case 2: SPMV_LAUNCH(k_bspmv_crs, (VT, T, EPI, NV, 2), A, E, ta); break;
+    case 4: SPMV_LAUNCH(k_bspmv_crs, (VT, T, EPI, NV, 4), A, E, ta); break;
+    case 8: SPMV_LAUNCH(k_bspmv_crs, (VT, T, EPI, NV, 8), A, E, ta); break;
+    case 16: SPMV_LAUNCH(k_bspmv_crs, (VT, T, EPI, NV, 16), A, E, ta); break;
+    case 32: SPMV_LAUNCH(k_bspmv_crs, (VT, T, EPI, NV, 32), A, E, ta); break;
+    default: SPMV_LAUNCH(k_bspmv_crs, (VT, T, EPI, NV, 64), A, E, ta); break;
     }
     LAUNCH_CHECK();
 }
