@@ -254,9 +254,11 @@ template <class T>
 __global__ __launch_bounds__(BT) void k_bfin_mu(BV bv, int k, State<T> *st, const T *partials) {
     State<T> *S = st + blockIdx.x;
     if (S->info >= 0) return;
-    __shared__ T red[SMAX];
+    __shared__ T red[SMAX], sM[PDOT_MAX * PDOT_MAX];
+    const int s = S->s;
+    for (int i = threadIdx.x; i < s * s; i += BT) sM[i] = S->M[i % s + SMAX * (i / s)];
     reduce_system(bv, partials, S->prow, red);
-    if (threadIdx.x == 0) scalar_mu(S, k, red);
+    if (threadIdx.x < WAVE) wave_mu(S, sM, s, k, red, (int)threadIdx.x);
 }
 
 template <class T>
@@ -281,9 +283,11 @@ template <class T>
 __global__ __launch_bounds__(BT) void k_bfin_cycle(BV bv, State<T> *st, const T *partials) {
     State<T> *S = st + blockIdx.x;
     if (S->info >= 0) return;
-    __shared__ T red[SMAX + 1];
+    __shared__ T red[SMAX + 1], sM[PDOT_MAX * PDOT_MAX];
+    const int s = S->s;
+    for (int i = threadIdx.x; i < s * s; i += BT) sM[i] = S->M[i % s + SMAX * (i / s)];
     reduce_system(bv, partials, 1 + S->prow, red);
-    if (threadIdx.x == 0) scalar_cycle(S, red, (double *)nullptr);
+    if (threadIdx.x < WAVE) wave_cycle(S, sM, s, red, (double *)nullptr, (int)threadIdx.x);
 }
 
 // flag[0] = 1 when every system has finished; flag[1 + k] = 1 while system

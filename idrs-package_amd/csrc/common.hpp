@@ -145,11 +145,88 @@ __device__ inline float shfl_xor(float v, int m) { return __shfl_xor(v, m, WAVE)
 template <class R>
 __device__ inline cplx<R> shfl_xor(cplx<R> v, int m) { return {__shfl_xor(v.re, m, WAVE), __shfl_xor(v.im, m, WAVE)}; }
 
-template <class T>
-__device__ inline T wave_sum(T v) {
+// The lane exchanges of a wave64 butterfly, without LDS: lane ^ 32 and
+// lane ^ 16 by the gfx950 row swaps, then inside a row of 16 by DPP.  After
+// the steps before it a value repeats with period 16, 8, ... lanes, so a
+// rotation by 8 or 4 lanes reaches the partner (lane ^ 8, lane ^ 4); the last
+// two are quad permutations.  A 64-bit exchange is two 32-bit moves of a few
+// cycles, where ds_bpermute pays LDS latency per step.
+template <int M>
+__device__ inline unsigned lane_xor32(unsigned v) {
+    constexpr int ctrl = M == 8 ? 0x128 : M == 4 ? 0x124 : M == 2 ? 0x4E : 0xB1;   // row_ror:8, row_ror:4, quad_perm
+    return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xF, 0xF, true);
+}
+template <int M>
+__device__ inline double wave_step(double v) {
+    union { double d; unsigned u[2]; } a, b, c;
+    a.d = v;
+    if constexpr (M == 32 || M == 16) {
+        // both halves of the swap: the pair's lower and upper member in every lane
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            if constexpr (M == 32) {
+                auto r = __builtin_amdgcn_permlane32_swap(a.u[i], a.u[i], false, false);
+                b.u[i] = r[0];
+                c.u[i] = r[1];
+            } else {
+                auto r = __builtin_amdgcn_permlane16_swap(a.u[i], a.u[i], false, false);
+                b.u[i] = r[0];
+                c.u[i] = r[1];
+            }
+        }
+        return b.d + c.d;
+    } else {
+        b.u[0] = lane_xor32<M>(a.u[0]);
+        b.u[1] = lane_xor32<M>(a.u[1]);
+        return v + b.d;
+    }
+}
+// Sum over the wavefront in every lane: the butterfly over lane ^ 32, 16, 8,
+// 4, 2, 1 (each step adds a commuting pair, so every lane holds the same bits).
+__device__ inline double wave_sum(double v) {
+    v = wave_step<32>(v);
+    v = wave_step<16>(v);
+    v = wave_step<8>(v);
+    v = wave_step<4>(v);
+    v = wave_step<2>(v);
+    return wave_step<1>(v);
+}
+__device__ inline float wave_sum(float v) {
 #pragma unroll
     for (int m = WAVE / 2; m >= 1; m >>= 1) v = v + shfl_xor(v, m);
     return v;
+}
+template <class R>
+__device__ inline cplx<R> wave_sum(cplx<R> v) { return {wave_sum(v.re), wave_sum(v.im)}; }
+
+// Sum over each row of 16 lanes, in every lane of the row
+__device__ inline double row_sum(double v) {
+    v = wave_step<8>(v);
+    v = wave_step<4>(v);
+    v = wave_step<2>(v);
+    return wave_step<1>(v);
+}
+template <class R>
+__device__ inline cplx<R> row_sum(cplx<R> v) { return {row_sum(v.re), row_sum(v.im)}; }
+
+// lane's value in every lane of the wavefront (lane wave-uniform)
+__device__ inline double lane_value(double v, int lane) {
+    union { double d; int i[2]; } a;
+    a.d = v;
+    a.i[0] = __builtin_amdgcn_readlane(a.i[0], lane);
+    a.i[1] = __builtin_amdgcn_readlane(a.i[1], lane);
+    return a.d;
+}
+__device__ inline float lane_value(float v, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+template <class R>
+__device__ inline cplx<R> lane_value(cplx<R> v, int lane) { return {lane_value(v.re, lane), lane_value(v.im, lane)}; }
+// orders a wavefront's earlier LDS or global writes before its later reads by
+// other lanes of the same wavefront
+__device__ inline void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
 // Sum NV values per thread over the block; result valid in thread 0.
