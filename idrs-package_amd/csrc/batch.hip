@@ -12,6 +12,7 @@
 // polls a single "all finished" flag one cycle behind, like the
 // single-system driver.
 #include "batch.hpp"
+#include "block.hpp"
 
 #include "idrs_state.hpp"
 #include "mixed.hpp"
@@ -455,6 +456,41 @@ void batch_idrs_solve(const Operator &A, int s, const T *b, T *x, const SolveOpt
     const int maxit = o.has_maxit ? o.maxit : (int)std::min<long>(2 * nmax, 1000);
     const long cap_it = maxit > 0 ? maxit : 10 * nmax + 1000;
     const int user_omega = (o.omega && o.n_omega >= 1) ? 1 : 0;
+
+    // Systems small enough each run whole in one workgroup, without waiting
+    // for each other (block.hip).
+    if (block_fits<T>(A, nmax, s, o)) {
+        DBuf scratch(block_scratch<T>(A, ntot, s, o)), bres(sizeof(BlockResult) * nsys);
+        DBuf bom(sizeof(T) * std::max(1, o.n_omega));
+        T *omega_d = nullptr;
+        if (user_omega) {
+            omega_d = bom.as<T>();
+            HIP_TRY(hipMemcpyAsync(omega_d, o.omega, sizeof(T) * o.n_omega, hipMemcpyHostToDevice, stream));
+        }
+        hipEvent_t e0, e1;
+        HIP_TRY(hipEventCreate(&e0));
+        HIP_TRY(hipEventCreate(&e1));
+        HIP_TRY(hipEventRecord(e0, stream));
+        block_solve<T>(A, nsys, part->row0, ntot, s, b, x, o, nullptr, omega_d, nullptr, 0, nullptr,
+                       cap_it / (s + 1) + 2, scratch.p, bres.as<BlockResult>(), stream);
+        HIP_TRY(hipEventRecord(e1, stream));
+        std::vector<BlockResult> hr(nsys);
+        HIP_TRY(hipMemcpyAsync(hr.data(), bres.p, sizeof(BlockResult) * nsys, hipMemcpyDeviceToHost, stream));
+        HIP_TRY(hipStreamSynchronize(stream));
+        float ms = 0.f;
+        HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
+        (void)hipEventDestroy(e0);
+        (void)hipEventDestroy(e1);
+        solve_ms = ms;
+        stats.assign(nsys, SolveStats{});
+        for (int q = 0; q < nsys; q++) {
+            stats[q].flag = hr[q].info < 0 ? 1 : hr[q].info;
+            stats[q].iterations = hr[q].iter;
+            stats[q].relres = hr[q].normr / hr[q].normb;
+            stats[q].solve_ms = ms;
+        }
+        return;
+    }
 
     const size_t vb = sizeof(T) * (size_t)ntot;
     DBuf bG(vb * s), bU(vb * s), br(vb), bt(vb), bw1(vb), bw2(vb), btmp(vb), bP(vb * prow);

@@ -24,6 +24,7 @@
 // Shadow spaces wider than PDOT_MAX rows take their P^T sums from a chunked
 // kernel (pdot.hpp) instead of the product epilogue and the update kernel.
 #include "idrs.hpp"
+#include "block.hpp"
 #include "idrs_state.hpp"
 #include "pdot.hpp"
 
@@ -385,233 +386,26 @@ __global__ __launch_bounds__(256) void k_prereduce(const State<T> *st, const T *
     }
 }
 
+// s up to FIN_S: the s x s logic by one wavefront (wave_mu, wave_cycle) on a
+// copy of M in LDS; wider ones by one thread
+constexpr int FIN_S = 16;
 template <class T>
-__global__ __launch_bounds__(FIN_THREADS) void k_fin_normb(State<T> *st, const T *partials, int nparts) {
-    __shared__ T red[1];
-    reduce_partials(partials, nparts, 1, red);
-    if (threadIdx.x == 0) {
-        st->normb = sqrt(sre(red[0]));
-        st->tolb = st->tol * st->normb;                                    // idrs.inc:94
-    }
-}
-
-template <class T>
-__global__ __launch_bounds__(FIN_THREADS) void k_fin_init(State<T> *st, const T *partials, int nparts, double *resvec) {
-    __shared__ T red[1];
-    reduce_partials(partials, nparts, 1, red);
-    if (threadIdx.x == 0) {
-        double nr = sqrt(sre(red[0]));
-        st->normr = nr;
-        if (resvec) resvec[0] = nr;                                        // idrs.inc:97
-        if (nr <= st->tolb) st->info = 0;                                  // idrs.inc:101
-    }
-}
-
-template <class T>
-__global__ __launch_bounds__(FIN_THREADS) void k_fin_final(State<T> *st, const T *partials, int nparts) {
-    __shared__ T red[1];
-    reduce_partials(partials, nparts, 1, red);
-    if (threadIdx.x == 0) {
-        double nr = sqrt(sre(red[0]));                                     // idrs.inc:304-307
-        st->normr = nr;
-        if (st->info == 0 && nr > st->tolb) st->info = 2;
-    }
-}
-
-// ---------------------------------------------------------------------------
-// MAKE_P (idrs_module.f90:839-937)
-// ---------------------------------------------------------------------------
-template <class T>
-__global__ void k_fill_uniform(long cnt, T *PT, unsigned long long seed) {
-    GRID_LOOP(q, cnt) {
-        if constexpr (Tr<T>::is_complex)
-            PT[q] = T(uniform01(seed, (uint64_t)q), uniform01(seed, (uint64_t)(cnt + q)));
-        else
-            PT[q] = uniform01(seed, (uint64_t)q);
-    }
-}
-
-template <class T>
-__global__ void k_copy_conj(long n, const T *__restrict__ r, T *__restrict__ PT) {
-    GRID_LOOP(q, n) PT[q] = Tr<T>::conj(r[q]);
-}
-
-// PT(j,:) / rho, the normalisation of a finished row
-template <class T>
-__device__ inline T gs_scaled(T p, double rho) {
-    if constexpr (Tr<T>::is_complex)
-        return T(p.re / rho, p.im / rho);
-    else
-        return p / rho;
-}
-
-// alpha(k) = dot_product(PT(j,:),PT(k,:)) [real] / dot_product(PT(k,:),PT(j,:)) [complex], k < j.
-// SC: row j-1 is first divided by st->rho and stored (k_gs_scale's step in
-// the same pass; the dot with it uses the stored value)
-template <class T, int NV, bool SC>
-__global__ __launch_bounds__(256) void k_gs_dots(long n, int s, int j, const State<T> *st, T *PT, T *partials,
-                                                 int nparts) {
-    __shared__ T lds[NV * 4];
-    const double rho = SC ? st->rho : 1.0;
-    T e[NV];
-#pragma unroll
-    for (int k = 0; k < NV; k++) e[k] = T(0);
-    GRID_LOOP(q, n) {
-        const T pj = PT[j + (long)s * q];
-        T pl = T(0);
-        if constexpr (SC) {
-            pl = gs_scaled(PT[j - 1 + (long)s * q], rho);
-            PT[j - 1 + (long)s * q] = pl;
-        }
-#pragma unroll
-        for (int k = 0; k < NV; k++)
-            if (k < j) e[k] = fmaT(Tr<T>::conj((SC && k == j - 1) ? pl : PT[k + (long)s * q]), pj, e[k]);
-    }
-    block_sum<T, NV>(e, lds);
-    if (threadIdx.x == 0)
-        for (int k = 0; k < NV; k++) partials[(long)k * nparts + blockIdx.x] = e[k];
-}
-
-// row 0 of a given P: PT = PT_raw (every row) and partials = |PT(0,:)|^2,
-// the copy and k_gs_update_norm's j = 0 pass in one
-template <class T>
-__global__ __launch_bounds__(256) void k_gs_first(long n, int s, const T *PT_raw, T *PT, T *partials) {
-    __shared__ T lds[4];
-    T e[1] = {T(0)};
-    GRID_LOOP(q, n) {
-        for (int i = 1; i < s; i++) PT[i + (long)s * q] = PT_raw[i + (long)s * q];
-        const T p = PT_raw[(long)s * q];
-        PT[(long)s * q] = p;
-        e[0] = e[0] + T(Tr<T>::abs2(p));
-    }
-    block_sum<T, 1>(e, lds);
-    if (threadIdx.x == 0) partials[blockIdx.x] = e[0];
-}
-
-// k_gs_dots for rows j above PDOT_MAX: grid row y sums the coefficients
-// k in [y*PDOT_MAX, min(j, (y+1)*PDOT_MAX)) with k_gs_dots' arithmetic
-template <class T>
-__global__ __launch_bounds__(256) void k_gs_dots_wide(long n, int s, int j, const T *__restrict__ PT, T *partials,
-                                                      int nparts) {
-    constexpr int NV = PDOT_MAX;
-    __shared__ T lds[NV * 4];
-    const int k0 = blockIdx.y * NV, cnt = min(NV, j - k0);
-    T e[NV];
-#pragma unroll
-    for (int k = 0; k < NV; k++) e[k] = T(0);
-    GRID_LOOP(q, n) {
-        const T pj = PT[j + (long)s * q];
-#pragma unroll
-        for (int k = 0; k < NV; k++)
-            if (k < cnt) e[k] = fmaT(Tr<T>::conj(PT[k0 + k + (long)s * q]), pj, e[k]);
-    }
-    block_sum<T, NV>(e, lds);
-    if (threadIdx.x == 0)
-        for (int k = 0; k < cnt; k++) partials[(long)(k0 + k) * nparts + blockIdx.x] = e[k];
-}
-
-template <class T>
-__global__ __launch_bounds__(FIN_THREADS) void k_fin_gs(State<T> *st, const T *partials, int nparts, int nv) {
-    __shared__ T red[SMAX];
-    reduce_partials(partials, nparts, nv, red);
-    if (threadIdx.x == 0)
-        for (int k = 0; k < nv; k++) st->gs[k] = red[k];
-}
-
-// PT(j,:) = PT(j,:) - alpha(k)*PT(k,:) for k < j; partials = |PT(j,:)|^2
-template <class T>
-__global__ __launch_bounds__(256) void k_gs_update_norm(long n, int s, int j, const State<T> *st, T *PT,
-                                                        T *partials) {
-    __shared__ T lds[4], sa[SMAX];
-    if (threadIdx.x < SMAX) sa[threadIdx.x] = st->gs[threadIdx.x];
-    __syncthreads();
-    T e[1] = {T(0)};
-    GRID_LOOP(q, n) {
-        T p = PT[j + (long)s * q];
-        for (int k = 0; k < j; k++) p = fmaT(-sa[k], PT[k + (long)s * q], p);
-        PT[j + (long)s * q] = p;
-        e[0] = e[0] + T(Tr<T>::abs2(p));
-    }
-    block_sum<T, 1>(e, lds);
-    if (threadIdx.x == 0) partials[blockIdx.x] = e[0];
-}
-
-template <class T>
-__global__ __launch_bounds__(FIN_THREADS) void k_fin_rho(State<T> *st, const T *partials, int nparts) {
-    __shared__ T red[1];
-    reduce_partials(partials, nparts, 1, red);
-    if (threadIdx.x == 0) st->rho = sqrt(sre(red[0]));
-}
-
-template <class T>
-__global__ void k_gs_scale(long n, int s, int j, const State<T> *st, T *PT) {
-    const double rho = st->rho;
-    GRID_LOOP(q, n) PT[j + (long)s * q] = gs_scaled(PT[j + (long)s * q], rho);
-}
-
-// ---------------------------------------------------------------------------
-// P_DOT of r at setup: partials of PT*r (no conjugation, or conjugated PT
-// for the one-row variants 3/4)
-// ---------------------------------------------------------------------------
-template <class T, int NV>
-__global__ __launch_bounds__(256) void k_pdot(long n, const T *__restrict__ w, const T *__restrict__ P, int prow,
-                                              int conjP, T *partials, int nparts) {
-    __shared__ T lds[NV * 4];
-    T e[NV];
-#pragma unroll
-    for (int i = 0; i < NV; i++) e[i] = T(0);
-    GRID_LOOP(q, n) {
-        const T wq = w[q];
-#pragma unroll
-        for (int i = 0; i < NV; i++)
-            if (i < prow) {
-                T p = ldnt(&P[q * prow + i]);
-                if (conjP) p = Tr<T>::conj(p);
-                e[i] = fmaT(p, wq, e[i]);
-            }
-    }
-    block_sum<T, NV>(e, lds);
-    if (threadIdx.x == 0)
-        for (int i = 0; i < NV; i++) partials[(long)i * nparts + blockIdx.x] = e[i];
-}
-
-template <class T>
-__global__ __launch_bounds__(FIN_THREADS) void k_fin_f(State<T> *st, const T *partials, int nparts) {
-    __shared__ T red[SMAX];
-    const int prow = st->prow;
-    reduce_partials(partials, nparts, prow, red);
-    if (threadIdx.x == 0)
-        for (int i = 0; i < st->s; i++) st->f[i] = i < prow ? red[i] : T(0);
-}
-
-// ---------------------------------------------------------------------------
-// one-block reduction + scalar logic kernels
-// ---------------------------------------------------------------------------
-// First level of a two-level reduction of many block partials: block b sums
-// its contiguous share of every value's partials ([v][nparts] in, [v][PRE]
-// out), in a fixed order, so the one-workgroup kernel after it reads PRE.
-constexpr int PRE = 64;
-template <class T>
-__global__ __launch_bounds__(256) void k_prereduce(const State<T> *st, const T *partials, int nparts, int nv,
-                                                   T *out) {
-    if (st->info >= 0) return;
-    __shared__ T lds[4];
-    const long p0 = (long)nparts * blockIdx.x / PRE, p1 = (long)nparts * (blockIdx.x + 1) / PRE;
-    for (int v = 0; v < nv; v++) {
-        T e[1] = {T(0)};
-        for (long p = p0 + threadIdx.x; p < p1; p += blockDim.x) e[0] = e[0] + partials[(long)v * nparts + p];
-        block_sum<T, 1>(e, lds);
-        if (threadIdx.x == 0) out[(long)v * PRE + blockIdx.x] = e[0];
-        __syncthreads();
-    }
+__device__ inline void stage_m(const State<T> *st, int s, T *sM) {
+    for (int i = threadIdx.x; i < s * s; i += blockDim.x) sM[i] = st->M[i % s + SMAX * (i / s)];
 }
 
 template <class T>
 __global__ __launch_bounds__(FIN_THREADS) void k_fin_mu(int k, State<T> *st, const T *partials, int nparts) {
     if (st->info >= 0) return;
-    __shared__ T red[SMAX];
+    __shared__ T red[SMAX], sM[FIN_S * FIN_S];
+    const int s = st->s;
+    if (s <= FIN_S) stage_m(st, s, sM);
     reduce_partials(partials, nparts, st->prow, red);
-    if (threadIdx.x == 0) scalar_mu(st, k, red);
+    if (s <= FIN_S) {
+        if (threadIdx.x < WAVE) wave_mu(st, sM, s, k, red, (int)threadIdx.x);
+    } else if (threadIdx.x == 0) {
+        scalar_mu(st, k, red);
+    }
 }
 
 template <class T>
@@ -964,6 +758,78 @@ struct LoopResHold {
 };
 }  // namespace
 
+// The solve of a small system by the one-workgroup kernel (block.hip):
+// checked options, the same outputs as the launches below.
+template <class T>
+static void solve_in_block(const Operator &A, long n, int s, const T *b, T *x, const SolveOpts<T> &o, SolveStats &out,
+                           long cap_it, bool user_omega, bool out_h, hipStream_t stream) {
+    Arena *ar = o.arena;
+    Buf scratch(block_scratch<T>(A, n, s, o), ar), bm1, bom, bh, bres, bout;
+    const T *m1 = o.has_m1 ? upload_diag_as<T>(o.M1, n, bm1, stream, ar) : nullptr;
+    T *omega_d = nullptr;
+    if (user_omega) {
+        bom = Buf(sizeof(T) * o.n_omega, ar);
+        omega_d = bom.as<T>();
+        HIP_TRY(hipMemcpyAsync(omega_d, o.omega, sizeof(T) * o.n_omega, hipMemcpyHostToDevice, stream));
+    }
+    double *resvec = nullptr;
+    if (o.resvec) {
+        bres = Buf(sizeof(double) * (cap_it + 2), ar);
+        resvec = bres.as<double>();
+    }
+    const size_t h_bytes = out_h ? sizeof(T) * (size_t)(o.nritz + 1) * o.nritz : 0;
+    // the result lands in pinned host memory (allocation-free: in the region)
+    constexpr unsigned MAPPED = hipHostMallocCoherent | hipHostMallocMapped;
+    struct Pinned {
+        void *p = nullptr;
+        ~Pinned() { pinned_give(p, sizeof(BlockResult), MAPPED); }
+    } pin;
+    BlockResult hr{}, *res = nullptr;
+    if (ar) {
+        bout = Buf(sizeof(BlockResult), ar);
+        res = bout.as<BlockResult>();
+    } else {
+        pin.p = pinned_take(sizeof(BlockResult), MAPPED);
+        HIP_TRY(hipHostGetDevicePointer((void **)&res, pin.p, 0));
+    }
+    std::chrono::steady_clock::time_point t0;
+    LoopResHold lres;
+    if (ar) {
+        HIP_TRY(hipStreamSynchronize(stream));
+        t0 = std::chrono::steady_clock::now();
+    } else {
+        lres.take();
+        HIP_TRY(hipEventRecord(lres.r.e0, stream));
+    }
+    if (out_h) {
+        bh = Buf(h_bytes, ar);
+        HIP_TRY(hipMemsetAsync(bh.p, 0, h_bytes, stream));   // H = 0 (idrs.inc:89)
+    }
+    block_solve<T>(A, 1, nullptr, n, s, b, x, o, m1, omega_d, resvec, (int)(cap_it + 2), bh.as<T>(),
+                   cap_it / (s + 1) + 2, scratch.p, res, stream);
+    if (ar) HIP_TRY(hipMemcpyAsync(&hr, res, sizeof hr, hipMemcpyDeviceToHost, stream));
+    else HIP_TRY(hipEventRecord(lres.r.e1, stream));
+    HIP_TRY(hipStreamSynchronize(stream));
+    float ms = 0.f;
+    if (ar) {
+        ms = std::chrono::duration<float, std::milli>(std::chrono::steady_clock::now() - t0).count();
+    } else {
+        hr = *(const BlockResult *)pin.p;
+        HIP_TRY(hipEventElapsedTime(&ms, lres.r.e0, lres.r.e1));
+    }
+    if (o.resvec) {
+        const long cnt = std::min<long>(std::min<long>(o.resvec_len, hr.iter + 1), cap_it + 2);
+        HIP_TRY(hipMemcpy(o.resvec, resvec, sizeof(double) * cnt, hipMemcpyDeviceToHost));
+    }
+    if (out_h) HIP_TRY(hipMemcpy(o.H, bh.p, h_bytes, hipMemcpyDeviceToHost));
+    out.flag = hr.info < 0 ? 1 : hr.info;
+    out.iterations = hr.iter;
+    out.relres = hr.normr / hr.normb;
+    out.solve_ms = ms;
+    out.spmv_ms = 0.0;
+    out.spmv_launches = 0;
+}
+
 template <class T>
 int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOpts<T> &o, SolveStats &out,
                hipStream_t stream) {
@@ -993,6 +859,12 @@ int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOp
     if (ar && out_h) throw std::invalid_argument("the Hessenberg output is not offered by the allocation-free solve");
     SpmvTimer &tm = spmv_timer();
     if (ar && tm.enabled) throw std::invalid_argument("SpMV timing needs events: not in the allocation-free solve");
+    if constexpr (std::is_same<T, double>::value || std::is_same<T, c128>::value) {
+        if (!tm.enabled && block_fits<T>(A, n, s, o)) {
+            solve_in_block<T>(A, n, s, b, x, o, out, cap_it, user_omega != 0, out_h, stream);
+            return 0;
+        }
+    }
     const int gv = vec_grid(n);
     const int gs = spmv_grid(*A.K);
     const size_t vb = sizeof(T) * (size_t)n;

@@ -66,6 +66,7 @@ struct SolveOpts {
     // solve makes no allocation of any kind (no graph, no events, no pinned
     // host memory: the host polls the flag with a blocking copy per cycle)
     Arena *arena = nullptr;
+    bool inner = false;              // the inner solve of another solver's iteration
 };
 
 template <class T>

@@ -1074,6 +1074,7 @@ static void qmr_driver(const Operator &A, long n, int ns, const std::vector<type
                     }
                 } else if (!multishift) {
                     SolveOpts<T> io;
+                    io.inner = true;
                     io.has_m1 = o.has_m1;
                     io.M1 = o.M1;
                     io.tol = in_tol;

@@ -159,6 +159,7 @@ static V *dev_upload(const V *h, size_t count) {
 static void finish_crs(DevMatrix *M, const std::vector<int> &rp0, const std::vector<int> &col0,
                        const std::vector<double> &rv, const std::vector<c128> &cv) {
     long nnz = M->nnz;
+    for (size_t i = 0; i + 1 < rp0.size(); i++) M->max_row = std::max(M->max_row, rp0[i + 1] - rp0[i]);
     M->row_ptr = dev_upload(rp0.data(), rp0.size());
     M->col = dev_upload(col0.data(), (size_t)nnz);
     if (M->kind == ValKind::Complex) {
@@ -564,6 +565,7 @@ DevMatrix *make_blockdiag(int nsys, const DevMatrix *const *Ks) {
     if (nsys < 1) throw std::invalid_argument("a batch needs at least one system");
     const ValKind kind = Ks[0]->kind;
     long nrows = 0, nnz = 0;
+    int max_row = 0;
     for (int b = 0; b < nsys; b++) {
         const DevMatrix *K = Ks[b];
         if (!K) throw std::invalid_argument("null system matrix");
@@ -572,6 +574,7 @@ DevMatrix *make_blockdiag(int nsys, const DevMatrix *const *Ks) {
         if (K->kind != kind) throw std::invalid_argument("batched systems must all be real or all complex");
         nrows += K->nrows;
         nnz += K->nnz;
+        max_row = std::max(max_row, K->max_row);
     }
     if (nrows > INT32_MAX || nnz > INT32_MAX) throw std::invalid_argument("batch too large for int32 indices");
     std::unique_ptr<DevMatrix> M(new DevMatrix);
@@ -580,6 +583,7 @@ DevMatrix *make_blockdiag(int nsys, const DevMatrix *const *Ks) {
     M->kind = kind;
     M->nrows = M->ncols = (int)nrows;
     M->nnz = nnz;
+    M->max_row = max_row;
     const size_t vsz = kind == ValKind::Complex ? sizeof(c128) : sizeof(double);
     HIP_TRY(hipMalloc(&M->row_ptr, sizeof(int) * (nrows + 1)));
     HIP_TRY(hipMalloc(&M->col, sizeof(int) * (nnz ? nnz : 1)));
@@ -661,6 +665,7 @@ DevMatrix *make_transpose(const DevMatrix &K) {
     T->nrows = m;
     T->ncols = n;
     T->nnz = nnz;
+    for (int j = 0; j < m; j++) T->max_row = std::max(T->max_row, trp[j + 1] - trp[j]);
     T->row_ptr = dev_upload(trp.data(), trp.size());
     T->col = dev_upload(tcol.data(), (size_t)nnz);
     T->tperm = dev_upload(perm.data(), (size_t)nnz);

@@ -74,6 +74,7 @@ struct DevMatrix {
     long nnz = 0;            // stored entries (CRS) or ndiag*nrows (DIA)
     // CRS (0-based on device)
     int *row_ptr = nullptr, *col = nullptr;
+    int max_row = 0;         // entries of the longest row
     int group = 8;           // lanes that share one row in the CRS kernel; 1: the sliced copy
     std::unique_ptr<Sell> sell;   // built for group 1 (autotune_group)
     // most row slabs (workgroups) of a one-thread-per-row product (DIA, the

@@ -1,0 +1,88 @@
+"""Small systems solved whole in one workgroup, against the oracle at the
+sizes where that kernel's shape changes: one row, a wavefront and a workgroup
+of rows and one more, the largest single system and the first above it, every
+stored form, and a batch up to its largest system.
+
+The fixed-count solutions agree to 1e-10 relative, the bar of the other GPU
+solves against the oracle; both sides take the same steps, so their rounding
+is all that differs.
+"""
+import numpy as np
+import pytest
+
+import idrs_amd
+import orc
+from helpers import rel
+from idrs_amd import problems as P
+
+pytestmark = pytest.mark.gpu
+
+
+def _system(n, seed, cplx=False):
+    """A banded nonsymmetric diagonally dominant matrix as CRS arrays and as
+    diagonals (offsets -7, -1, 0, 2)."""
+    rng = np.random.default_rng(seed)
+    offs = [o for o in (-7, -1, 0, 2) if abs(o) < n]
+    i = np.arange(n)
+    vals = rng.uniform(-1, 1, (n, len(offs))) + (1j * rng.uniform(-1, 1, (n, len(offs))) if cplx else 0)
+    vals[:, offs.index(0)] = 4.0 + rng.uniform(0, 1, n)
+    ok = np.stack([(i + o >= 0) & (i + o < n) for o in offs], axis=1)
+    vals = np.where(ok, vals, 0)
+    rp = np.concatenate([[1], 1 + np.cumsum(ok.sum(1))]).astype(np.int32)
+    col = (i[:, None] + np.array(offs) + 1)[ok].astype(np.int32)
+    return P.Crs(n, rp, col, np.ascontiguousarray(vals[ok])), (np.array(offs, dtype=np.int32), vals)
+
+
+@pytest.mark.parametrize("n,s,form", [
+    (1, 1, "crs"), (2, 1, "crs"), (63, 2, "dia"), (64, 4, "crs"), (65, 5, "crs"), (1023, 4, "dia"), (1024, 3, "crs"),
+    (1025, 16, "crs"), (2047, 4, "complex"), (2049, 8, "dia"), (2560, 4, "crs"), (2561, 4, "crs"),
+    (1500, 4, "poly"), (1500, 4, "m1"), (700, 2, "x0"), (700, 1, "variant2"), (700, 1, "variant4")])
+def test_small_solves_match_oracle(gpu, n, s, form):
+    cplx = form == "complex"
+    crs, (offs, vals) = _system(n, 3 + n, cplx)
+    rng = np.random.default_rng(n)
+    b = rng.uniform(-1, 1, n) + (1j * rng.uniform(-1, 1, n) if cplx else 0)
+    PT = P.gaussian_shadow(n, s, seed=1, complex=cplx)
+    kw, okw, mk = {}, {}, dict(which_precon=0)
+    if form == "dia":
+        K = idrs_amd.dia_format(n, n, offs, rvals=vals)
+    else:
+        K = idrs_amd.crs_format(n, n, crs.row_ptr, crs.col_ind, **{"cval" if cplx else "rval": crs.val})
+    if form == "poly":
+        mk = dict(which_precon=1, degree=3, alpha=orc.chebyshev(3, np.array([0.3, 1.7])))
+    A = idrs_amd.Matrix(K, which_precon=mk["which_precon"])
+    if form == "poly":
+        idrs_amd.real_preconditioner(A, 2, 3, foci=[0.3, 1.7])
+    Ao = orc.OracleMatrix(orc.CRS, n, crs=crs, complex_vectors=cplx, **mk)
+    if form == "m1":
+        kw["M1"], okw["M1"] = idrs_amd.Matrix(K, which_precon=1), orc.OracleMatrix(orc.CRS, n, crs=crs, which_precon=1)
+    if form == "x0":
+        kw["x0"] = okw["x0"] = rng.standard_normal(n)
+    if form.startswith("variant"):
+        kw["variant"] = okw["variant"] = int(form[-1])
+    k = min(10, n)
+    g = idrs_amd.idrs(A, b, s, tolerance=0.0, maximum_iterations=k, PT_raw=PT, resvec=True, **kw)
+    o = orc.idrs(Ao, b, s, tolerance=0.0, maximum_iterations=k, PT_raw=PT, **okw)
+    assert g.iterations == o[3]
+    if n > 2:   # one or two unknowns end in a breakdown on both sides
+        assert g.flag == o[1] and rel(g.x, o[0]) < 1e-10
+    c = idrs_amd.idrs(A, b, s, tolerance=1e-9, maximum_iterations=500, PT_raw=PT, **kw)
+    co = orc.idrs(Ao, b, s, tolerance=1e-9, maximum_iterations=500, PT_raw=PT, **okw)
+    assert c.flag == co[1] and abs(c.iterations - co[3]) <= 2
+
+
+@pytest.mark.parametrize("sizes,s", [([1, 64, 65, 900], 2), ([4096, 3, 1025, 2048, 4095], 4), ([4097, 30], 2)])
+def test_small_batches_match_oracle(gpu, sizes, s):
+    systems = [_system(n, 11 + n)[0] for n in sizes]
+    K = idrs_amd.batch_format([idrs_amd.crs_format(c.n, c.n, c.row_ptr, c.col_ind, rval=c.val) for c in systems])
+    b = np.random.default_rng(5).uniform(-1, 1, sum(sizes))
+    r = idrs_amd.idrs_batched(idrs_amd.Matrix(K), b, s, tolerance=1e-9, maximum_iterations=300)
+    at = 0
+    for k, c in enumerate(systems):
+        bk = b[at:at + c.n]
+        o = orc.idrs(orc.OracleMatrix(orc.CRS, c.n, crs=c), bk, s, tolerance=1e-9, maximum_iterations=300)
+        assert abs(int(r.iterations[k]) - o[3]) <= 2
+        if c.n > s:   # a system of at most s unknowns ends in a breakdown
+            assert r.flag[k] == o[1] == 0
+            assert np.linalg.norm(c.matvec(r.x[at:at + c.n]) - bk) <= 1.01e-9 * np.linalg.norm(bk)
+        at += c.n
