@@ -28,6 +28,7 @@
 #include "general.hpp"
 #include "spmv_epi.hpp"
 #include "spmv_launch.hpp"
+#include "rowcode.hpp"
 #include "ritz.hpp"
 #include "lu.hpp"
 
@@ -35,6 +36,7 @@
 #include <climits>
 #include <cstdarg>
 #include <cstring>
+#include <mutex>
 #include <numeric>
 #include <stdexcept>
 
@@ -445,10 +447,39 @@ static void with_args(const Operator &op, F &&f) {
     }
 }
 
+// The row code serves the products that sum a row in stored order: DIA, and
+// CRS in the sliced layout (lanes per row sum in another order).
+const RowCode *op_rowcode(const Operator &op) {
+    const DevMatrix &K = *op.K;
+    if (K.fmt == DevFmt::CRS && !(K.group == 1 && K.sell)) return nullptr;
+    if (op.values32 && op.seed != std::complex<double>(0.0, 0.0)) return nullptr;   // refused by with_args
+    if (op.seed.imag() != 0.0) return nullptr;
+    return (op.sval ? op.rowcode : K.rowcode).get();
+}
+
+// the argument block of a row-coded product of op (x, xs, z, a, y to be set)
+static SpmvArgs<double, double> rowcode_args(const Operator &op, int epi, const EpiArgs<double> &E) {
+    const DevMatrix &K = *op.K;
+    auto A = base_args<double, double>(K, nullptr);
+    A.has_seed = op.seed != std::complex<double>(0.0, 0.0);
+    A.sdiag = op.which_precon == 1 ? (const double *)op.pdiag : nullptr;
+    A.seed = op.seed.real();
+    const size_t vecs = 4 + (epi == EPI_PDOT ? (size_t)E.prow : 0);
+    A.keep = vecs * sizeof(double) * (size_t)K.nrows <= KEEP_BYTES;
+    return A;
+}
+
 template <class T>
 void op_spmv(const Operator &op, const T *x, T xs, const T *z, T a, T *y, int epi, const EpiArgs<T> &E,
              const int *info, hipStream_t st, const TileCtx *tc) {
     const DevMatrix &K = *op.K;
+    if constexpr (std::is_same<T, double>::value) {
+        if (const RowCode *rc = tc ? nullptr : op_rowcode(op)) {
+            SpmvArgs<double, double> A = rowcode_args(op, epi, E);
+            A.x = x; A.xs = xs; A.z = z; A.a = a; A.y = y;
+            return rowcode_spmv(K, *rc, op.values32, A, E, epi, info, st);
+        }
+    }
     with_args<T>(op, [&](auto &A) {
         A.x = x; A.xs = xs; A.z = z; A.a = a; A.y = y;
         set_keep(op, A, epi, E);
@@ -465,9 +496,7 @@ void op_spmv_cols(const Operator &op, int nc, long ld, const T *x, T xs, const T
     for (int j0 = 0; j0 < nc; j0 += SPMV_COLS) {
         const int m = std::min(SPMV_COLS, nc - j0);
         bool done = false;
-        with_args<T>(op, [&](auto &A) {
-            A.xs = xs;
-            set_keep(op, A, EPI_NONE, none);
+        auto columns = [&] {
             ColArgs<T> C{};
             C.nc = m;
             C.ld = ld;
@@ -475,7 +504,20 @@ void op_spmv_cols(const Operator &op, int nc, long ld, const T *x, T xs, const T
             C.z = z ? z + (long)j0 * ld : nullptr;
             C.y = y + (long)j0 * ld;
             for (int j = 0; j < m; j++) C.a[j] = a ? a[j0 + j] : T(0);
-            done = launch_cols(K, A, C, st);
+            return C;
+        };
+        if constexpr (std::is_same<T, double>::value) {
+            if (const RowCode *rc = op_rowcode(op)) {
+                SpmvArgs<double, double> A = rowcode_args(op, EPI_NONE, none);
+                A.xs = xs;
+                rowcode_cols(K, *rc, op.values32, A, columns(), st);
+                continue;
+            }
+        }
+        with_args<T>(op, [&](auto &A) {
+            A.xs = xs;
+            set_keep(op, A, EPI_NONE, none);
+            done = launch_cols(K, A, columns(), st);
         });
         if (!done)
             for (int j = j0; j < j0 + m; j++)
@@ -718,6 +760,8 @@ static void *sliced_copy(const Sell &S, const void *src, bool cplx, hipStream_t 
 // buffer (a free would synchronize the device on every refresh); the FP32
 // copy is dropped and rebuilt when next needed
 static void refresh_sliced(DevMatrix &K, hipStream_t st) {
+    K.rowcode.reset();
+    K.rowcode_tried = true;
     if (!K.sell) return;
     if (K.sell->sl_val32) {
         (void)hipFree(K.sell->sl_val32);
@@ -972,7 +1016,22 @@ bool op_prepared(const Operator &op) {
     return sliced && (!op.general() || (op.gws && op.gws_rows == op.rows()));
 }
 
+// Looks for the row code of the values that op's products read, once per
+// matrix (scaled values: per operator).  With fresh values every few solves
+// (set_values, transposes) it is not looked for.
+static void prepare_rowcode(const Operator &op, hipStream_t st) {
+    static std::mutex mu;
+    const DevMatrix &K = *op.K;
+    std::lock_guard<std::mutex> g(mu);
+    bool &tried = op.sval ? op.rowcode_tried : K.rowcode_tried;
+    if (tried || (op.sval && K.tperm)) return;
+    if (K.fmt == DevFmt::CRS && !(K.group == 1 && K.sell)) return;   // not read in that layout
+    (op.sval ? op.rowcode : K.rowcode) = make_rowcode(op, st);
+    tried = true;
+}
+
 void op_prepare(const Operator &op, hipStream_t st) {
+    prepare_rowcode(op, st);
     if (op_prepared(op)) return;
     const DevMatrix &K = *op.K;
     if (!(K.fmt != DevFmt::CRS || !K.sell || !op.sval || op.sl_sval))
@@ -1025,6 +1084,12 @@ int autotune_group(DevMatrix &K, int reps, hipStream_t st, std::vector<std::pair
             bool sell_ok = false;
             if (!K.sell && K.nnz > 0) build_sell(K, st);
             if (K.sell) sell_ok = K.sell->nent <= K.nnz + K.nnz / 4;
+            if (sell_ok) {   // the sliced layout is timed with its row code
+                K.group = 1;
+                Operator own;
+                own.K = &K;
+                prepare_rowcode(own, st);
+            }
             for (int g : {1, g0 / 2, g0, g0 * 2, g0 * 4}) {
                 if (g == 1 ? !sell_ok : (g < 2 || g > 64)) continue;
                 K.group = g;
@@ -1167,6 +1232,8 @@ static void drop_unit_diagonal(Operator &op, bool cvals, hipStream_t st) {
         HIP_TRY(hipMemcpyAsync(dst + vsz * n * z0, src + vsz * n * (z0 + 1), vsz * n * (K.ndiag - 1 - z0),
                                hipMemcpyDeviceToDevice, st));
     HIP_TRY(hipStreamSynchronize(st));
+    op.rowcode.reset();
+    op.rowcode_tried = false;
     (void)hipFree(op.sval);
     op.sval = packed;
     op.unit_diag = z0;
@@ -1192,6 +1259,8 @@ void op_set_diag_precon(Operator &op, int which, const std::complex<double> *shi
     (void)hipFree(op.sl_sval);
     (void)hipFree(op.sl_sval32);
     op.pdiag = op.sval = op.sval32 = nullptr;
+    op.rowcode.reset();
+    op.rowcode_tried = false;
     op.sl_sval = op.sl_sval32 = nullptr;
     op.unit_diag = -1;
     op.which_precon = which;
@@ -1274,6 +1343,8 @@ void op_set_diag_values(Operator &op, const std::vector<std::complex<double>> &d
     (void)hipFree(op.sl_sval);
     (void)hipFree(op.sl_sval32);
     op.pdiag = op.sval = op.sval32 = nullptr;
+    op.rowcode.reset();
+    op.rowcode_tried = false;
     op.sl_sval = op.sl_sval32 = nullptr;
     op.unit_diag = -1;
     op.which_precon = 1;

@@ -66,6 +66,8 @@ struct Sell {
     ~Sell();
 };
 
+struct RowCode;
+
 struct DevMatrix {
     int orig_format = 0;     // user_module matrix_format: 2 CRS, 3 COO, 4 CDS, 5 DIA
     DevFmt fmt = DevFmt::CRS;
@@ -95,6 +97,10 @@ struct DevMatrix {
     std::unique_ptr<Partition> part;
     // set for transposes (make_transpose): val[p] = source val[tperm[p]]
     int *tperm = nullptr;
+    // row code of K's own values (rowcode.hpp), made by op_prepare; tried:
+    // looked for, or values that change too often to look
+    mutable std::shared_ptr<RowCode> rowcode;
+    mutable bool rowcode_tried = false;
     ~DevMatrix();
 };
 
@@ -143,6 +149,9 @@ struct Operator {
     std::shared_ptr<LuFactor> lu;
     bool shift_invert = false;
     std::complex<double> si_shift{0.0, 0.0};
+    // row code of the scaled values, made by op_prepare
+    mutable std::shared_ptr<RowCode> rowcode;
+    mutable bool rowcode_tried = false;
     mutable void *gws = nullptr;     // workspace of the general path (gen_prepare)
     mutable long gws_rows = 0;
     bool general() const { return Mm || Cm || block || ndefl > 0 || lu || shift_invert; }
