@@ -516,9 +516,9 @@ __global__ __launch_bounds__(256) void k_orth_update(long n, int k, const State<
 
 // v = r/M1 before the omega step's product (idrs.inc:266-270)
 template <class T>
-__global__ __launch_bounds__(256) void k_form_v(long n, const State<T> *st, const T *__restrict__ r,
+__global__ __launch_bounds__(256) void k_form_v(long n, const int *info, const T *__restrict__ r,
                                                 const T *__restrict__ m1, T *__restrict__ v) {
-    if (st->info >= 0) return;
+    if (*info >= 0) return;
     GRID_LOOP(q, n) v[q] = sdiv(r[q], m1[q]);
 }
 
@@ -561,6 +561,298 @@ __global__ __launch_bounds__(256) void k_omega_update(long n, const State<T> *st
     block_sum<T, NV + 1>(e, lds);
     if (threadIdx.x == 0)
         for (int i = 0; i <= NV; i++) partials[(long)i * nparts + blockIdx.x] = e[i];
+}
+
+// ---------------------------------------------------------------------------
+// Folded cycle: the reductions and the scalar steps run at the start of the
+// streaming kernel that uses them, redundantly in every workgroup, instead of
+// in one-workgroup kernels of their own: 2 launches per inner step instead of
+// 4.  A launch-bound step (32^3) took 25 us, 12 of them in k_fin_mu and
+// k_fin_norm and the gaps around them.  Each streaming kernel reads the state
+// slot its predecessor wrote and workgroup 0 writes the next slot (a slot is
+// never written while it is read).  ||r|| of an inner step is judged by the
+// next streaming kernel, so a solve that ends there has run one product more,
+// which nothing uses.  Sums, logic and vector arithmetic are those of the
+// kernels above, in the same order: the same bits.
+// ---------------------------------------------------------------------------
+template <class T>
+using Slot = State<T, FIN_S>;
+constexpr int FOLD_PARTS = 2048;   // most partials a workgroup sums per value
+constexpr long FOLD_ROWS = 1L << 18;
+
+template <class T>
+__global__ void k_fold_init(const State<T> *st, Slot<T> *sl) {
+    const int s = st->s;
+    for (int i = threadIdx.x; i < FIN_S; i += blockDim.x) sl->f[i] = i < s ? st->f[i] : T(0);
+    for (int i = threadIdx.x; i < FIN_S * FIN_S; i += blockDim.x) sl->M[i] = T(0);
+    if (threadIdx.x == 0) {
+        sl->om = st->om;
+        sl->normb = st->normb;
+        sl->tolb = st->tolb;
+        sl->normr = st->normr;
+        sl->kappa = st->kappa;
+        sl->rho = st->rho;
+        sl->tol = st->tol;
+        sl->info = st->info;
+        sl->iter = st->iter;
+        sl->jj = st->jj;
+        sl->maxit = st->maxit;
+        sl->s = s;
+        sl->method = st->method;
+        sl->prow = st->prow;
+        sl->conjP = st->conjP;
+        sl->user_omega = st->user_omega;
+        sl->n_omega = st->n_omega;
+        sl->inispace = st->inispace;
+        sl->rv_cap = st->rv_cap;
+        sl->H = st->H;
+        sl->nritz = st->nritz;
+    }
+}
+
+// the sums of reduce_partials, bit for bit, by 256 threads (nparts <=
+// FOLD_PARTS): a wavefront takes the shares of wavefronts wid, wid + 4, ... of
+// the 1024-thread kernel.  scr: nv * 16 values.  No barrier at the end.
+template <class T>
+__device__ inline void fold_sums(const T *__restrict__ partials, int nparts, int nv, T *scr) {
+    constexpr int NW = FIN_THREADS / WAVE;
+    const int lane = threadIdx.x % WAVE, wid = threadIdx.x / WAVE;
+    for (int v = wid; v < NW; v += 256 / WAVE)
+        for (int q = 0; q < nv; q++) {
+            T a = T(0);
+            if (v * WAVE < nparts) {
+                for (int p = v * WAVE + lane; p < nparts; p += FIN_THREADS) a = a + partials[(long)q * nparts + p];
+                a = wave_sum(a);
+            }
+            if (lane == 0) scr[q * NW + v] = a;
+        }
+}
+// value q of fold_sums, after a barrier
+template <class T>
+__device__ inline T fold_value(const T *scr, int q) {
+    constexpr int NW = FIN_THREADS / WAVE;
+    T t = scr[q * NW];
+    for (int w = 1; w < NW; w++) t = t + scr[q * NW + w];
+    return t;
+}
+// in -> LDS; only workgroup 0 keeps the Hessenberg output
+template <class T>
+__device__ inline void fold_load(const Slot<T> *in, Slot<T> *sl) {
+    static_assert(sizeof(Slot<T>) % 8 == 0, "whole words");
+    const unsigned long long *a = (const unsigned long long *)in;
+    unsigned long long *b = (unsigned long long *)sl;
+    for (int i = threadIdx.x; i < (int)(sizeof(Slot<T>) / 8); i += 256) b[i] = a[i];
+}
+template <class T>
+__device__ inline void fold_store(const Slot<T> *sl, Slot<T> *out) {
+    if (blockIdx.x != 0) return;
+    const unsigned long long *a = (const unsigned long long *)sl;
+    unsigned long long *b = (unsigned long long *)out;
+    for (int i = threadIdx.x; i < (int)(sizeof(Slot<T>) / 8); i += 256) b[i] = a[i];
+}
+
+// scalar_cycle of the previous cycle (npin 0: none, the first cycle), then
+// k_form_u for U(:,0)
+template <class T>
+__global__ __launch_bounds__(256) void k_form_u_fold(long n, const Slot<T> *in, Slot<T> *out, const T *pin, int npin,
+                                                     const T *__restrict__ r, const T *__restrict__ G,
+                                                     T *__restrict__ U, const T *__restrict__ m1, double *resvec) {
+    __shared__ Slot<T> sl;
+    __shared__ T scr[(FIN_S + 1) * (FIN_THREADS / WAVE)], red[FIN_S + 1];
+    fold_load(in, &sl);
+    const int prow = in->prow;
+    if (npin) fold_sums(pin, npin, 1 + prow, scr);
+    __syncthreads();
+    if (threadIdx.x < WAVE && npin && sl.info < 0) {
+        if (threadIdx.x <= prow) red[threadIdx.x] = fold_value(scr, threadIdx.x);
+        wave_fence();
+        wave_cycle(&sl, sl.M, FIN_S, red, blockIdx.x == 0 ? resvec : nullptr, (int)threadIdx.x);
+    }
+    __syncthreads();
+    fold_store(&sl, out);
+    if (sl.info >= 0) return;
+    const int s = sl.s, jj = sl.jj;
+    const T om = sl.om;
+    if (jj > 0) {
+        GRID_LOOP(q, n) {
+            T v = r[q];
+            for (int i = 0; i < s; i++) v = fmaT(-sl.gamma[i], G[(long)i * n + q], v);
+            T t = om * precon_div(v, m1, q);
+            for (int i = 0; i < s; i++) t = fmaT(sl.gamma[i], U[(long)i * n + q], t);
+            U[q] = t;
+        }
+    } else if (!sl.inispace) {
+        GRID_LOOP(q, n) U[q] = precon_div(r[q], m1, q);
+    }
+}
+
+// scalar_norm of the previous inner step (npn 0: none), scalar_mu, then
+// k_orth_update.  S4: s <= 4, where a thread's first row is loaded before the
+// reductions' barriers.
+template <class T, bool S4>
+__global__ __launch_bounds__(256) void k_orth_fold(long n, int k, const Slot<T> *in, Slot<T> *out, const T *pmu,
+                                                   int npmu, const T *pn, int npn, T *__restrict__ G,
+                                                   T *__restrict__ U, T *__restrict__ r, T *__restrict__ x,
+                                                   const T *__restrict__ m1, double *resvec, T *partials) {
+    __shared__ Slot<T> sl;
+    __shared__ T scr[(FIN_S + 1) * (FIN_THREADS / WAVE)], red[FIN_S + 1], lds[4];
+    fold_load(in, &sl);
+    const int prow = in->prow, s = in->s, jj = in->jj;
+    const bool next = (k + 1 < s);
+    const long q0 = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const bool cols = next && jj > 0;   // columns beyond k are read
+    T gi[4], ui[4], g0 = T(0), u0 = T(0), r0 = T(0), x0 = T(0);
+    if constexpr (S4) {
+        const long q = q0 < n ? q0 : 0;
+        g0 = G[(long)k * n + q];
+        u0 = U[(long)k * n + q];
+        r0 = r[q];
+        x0 = x[q];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const bool want = i < k || (i > k && i < s && cols);
+            gi[i] = want ? G[(long)i * n + q] : T(0);
+            ui[i] = want ? U[(long)i * n + q] : T(0);
+        }
+    }
+    fold_sums(pmu, npmu, prow, scr);
+    if (npn) fold_sums(pn, npn, 1, scr + prow * (FIN_THREADS / WAVE));
+    __syncthreads();
+    if (threadIdx.x < WAVE && sl.info < 0) {
+        if (blockIdx.x != 0 && threadIdx.x == 0) sl.H = nullptr;
+        if (threadIdx.x < prow + (npn ? 1 : 0)) red[threadIdx.x] = fold_value(scr, threadIdx.x);
+        wave_fence();
+        if (npn && threadIdx.x == 0) scalar_norm(&sl, sqrt(sre(red[prow])), blockIdx.x == 0 ? resvec : nullptr);
+        wave_fence();
+        if (sl.info < 0) wave_mu(&sl, sl.M, FIN_S, k, red, (int)threadIdx.x);
+    }
+    __syncthreads();
+    fold_store(&sl, out);
+    if (sl.info >= 0) return;
+    const T beta = sl.beta[k], om = sl.om;
+    const int ini = sl.inispace;
+    T e[1] = {T(0)};
+    GRID_LOOP(q, n) {
+        T gk, uk, rq, xq;
+        if (S4 && q == q0) {
+            gk = g0;
+            uk = u0;
+            rq = r0;
+            xq = x0;
+        } else {
+            gk = G[(long)k * n + q];
+            uk = U[(long)k * n + q];
+            rq = r[q];
+            xq = x[q];
+            if constexpr (S4) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const bool want = i < k || (i > k && i < s && cols);
+                    gi[i] = want ? G[(long)i * n + q] : T(0);
+                    ui[i] = want ? U[(long)i * n + q] : T(0);
+                }
+            }
+        }
+        if constexpr (S4) {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (i < k) {
+                    gk = fmaT(-sl.alpha[i], gi[i], gk);
+                    uk = fmaT(-sl.alpha[i], ui[i], uk);
+                }
+        } else {
+            for (int i = 0; i < k; i++) {
+                gk = fmaT(-sl.alpha[i], G[(long)i * n + q], gk);
+                uk = fmaT(-sl.alpha[i], U[(long)i * n + q], uk);
+            }
+        }
+        G[(long)k * n + q] = gk;
+        U[(long)k * n + q] = uk;
+        rq = fmaT(-beta, gk, rq);
+        x[q] = fmaT(beta, uk, xq);
+        r[q] = rq;
+        e[0] = e[0] + T(Tr<T>::abs2(rq));
+        if (next) {
+            if (jj > 0) {
+                T v = rq;
+                if constexpr (S4) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        if (i > k && i < s) v = fmaT(-sl.gamma[i], gi[i], v);
+                } else {
+                    for (int i = k + 1; i < s; i++) v = fmaT(-sl.gamma[i], G[(long)i * n + q], v);
+                }
+                T t = om * precon_div(v, m1, q);
+                if constexpr (S4) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        if (i > k && i < s) t = fmaT(sl.gamma[i], ui[i], t);
+                } else {
+                    for (int i = k + 1; i < s; i++) t = fmaT(sl.gamma[i], U[(long)i * n + q], t);
+                }
+                U[(long)(k + 1) * n + q] = t;
+            } else if (!ini) {
+                U[(long)(k + 1) * n + q] = precon_div(rq, m1, q);
+            }
+        }
+    }
+    block_sum<T, 1>(e, lds);
+    if (threadIdx.x == 0) partials[blockIdx.x] = e[0];
+}
+
+// scalar_norm of the last inner step, scalar_om, then k_omega_update
+template <class T, int NV>
+__global__ __launch_bounds__(256) void k_omega_fold(long n, const Slot<T> *in, Slot<T> *out, const T *pom, int npom,
+                                                    const T *pn, int npn, const T *omega, const T *v,
+                                                    const T *__restrict__ t, T *r, T *__restrict__ x,
+                                                    const T *__restrict__ P, int prow, int conjP, double *resvec,
+                                                    T *partials, int nparts) {
+    __shared__ Slot<T> sl;
+    __shared__ T scr[4 * (FIN_THREADS / WAVE)], red[4], lds[(NV + 1) * 4];
+    fold_load(in, &sl);
+    fold_sums(pom, npom, 3, scr);
+    fold_sums(pn, npn, 1, scr + 3 * (FIN_THREADS / WAVE));
+    __syncthreads();
+    if (threadIdx.x < WAVE && sl.info < 0) {
+        if (threadIdx.x < 4) red[threadIdx.x] = fold_value(scr, threadIdx.x);
+        wave_fence();
+        if (threadIdx.x == 0) {
+            scalar_norm(&sl, sqrt(sre(red[3])), blockIdx.x == 0 ? resvec : nullptr);
+            if (sl.info < 0) scalar_om(&sl, red, omega);
+        }
+    }
+    __syncthreads();
+    fold_store(&sl, out);
+    if (sl.info >= 0) return;
+    const T om = sl.om;
+    T e[NV + 1];
+#pragma unroll
+    for (int i = 0; i <= NV; i++) e[i] = T(0);
+    GRID_LOOP(q, n) {
+        const T vq = v[q];
+        const T rq = fmaT(-om, t[q], r[q]);
+        x[q] = fmaT(om, vq, x[q]);
+        r[q] = rq;
+        e[0] = e[0] + T(Tr<T>::abs2(rq));
+#pragma unroll
+        for (int i = 0; i < NV; i++)
+            if (i < prow) {
+                T p = P[q * prow + i];
+                if (conjP) p = Tr<T>::conj(p);
+                e[1 + i] = fmaT(p, rq, e[1 + i]);
+            }
+    }
+    block_sum<T, NV + 1>(e, lds);
+    if (threadIdx.x == 0)
+        for (int i = 0; i <= NV; i++) partials[(long)i * nparts + blockIdx.x] = e[i];
+}
+
+// the last slot's outcome back into the state, as the solve's end reads it
+template <class T>
+__global__ void k_fold_done(const Slot<T> *sl, State<T> *st) {
+    st->info = sl->info;
+    st->iter = sl->iter;
+    st->normr = sl->normr;
 }
 
 // ---------------------------------------------------------------------------
@@ -977,7 +1269,69 @@ int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOp
         LAUNCH_CHECK();
     };
 
-    auto enqueue_cycle = [&]() {
+    // The folded cycle while a workgroup's share of the partials stays small
+    // (the allocation-free solve has no room for the slots)
+    const bool fold = !ar && prow <= PDOT_MAX && s <= FIN_S && n <= FOLD_ROWS && enparts <= FOLD_PARTS && gv <= FOLD_PARTS;
+    // slots of the state, two norm buffers, and the omega step's partials
+    Buf bslot, bpn, bpc;
+    Slot<T> *slot = nullptr;
+    T *pn[2] = {nullptr, nullptr}, *pc = nullptr;
+    if (fold) {
+        bslot = Buf(sizeof(Slot<T>) * (s + 2));
+        bpn = Buf(sizeof(T) * 2 * gv);
+        bpc = Buf(sizeof(T) * (1 + PDOT_MAX) * gv);
+        slot = bslot.as<Slot<T>>();
+        pn[0] = bpn.as<T>();
+        pn[1] = pn[0] + gv;
+        pc = bpc.as<T>();
+        hipLaunchKernelGGL((k_fold_init<T>), dim3(1), dim3(64), 0, stream, st, slot);
+        LAUNCH_CHECK();
+    }
+    const int *info_p = fold ? &slot[0].info : info;   // what the host polls
+    int fold_first = 1;
+    auto enqueue_fold = [&]() {
+        // slot i is read by the i-th streaming kernel of the cycle, which
+        // writes slot i + 1; the last writes slot 0.  The first cycle has no
+        // omega step behind it: its partials count is zero.
+        hipLaunchKernelGGL((k_form_u_fold<T>), dim3(gv), dim3(256), 0, stream, n, (const Slot<T> *)slot, slot + 1,
+                           (const T *)pc, fold_first ? 0 : gv, (const T *)r, (const T *)G, U, m1, resvec);
+        LAUNCH_CHECK();
+        for (int k = 0; k < s; k++) {
+            const Slot<T> *in = slot + 1 + k;
+            Slot<T> *out = slot + 2 + k;
+            op_apply<T>(A, U + (long)k * n, G + (long)k * n, w1, w2, EPI_PDOT, epd, &in->info, stream);
+            prereduce(prow);
+            const T *pin = k > 0 ? pn[(k - 1) % 2] : nullptr;
+            if (s <= 4)
+                hipLaunchKernelGGL((k_orth_fold<T, true>), dim3(gv), dim3(256), 0, stream, n, k, in, out, epart, enparts,
+                                   pin, k > 0 ? gv : 0, G, U, r, x, m1, resvec, pn[k % 2]);
+            else
+                hipLaunchKernelGGL((k_orth_fold<T, false>), dim3(gv), dim3(256), 0, stream, n, k, in, out, epart,
+                                   enparts, pin, k > 0 ? gv : 0, G, U, r, x, m1, resvec, pn[k % 2]);
+            LAUNCH_CHECK();
+        }
+        const Slot<T> *in = slot + 1 + s;
+        if (m1) {
+            hipLaunchKernelGGL((k_form_v<T>), dim3(gv), dim3(256), 0, stream, n, &in->info, r, m1, v);
+            LAUNCH_CHECK();
+        }
+        op_apply<T>(A, v, t, w1, w2, EPI_OMEGA, eom, &in->info, stream);
+        prereduce(3);
+#define OF(NV)                                                                                                       \
+    hipLaunchKernelGGL((k_omega_fold<T, NV>), dim3(gv), dim3(256), 0, stream, n, in, slot, epart, enparts,           \
+                       (const T *)pn[(s - 1) % 2], gv, (const T *)omega_d, (const T *)v, (const T *)t, r, x,         \
+                       (const T *)P, prow, conjP, resvec, pc, gv)
+        if (prow <= 1) OF(1);
+        else if (prow <= 2) OF(2);
+        else if (prow <= 4) OF(4);
+        else if (prow <= 8) OF(8);
+        else OF(16);
+#undef OF
+        LAUNCH_CHECK();
+        fold_first = 0;
+    };
+
+    auto enqueue_plain = [&]() {
         hipLaunchKernelGGL((k_form_u<T>), dim3(gv), dim3(256), 0, stream, n, 0, st, r, G, U, m1);
         LAUNCH_CHECK();
         for (int k = 0; k < s; k++) {
@@ -999,7 +1353,7 @@ int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOp
             LAUNCH_CHECK();
         }
         if (m1) {
-            hipLaunchKernelGGL((k_form_v<T>), dim3(gv), dim3(256), 0, stream, n, st, r, m1, v);
+            hipLaunchKernelGGL((k_form_v<T>), dim3(gv), dim3(256), 0, stream, n, info, r, m1, v);
             LAUNCH_CHECK();
         }
         op_apply<T>(A, v, t, w1, w2, EPI_OMEGA, eom, info, stream);
@@ -1009,6 +1363,11 @@ int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOp
         launch_omega_update<T>(n, st, v, t, r, x, P, prow, conjP, part, stream);
         hipLaunchKernelGGL((k_fin_cycle<T>), dim3(1), dim3(FIN_THREADS), 0, stream, st, part, gv, resvec);
         LAUNCH_CHECK();
+    };
+
+    auto enqueue_cycle = [&]() {
+        if (fold) enqueue_fold();
+        else enqueue_plain();
     };
 
     // enqueue cycles, polling the device flag one cycle behind (pinned
@@ -1026,7 +1385,7 @@ int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOp
     const bool use_graph = !ar && !tm.enabled && (o.graph_mode == 1 || (o.graph_mode == 0 && n <= (1L << 21)));
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
-    if (use_graph) {
+    auto capture = [&]() {
         HIP_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeRelaxed));
         try {
             enqueue_cycle();
@@ -1038,11 +1397,14 @@ int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOp
         }
         HIP_TRY(hipStreamEndCapture(stream, &graph));
         HIP_TRY(hipGraphInstantiate(&gexec, graph, nullptr, nullptr, 0));
-    }
+    };
     bool done = false;
     try {
         for (long c = 0; c < max_cycles && !done; c++) {
-            if (use_graph) HIP_TRY(hipGraphLaunch(gexec, stream));
+            // the first folded cycle differs from the others in an argument:
+            // it runs as launches, while the host captures the others
+            if (use_graph && !gexec && (c > 0 || !fold)) capture();
+            if (gexec) HIP_TRY(hipGraphLaunch(gexec, stream));
             else enqueue_cycle();
             if (ar) {
                 HIP_TRY(hipMemcpyAsync(&h_info[0], info, sizeof(int), hipMemcpyDeviceToHost, stream));
@@ -1050,12 +1412,19 @@ int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOp
                 if (h_info[0] >= 0) done = true;
                 continue;
             }
-            HIP_TRY(hipMemcpyAsync(&h_info[c % 2], info, sizeof(int), hipMemcpyDeviceToHost, stream));
+            HIP_TRY(hipMemcpyAsync(&h_info[c % 2], info_p, sizeof(int), hipMemcpyDeviceToHost, stream));
             HIP_TRY(hipEventRecord(pe[c % 2], stream));
             if (c >= 1) {
                 HIP_TRY(hipEventSynchronize(pe[(c - 1) % 2]));
                 if (h_info[(c - 1) % 2] >= 0) done = true;
             }
+        }
+        if (fold) {   // the last omega step's norm, and the outcome into the state
+            hipLaunchKernelGGL((k_form_u_fold<T>), dim3(gv), dim3(256), 0, stream, n, (const Slot<T> *)slot, slot + 1,
+                               (const T *)pc, gv, (const T *)r, (const T *)G, U, m1, resvec);
+            LAUNCH_CHECK();
+            hipLaunchKernelGGL((k_fold_done<T>), dim3(1), dim3(1), 0, stream, (const Slot<T> *)(slot + 1), st);
+            LAUNCH_CHECK();
         }
         // final true residual (idrs.inc:304-310)
         op_apply<T>(A, x, tmp, w1, w2, EPI_NONE, none, nullptr, stream);
