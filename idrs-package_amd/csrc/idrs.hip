@@ -612,20 +612,42 @@ __global__ void k_fold_init(const State<T> *st, Slot<T> *sl) {
 
 // the sums of reduce_partials, bit for bit, by 256 threads (nparts <=
 // FOLD_PARTS): a wavefront takes the shares of wavefronts wid, wid + 4, ... of
-// the 1024-thread kernel.  scr: nv * 16 values.  No barrier at the end.
+// the 1024-thread kernel, four values at a time with all their loads in
+// flight.  scr: nv * 16 values.  No barrier at the end.
 template <class T>
 __device__ inline void fold_sums(const T *__restrict__ partials, int nparts, int nv, T *scr) {
-    constexpr int NW = FIN_THREADS / WAVE;
+    constexpr int NW = FIN_THREADS / WAVE, NR = 256 / WAVE, V = NW / NR;
     const int lane = threadIdx.x % WAVE, wid = threadIdx.x / WAVE;
-    for (int v = wid; v < NW; v += 256 / WAVE)
-        for (int q = 0; q < nv; q++) {
-            T a = T(0);
-            if (v * WAVE < nparts) {
-                for (int p = v * WAVE + lane; p < nparts; p += FIN_THREADS) a = a + partials[(long)q * nparts + p];
-                a = wave_sum(a);
+    for (int q0 = 0; q0 < nv; q0 += 4) {
+        T a[V][4];
+#pragma unroll
+        for (int j = 0; j < V; j++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int p = (wid + j * NR) * WAVE + lane;
+                const bool ok = q0 + q < nv && p < nparts;
+                a[j][q] = ok ? partials[(long)(q0 + q) * nparts + p] : T(0);
             }
-            if (lane == 0) scr[q * NW + v] = a;
+        if (nparts > FIN_THREADS)
+#pragma unroll
+            for (int j = 0; j < V; j++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int p = (wid + j * NR) * WAVE + lane + FIN_THREADS;
+                    if (q0 + q < nv && p < nparts) a[j][q] = a[j][q] + partials[(long)(q0 + q) * nparts + p];
+                }
+#pragma unroll
+        for (int j = 0; j < V; j++) {
+            if ((wid + j * NR) * WAVE < nparts)
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    if (q0 + q < nv) a[j][q] = wave_sum(a[j][q]);
+            if (lane == 0)
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    if (q0 + q < nv) scr[(q0 + q) * NW + wid + j * NR] = a[j][q];
         }
+    }
 }
 // value q of fold_sums, after a barrier
 template <class T>
@@ -654,13 +676,12 @@ __device__ inline void fold_store(const Slot<T> *sl, Slot<T> *out) {
 // scalar_cycle of the previous cycle (npin 0: none, the first cycle), then
 // k_form_u for U(:,0)
 template <class T>
-__global__ __launch_bounds__(256) void k_form_u_fold(long n, const Slot<T> *in, Slot<T> *out, const T *pin, int npin,
+__global__ __launch_bounds__(256) void k_form_u_fold(long n, int prow, const Slot<T> *in, Slot<T> *out, const T *pin, int npin,
                                                      const T *__restrict__ r, const T *__restrict__ G,
                                                      T *__restrict__ U, const T *__restrict__ m1, double *resvec) {
     __shared__ Slot<T> sl;
     __shared__ T scr[(FIN_S + 1) * (FIN_THREADS / WAVE)], red[FIN_S + 1];
     fold_load(in, &sl);
-    const int prow = in->prow;
     if (npin) fold_sums(pin, npin, 1 + prow, scr);
     __syncthreads();
     if (threadIdx.x < WAVE && npin && sl.info < 0) {
@@ -690,14 +711,15 @@ __global__ __launch_bounds__(256) void k_form_u_fold(long n, const Slot<T> *in, 
 // k_orth_update.  S4: s <= 4, where a thread's first row is loaded before the
 // reductions' barriers.
 template <class T, bool S4>
-__global__ __launch_bounds__(256) void k_orth_fold(long n, int k, const Slot<T> *in, Slot<T> *out, const T *pmu,
-                                                   int npmu, const T *pn, int npn, T *__restrict__ G,
+__global__ __launch_bounds__(256) void k_orth_fold(long n, int k, int s, int prow, int first, const Slot<T> *in,
+                                                   Slot<T> *out, const T *pmu, int npmu, const T *pn, int npn,
+                                                   T *__restrict__ G,
                                                    T *__restrict__ U, T *__restrict__ r, T *__restrict__ x,
                                                    const T *__restrict__ m1, double *resvec, T *partials) {
     __shared__ Slot<T> sl;
     __shared__ T scr[(FIN_S + 1) * (FIN_THREADS / WAVE)], red[FIN_S + 1], lds[4];
     fold_load(in, &sl);
-    const int prow = in->prow, s = in->s, jj = in->jj;
+    const int jj = first ? 0 : 1;
     const bool next = (k + 1 < s);
     const long q0 = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const bool cols = next && jj > 0;   // columns beyond k are read
@@ -1293,7 +1315,7 @@ int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOp
         // slot i is read by the i-th streaming kernel of the cycle, which
         // writes slot i + 1; the last writes slot 0.  The first cycle has no
         // omega step behind it: its partials count is zero.
-        hipLaunchKernelGGL((k_form_u_fold<T>), dim3(gv), dim3(256), 0, stream, n, (const Slot<T> *)slot, slot + 1,
+        hipLaunchKernelGGL((k_form_u_fold<T>), dim3(gv), dim3(256), 0, stream, n, prow, (const Slot<T> *)slot, slot + 1,
                            (const T *)pc, fold_first ? 0 : gv, (const T *)r, (const T *)G, U, m1, resvec);
         LAUNCH_CHECK();
         for (int k = 0; k < s; k++) {
@@ -1303,10 +1325,10 @@ int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOp
             prereduce(prow);
             const T *pin = k > 0 ? pn[(k - 1) % 2] : nullptr;
             if (s <= 4)
-                hipLaunchKernelGGL((k_orth_fold<T, true>), dim3(gv), dim3(256), 0, stream, n, k, in, out, epart, enparts,
+                hipLaunchKernelGGL((k_orth_fold<T, true>), dim3(gv), dim3(256), 0, stream, n, k, s, prow, fold_first, in, out, epart, enparts,
                                    pin, k > 0 ? gv : 0, G, U, r, x, m1, resvec, pn[k % 2]);
             else
-                hipLaunchKernelGGL((k_orth_fold<T, false>), dim3(gv), dim3(256), 0, stream, n, k, in, out, epart,
+                hipLaunchKernelGGL((k_orth_fold<T, false>), dim3(gv), dim3(256), 0, stream, n, k, s, prow, fold_first, in, out, epart,
                                    enparts, pin, k > 0 ? gv : 0, G, U, r, x, m1, resvec, pn[k % 2]);
             LAUNCH_CHECK();
         }
@@ -1420,7 +1442,7 @@ int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOp
             }
         }
         if (fold) {   // the last omega step's norm, and the outcome into the state
-            hipLaunchKernelGGL((k_form_u_fold<T>), dim3(gv), dim3(256), 0, stream, n, (const Slot<T> *)slot, slot + 1,
+            hipLaunchKernelGGL((k_form_u_fold<T>), dim3(gv), dim3(256), 0, stream, n, prow, (const Slot<T> *)slot, slot + 1,
                                (const T *)pc, gv, (const T *)r, (const T *)G, U, m1, resvec);
             LAUNCH_CHECK();
             hipLaunchKernelGGL((k_fold_done<T>), dim3(1), dim3(1), 0, stream, (const Slot<T> *)(slot + 1), st);
