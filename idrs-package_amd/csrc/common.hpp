@@ -260,21 +260,34 @@ template <class T>
 __device__ inline void reduce_partials(const T *__restrict__ partials, int nparts, int nv, T *out) {
     __shared__ T lds[MAX_RED * (FIN_THREADS / WAVE)];
     const int nw = blockDim.x / WAVE, lane = threadIdx.x % WAVE, wid = threadIdx.x / WAVE;
-    for (int q = 0; q < nv; q++) {
-        // four independent partial sums per thread keep several loads in flight
-        T a0 = T(0), a1 = T(0), a2 = T(0), a3 = T(0);
-        const T *pq = partials + (long)q * nparts;
+    // four values at a time, each with four independent partial sums per
+    // thread: their loads are in flight together (8 values of 3900 partials
+    // one after another took 13 us)
+    for (int q0 = 0; q0 < nv; q0 += 4) {
+        T a[4][4];
+        const T *pq[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            pq[j] = partials + (long)min(q0 + j, nv - 1) * nparts;
+#pragma unroll
+            for (int i = 0; i < 4; i++) a[j][i] = T(0);
+        }
         int p = threadIdx.x;
         const int step = blockDim.x;
-        for (; p + 3 * step < nparts; p += 4 * step) {
-            a0 = a0 + pq[p];
-            a1 = a1 + pq[p + step];
-            a2 = a2 + pq[p + 2 * step];
-            a3 = a3 + pq[p + 3 * step];
+        for (; p + 3 * step < nparts; p += 4 * step)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) a[j][i] = a[j][i] + pq[j][p + i * step];
+        for (; p < nparts; p += step)
+#pragma unroll
+            for (int j = 0; j < 4; j++) a[j][0] = a[j][0] + pq[j][p];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (q0 + j >= nv) break;
+            const T v = wave_sum((a[j][0] + a[j][1]) + (a[j][2] + a[j][3]));
+            if (lane == 0) lds[(q0 + j) * (FIN_THREADS / WAVE) + wid] = v;
         }
-        for (; p < nparts; p += step) a0 = a0 + pq[p];
-        T v = wave_sum((a0 + a1) + (a2 + a3));
-        if (lane == 0) lds[q * (FIN_THREADS / WAVE) + wid] = v;
     }
     __syncthreads();
     if (threadIdx.x < nv) {
