@@ -1079,11 +1079,14 @@ int autotune_group(DevMatrix &K, int reps, hipStream_t st, std::vector<std::pair
         if (K.fmt == DevFmt::CRS) {
             const int g0 = K.group == 1 ? 2 : K.group;
             float best_ms = 0.f;
-            // the sliced copy is a candidate when its padding stays within
-            // 1/4 of the stored entries (built for the timing, kept if chosen)
+            // the sliced copy is a candidate when its padding (never read)
+            // stays within the stored entries (built for the timing, kept if
+            // chosen): the transpose of a random matrix, whose rows vary in
+            // length, is 1.6 times padded and still faster than lanes per row
+            // (16 entries a row, 1e6 rows: 135 against 173 us)
             bool sell_ok = false;
             if (!K.sell && K.nnz > 0) build_sell(K, st);
-            if (K.sell) sell_ok = K.sell->nent <= K.nnz + K.nnz / 4;
+            if (K.sell) sell_ok = K.sell->nent <= 2 * K.nnz;
             if (sell_ok) {   // the sliced layout is timed with its row code
                 K.group = 1;
                 Operator own;
