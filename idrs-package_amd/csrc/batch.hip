@@ -9,8 +9,8 @@
 // per system).  A system that has met its tolerance (or maxit, or broke down)
 // is frozen: its tiles return at once in every later launch, so the batch's
 // cost per cycle falls as systems finish.  The host enqueues whole cycles and
-// polls a single "all finished" flag one cycle behind, like the
-// single-system driver.
+// polls one flag per system one cycle behind, like the single-system
+// driver.
 #include "batch.hpp"
 #include "block.hpp"
 
@@ -249,113 +249,170 @@ __global__ __launch_bounds__(BT) void k_bfin_f(BV bv, State<T> *st, const T *par
 }
 
 // ---------------------------------------------------------------------------
-// per-system reduction + scalar steps of the cycle
+// The cycle (idrs.inc:155-299) per tile, folded as the single solve's
+// (idrs.hip): the per-system sums and scalar steps run at the start of the tile kernel that uses them, in every
+// tile of the system, from the system's state slot that the kernel before
+// wrote; the system's first tile writes the next slot.  The sums are
+// reduce_system's, so the results are the same bits with half the launches
+// (the one-workgroup-per-system kernels took 4 to 5 us each, most of it
+// latency: 96 systems of 64^2 to 180^2 rows, IDR(2), 43 -> 38.3 ms).
 // ---------------------------------------------------------------------------
 template <class T>
-__global__ __launch_bounds__(BT) void k_bfin_mu(BV bv, int k, State<T> *st, const T *partials) {
-    State<T> *S = st + blockIdx.x;
-    if (S->info >= 0) return;
-    __shared__ T red[SMAX], sM[PDOT_MAX * PDOT_MAX];
-    const int s = S->s;
-    for (int i = threadIdx.x; i < s * s; i += BT) sM[i] = S->M[i % s + SMAX * (i / s)];
-    reduce_system(bv, partials, S->prow, red);
-    if (threadIdx.x < WAVE) wave_mu(S, sM, s, k, red, (int)threadIdx.x);
-}
+using BSlot = State<T, PDOT_MAX>;
 
 template <class T>
-__global__ __launch_bounds__(BT) void k_bfin_norm(BV bv, State<T> *st, const T *partials) {
-    State<T> *S = st + blockIdx.x;
-    if (S->info >= 0) return;
-    __shared__ T red[1];
-    reduce_system(bv, partials, 1, red);
-    if (threadIdx.x == 0) scalar_norm(S, sqrt(sre(red[0])), (double *)nullptr);
-}
-
-template <class T>
-__global__ __launch_bounds__(BT) void k_bfin_om(BV bv, State<T> *st, const T *partials, const T *omega) {
-    State<T> *S = st + blockIdx.x;
-    if (S->info >= 0) return;
-    __shared__ T red[3];
-    reduce_system(bv, partials, 3, red);
-    if (threadIdx.x == 0) scalar_om(S, red, omega);
-}
-
-template <class T>
-__global__ __launch_bounds__(BT) void k_bfin_cycle(BV bv, State<T> *st, const T *partials) {
-    State<T> *S = st + blockIdx.x;
-    if (S->info >= 0) return;
-    __shared__ T red[SMAX + 1], sM[PDOT_MAX * PDOT_MAX];
-    const int s = S->s;
-    for (int i = threadIdx.x; i < s * s; i += BT) sM[i] = S->M[i % s + SMAX * (i / s)];
-    reduce_system(bv, partials, 1 + S->prow, red);
-    if (threadIdx.x < WAVE) wave_cycle(S, sM, s, red, (double *)nullptr, (int)threadIdx.x);
-}
-
-// flag[0] = 1 when every system has finished; flag[1 + k] = 1 while system
-// k runs
-template <class T>
-__global__ __launch_bounds__(BT) void k_bdone(int nsys, const State<T> *st, int *flag) {
-    __shared__ int open;
-    if (threadIdx.x == 0) open = 0;
-    __syncthreads();
-    int mine = 0;
-    for (int b = threadIdx.x; b < nsys; b += BT) {
-        const int live = (st[b].info < 0) ? 1 : 0;
-        flag[1 + b] = live;
-        mine |= live;
+__global__ __launch_bounds__(BT) void k_bfold_init(const State<T> *st, BSlot<T> *slot) {
+    const State<T> *S = st + blockIdx.x;
+    BSlot<T> *sl = slot + blockIdx.x;
+    for (int i = threadIdx.x; i < PDOT_MAX; i += BT) sl->f[i] = i < S->s ? S->f[i] : T(0);
+    for (int i = threadIdx.x; i < PDOT_MAX * PDOT_MAX; i += BT) sl->M[i] = T(0);
+    if (threadIdx.x == 0) {
+        sl->om = S->om;
+        sl->normb = S->normb;
+        sl->tolb = S->tolb;
+        sl->normr = S->normr;
+        sl->kappa = S->kappa;
+        sl->tol = S->tol;
+        sl->info = S->info;
+        sl->iter = S->iter;
+        sl->jj = S->jj;
+        sl->maxit = S->maxit;
+        sl->s = S->s;
+        sl->method = S->method;
+        sl->prow = S->prow;
+        sl->conjP = S->conjP;
+        sl->user_omega = S->user_omega;
+        sl->n_omega = S->n_omega;
+        sl->inispace = 0;
+        sl->rv_cap = 0;
+        sl->H = nullptr;
+        sl->nritz = 0;
     }
-    if (mine) atomicOr(&open, 1);
-    __syncthreads();
-    if (threadIdx.x == 0) flag[0] = open ? 0 : 1;
 }
 
-// ---------------------------------------------------------------------------
-// streaming kernels of the cycle (idrs.inc:155-299), per tile
-// ---------------------------------------------------------------------------
+// the outcomes back into the states
 template <class T>
-__global__ __launch_bounds__(BT) void k_bform_u(BV bv, long ntot, int k, const State<T> *st, const T *__restrict__ r,
+__global__ void k_bfold_done(int nsys, const BSlot<T> *slot, State<T> *st) {
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b >= nsys) return;
+    st[b].info = slot[b].info;
+    st[b].iter = slot[b].iter;
+    st[b].normr = slot[b].normr;
+}
+
+template <class T>
+__device__ inline void bslot_copy(const BSlot<T> *in, BSlot<T> *out) {
+    static_assert(sizeof(BSlot<T>) % 8 == 0, "whole words");
+    const unsigned long long *a = (const unsigned long long *)in;
+    unsigned long long *b = (unsigned long long *)out;
+    for (int i = threadIdx.x; i < (int)(sizeof(BSlot<T>) / 8); i += BT) b[i] = a[i];
+}
+
+// reduce_system's sums for system sys: four values' loads in flight; scr holds
+// 4 wavefronts' parts per value, bsum_value adds them after a barrier
+template <class T>
+__device__ inline void bsums(const BV &bv, int sys, const T *__restrict__ partials, int nv, T *scr) {
+    const int t0 = bv.tile0[sys], t1 = bv.tile0[sys + 1];
+    const int lane = threadIdx.x % WAVE, wid = threadIdx.x / WAVE;
+    for (int q0 = 0; q0 < nv; q0 += 4) {
+        T a[4] = {T(0), T(0), T(0), T(0)};
+        for (int t = t0 + threadIdx.x; t < t1; t += BT)
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                if (q0 + q < nv) a[q] = a[q] + partials[(long)(q0 + q) * bv.ntiles + t];
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (q0 + q < nv) {
+                a[q] = wave_sum(a[q]);
+                if (lane == 0) scr[(q0 + q) * (BT / WAVE) + wid] = a[q];
+            }
+    }
+}
+template <class T>
+__device__ inline T bsum_value(const T *scr, int q) {
+    T v = scr[q * (BT / WAVE)];
+    for (int w = 1; w < BT / WAVE; w++) v = v + scr[q * (BT / WAVE) + w];
+    return v;
+}
+
+// U(:,0) (idrs.inc:155-190)
+template <class T>
+__global__ __launch_bounds__(BT) void k_bform_u(BV bv, long ntot, const BSlot<T> *in, const T *__restrict__ r,
                                                 const T *__restrict__ G, T *__restrict__ U) {
-    const State<T> *S = st + bv.tile_sys[blockIdx.x];
+    const BSlot<T> *S = in + bv.tile_sys[blockIdx.x];
     if (S->info >= 0) return;
-    __shared__ T sg[SMAX];
-    const int s = S->s, jj = S->jj;
-    if (threadIdx.x < SMAX) sg[threadIdx.x] = S->gamma[threadIdx.x];
+    __shared__ T sg[PDOT_MAX];
+    const int s = S->s;
+    if (threadIdx.x < PDOT_MAX) sg[threadIdx.x] = S->gamma[threadIdx.x];
     __syncthreads();
     const T om = S->om;
-    if (jj > 0) {
+    if (S->jj > 0) {
         TILE_ROWS(q) {
             T v = r[q];
-            for (int i = k; i < s; i++) v = fmaT(-sg[i], G[(long)i * ntot + q], v);
+            for (int i = 0; i < s; i++) v = fmaT(-sg[i], G[(long)i * ntot + q], v);
             T t = om * v;
-            for (int i = k; i < s; i++) t = fmaT(sg[i], U[(long)i * ntot + q], t);
-            U[(long)k * ntot + q] = t;
+            for (int i = 0; i < s; i++) t = fmaT(sg[i], U[(long)i * ntot + q], t);
+            U[q] = t;
         }
     } else {
-        TILE_ROWS(q) U[(long)k * ntot + q] = r[q];
+        TILE_ROWS(q) U[q] = r[q];
     }
 }
 
+// the end of the cycle, one workgroup per system: scalar_cycle, and
+// live[k] = 1 while system k runs (its tiles may be dropped before the next
+// cycle, so this step reads the partials before they are)
 template <class T>
-__global__ __launch_bounds__(BT) void k_borth_update(BV bv, long ntot, int k, const State<T> *st, T *__restrict__ G,
-                                                     T *__restrict__ U, T *__restrict__ r, T *__restrict__ x,
-                                                     T *partials) {
-    const State<T> *S = st + bv.tile_sys[blockIdx.x];
-    if (S->info >= 0) return;
-    __shared__ T sa[SMAX], sg[SMAX], lds[BT / WAVE];
-    const int s = S->s, jj = S->jj;
-    if (threadIdx.x < SMAX) {
-        sa[threadIdx.x] = S->alpha[threadIdx.x];
-        sg[threadIdx.x] = S->gamma[threadIdx.x];
+__global__ __launch_bounds__(BT) void k_bcycle(BV bv, int prow, const BSlot<T> *in, BSlot<T> *out, const T *partials,
+                                               int *live) {
+    __shared__ BSlot<T> sl;
+    __shared__ T scr[(PDOT_MAX + 1) * (BT / WAVE)], red[PDOT_MAX + 1];
+    const int sys = blockIdx.x;
+    bslot_copy(in + sys, &sl);
+    bsums(bv, sys, partials, 1 + prow, scr);
+    __syncthreads();
+    if (threadIdx.x < WAVE && sl.info < 0) {
+        if (threadIdx.x <= prow) red[threadIdx.x] = bsum_value(scr, threadIdx.x);
+        wave_fence();
+        wave_cycle(&sl, sl.M, PDOT_MAX, red, (double *)nullptr, (int)threadIdx.x);
     }
     __syncthreads();
-    const T beta = S->beta[k], om = S->om;
+    bslot_copy(&sl, out + sys);
+    if (threadIdx.x == 0) live[sys] = sl.info < 0 ? 1 : 0;
+}
+
+// scalar_norm of the previous inner step (k > 0), scalar_mu, then G(:,k), U(:,k), r, x
+// and U(:,k+1)
+template <class T>
+__global__ __launch_bounds__(BT) void k_borth_fold(BV bv, long ntot, int k, int prow, const BSlot<T> *in, BSlot<T> *out,
+                                                   const T *pmu, const T *pn, T *__restrict__ G, T *__restrict__ U,
+                                                   T *__restrict__ r, T *__restrict__ x, T *partials) {
+    __shared__ BSlot<T> sl;
+    __shared__ T scr[(PDOT_MAX + 1) * (BT / WAVE)], red[PDOT_MAX + 1], lds[BT / WAVE];
+    const int sys = bv.tile_sys[blockIdx.x];
+    bslot_copy(in + sys, &sl);
+    bsums(bv, sys, pmu, prow, scr);
+    if (k > 0) bsums(bv, sys, pn, 1, scr + prow * (BT / WAVE));
+    __syncthreads();
+    if (threadIdx.x < WAVE && sl.info < 0) {
+        if (threadIdx.x < prow + (k > 0 ? 1 : 0)) red[threadIdx.x] = bsum_value(scr, threadIdx.x);
+        wave_fence();
+        if (k > 0 && threadIdx.x == 0) scalar_norm(&sl, sqrt(sre(red[prow])), (double *)nullptr);
+        wave_fence();
+        if (sl.info < 0) wave_mu(&sl, sl.M, PDOT_MAX, k, red, (int)threadIdx.x);
+    }
+    __syncthreads();
+    if (blockIdx.x == bv.tile0[sys]) bslot_copy(&sl, out + sys);
+    if (sl.info >= 0) return;
+    const int s = sl.s, jj = sl.jj;
+    const T beta = sl.beta[k], om = sl.om;
     const bool next = (k + 1 < s);
     T e[1] = {T(0)};
     TILE_ROWS(q) {
         T gk = G[(long)k * ntot + q], uk = U[(long)k * ntot + q];
         for (int i = 0; i < k; i++) {
-            gk = fmaT(-sa[i], G[(long)i * ntot + q], gk);
-            uk = fmaT(-sa[i], U[(long)i * ntot + q], uk);
+            gk = fmaT(-sl.alpha[i], G[(long)i * ntot + q], gk);
+            uk = fmaT(-sl.alpha[i], U[(long)i * ntot + q], uk);
         }
         G[(long)k * ntot + q] = gk;
         U[(long)k * ntot + q] = uk;
@@ -366,9 +423,9 @@ __global__ __launch_bounds__(BT) void k_borth_update(BV bv, long ntot, int k, co
         if (next) {
             if (jj > 0) {
                 T v = rq;
-                for (int i = k + 1; i < s; i++) v = fmaT(-sg[i], G[(long)i * ntot + q], v);
+                for (int i = k + 1; i < s; i++) v = fmaT(-sl.gamma[i], G[(long)i * ntot + q], v);
                 T t = om * v;
-                for (int i = k + 1; i < s; i++) t = fmaT(sg[i], U[(long)i * ntot + q], t);
+                for (int i = k + 1; i < s; i++) t = fmaT(sl.gamma[i], U[(long)i * ntot + q], t);
                 U[(long)(k + 1) * ntot + q] = t;
             } else {
                 U[(long)(k + 1) * ntot + q] = rq;
@@ -379,14 +436,31 @@ __global__ __launch_bounds__(BT) void k_borth_update(BV bv, long ntot, int k, co
     if (threadIdx.x == 0) partials[blockIdx.x] = e[0];
 }
 
+// scalar_norm of the last inner step, scalar_om, then r, x, ||r||^2 and P^T r
 template <class T, int NV>
-__global__ __launch_bounds__(BT) void k_bomega_update(BV bv, const State<T> *st, const T *__restrict__ t, T *r,
-                                                      T *__restrict__ x, const T *__restrict__ P, int prow, int conjP,
-                                                      T *partials) {
-    const State<T> *S = st + bv.tile_sys[blockIdx.x];
-    if (S->info >= 0) return;
-    __shared__ T lds[(NV + 1) * (BT / WAVE)];
-    const T om = S->om;
+__global__ __launch_bounds__(BT) void k_bomega_fold(BV bv, const BSlot<T> *in, BSlot<T> *out, const T *pom,
+                                                    const T *pn, const T *omega, const T *__restrict__ t, T *r,
+                                                    T *__restrict__ x, const T *__restrict__ P, int prow, int conjP,
+                                                    T *partials) {
+    __shared__ BSlot<T> sl;
+    __shared__ T scr[4 * (BT / WAVE)], red[4], lds[(NV + 1) * (BT / WAVE)];
+    const int sys = bv.tile_sys[blockIdx.x];
+    bslot_copy(in + sys, &sl);
+    bsums(bv, sys, pom, 3, scr);
+    bsums(bv, sys, pn, 1, scr + 3 * (BT / WAVE));
+    __syncthreads();
+    if (threadIdx.x < WAVE && sl.info < 0) {
+        if (threadIdx.x < 4) red[threadIdx.x] = bsum_value(scr, threadIdx.x);
+        wave_fence();
+        if (threadIdx.x == 0) {
+            scalar_norm(&sl, sqrt(sre(red[3])), (double *)nullptr);
+            if (sl.info < 0) scalar_om(&sl, red, omega);
+        }
+    }
+    __syncthreads();
+    if (blockIdx.x == bv.tile0[sys]) bslot_copy(&sl, out + sys);
+    if (sl.info >= 0) return;
+    const T om = sl.om;
     T e[NV + 1];
 #pragma unroll
     for (int i = 0; i <= NV; i++) e[i] = T(0);
@@ -494,7 +568,7 @@ void batch_idrs_solve(const Operator &A, int s, const T *b, T *x, const SolveOpt
 
     const size_t vb = sizeof(T) * (size_t)ntot;
     DBuf bG(vb * s), bU(vb * s), br(vb), bt(vb), bw1(vb), bw2(vb), btmp(vb), bP(vb * prow);
-    DBuf bpart(sizeof(T) * (size_t)MAX_NV * ntiles), bst(sizeof(State<T>) * nsys), bflag(sizeof(int) * (nsys + 1));
+    DBuf bpart(sizeof(T) * (size_t)MAX_NV * ntiles), bst(sizeof(State<T>) * nsys), bflag(sizeof(int) * nsys);
     // two sets of compacted tile lists (tiles of unfinished systems only),
     // alternated so a set is rewritten only when no queued launch reads it
     DBuf ctile_sys[2] = {DBuf(sizeof(int) * ntiles), DBuf(sizeof(int) * ntiles)};
@@ -579,34 +653,45 @@ void batch_idrs_solve(const Operator &A, int s, const T *b, T *x, const SolveOpt
     eom.r = r;
     eom.partials = part_d;
 
+    // State slots of the folded cycle, [slot][system]: inner step k reads
+    // slot k and writes slot k + 1, the omega step slot s + 1, the end of the
+    // cycle slot 0.  Two buffers of the inner steps' norm partials.
+    DBuf bslot(sizeof(BSlot<T>) * (size_t)nsys * (s + 2)), bpn(sizeof(T) * 2 * (size_t)ntiles);
+    BSlot<T> *slot = bslot.as<BSlot<T>>();
+    T *pn[2] = {bpn.as<T>(), bpn.as<T>() + ntiles};
+    hipLaunchKernelGGL((k_bfold_init<T>), gsys, dim3(BT), 0, stream, (const State<T> *)st, slot);
+    LAUNCH_CHECK();
+    static_assert(sizeof(BSlot<T>) % sizeof(int) == 0, "slot stride in ints");
+    live.stride = (int)(sizeof(BSlot<T>) / sizeof(int));
+    // the omega step's partials lie behind its product's three in part_d
+    T *pc = part_d + 3 * (size_t)ntiles;
+    static_assert(MAX_NV >= 3 + PDOT_MAX + 1, "room for both");
     auto enqueue_cycle = [&]() {
-        hipLaunchKernelGGL((k_bform_u<T>), gt, dim3(BT), 0, stream, bv, ntot, 0, (const State<T> *)st, (const T *)r,
+        hipLaunchKernelGGL((k_bform_u<T>), gt, dim3(BT), 0, stream, bv, ntot, (const BSlot<T> *)slot, (const T *)r,
                            (const T *)G, U);
         LAUNCH_CHECK();
         for (int k = 0; k < s; k++) {
+            BSlot<T> *in = slot + (size_t)nsys * k;
+            live.info = &in->info;
             op_apply<T>(A, U + (long)k * ntot, G + (long)k * ntot, w1, w2, EPI_PDOT, epd, nullptr, stream, &live);
-            hipLaunchKernelGGL((k_bfin_mu<T>), gsys, dim3(BT), 0, stream, bv, k, st, (const T *)part_d);
-            LAUNCH_CHECK();
-            hipLaunchKernelGGL((k_borth_update<T>), gt, dim3(BT), 0, stream, bv, ntot, k, (const State<T> *)st, G, U,
-                               r, x, part_d);
-            LAUNCH_CHECK();
-            hipLaunchKernelGGL((k_bfin_norm<T>), gsys, dim3(BT), 0, stream, bv, st, (const T *)part_d);
+            hipLaunchKernelGGL((k_borth_fold<T>), gt, dim3(BT), 0, stream, bv, ntot, k, prow, (const BSlot<T> *)in,
+                               in + nsys, (const T *)part_d, (const T *)pn[(k + 1) % 2], G, U, r, x, pn[k % 2]);
             LAUNCH_CHECK();
         }
+        const BSlot<T> *in = slot + (size_t)nsys * s;
+        BSlot<T> *out = slot + (size_t)nsys * (s + 1);
+        live.info = &in->info;
         op_apply<T>(A, r, t, w1, w2, EPI_OMEGA, eom, nullptr, stream, &live);
-        hipLaunchKernelGGL((k_bfin_om<T>), gsys, dim3(BT), 0, stream, bv, st, (const T *)part_d, (const T *)omega_d);
-        LAUNCH_CHECK();
-        NV_SWITCH(prow, k_bomega_update, gt, dim3(BT), 0, stream, bv, (const State<T> *)st, (const T *)t, r, x,
-                  (const T *)P, prow, conjP, part_d);
-        hipLaunchKernelGGL((k_bfin_cycle<T>), gsys, dim3(BT), 0, stream, bv, st, (const T *)part_d);
-        LAUNCH_CHECK();
-        hipLaunchKernelGGL((k_bdone<T>), dim3(1), dim3(BT), 0, stream, nsys, (const State<T> *)st, flag);
+        NV_SWITCH(prow, k_bomega_fold, gt, dim3(BT), 0, stream, bv, in, out, (const T *)part_d,
+                  (const T *)pn[(s - 1) % 2], (const T *)omega_d, (const T *)t, r, x, (const T *)P, prow, conjP, pc);
+        hipLaunchKernelGGL((k_bcycle<T>), gsys, dim3(BT), 0, stream, bv, prow, (const BSlot<T> *)out, slot,
+                           (const T *)pc, flag);
         LAUNCH_CHECK();
     };
 
-    // h_flag: two slots of nsys+1 ints (done flag, then one live flag per system)
+    // h_flag: two slots of one live flag per system
     int *h_flag = nullptr;
-    HIP_TRY(hipHostMalloc((void **)&h_flag, 2 * sizeof(int) * (nsys + 1), hipHostMallocDefault));
+    HIP_TRY(hipHostMalloc((void **)&h_flag, 2 * sizeof(int) * nsys, hipHostMallocDefault));
     int cset = 0;            // compacted set the next rewrite uses
     // Restricts every later tile launch to the unfinished systems' tiles once
     // they are at most 3/4 of the tiles launched so far.  Finished systems
@@ -693,16 +778,19 @@ void batch_idrs_solve(const Operator &A, int s, const T *b, T *x, const SolveOpt
             } else {
                 enqueue_cycle();
             }
-            int *slot = h_flag + (c % 2) * (nsys + 1);
-            HIP_TRY(hipMemcpyAsync(slot, flag, sizeof(int) * (nsys + 1), hipMemcpyDeviceToHost, stream));
+            HIP_TRY(hipMemcpyAsync(h_flag + (c % 2) * nsys, flag, sizeof(int) * nsys, hipMemcpyDeviceToHost, stream));
             HIP_TRY(hipEventRecord(pe[c % 2], stream));
             if (c >= 1) {
                 HIP_TRY(hipEventSynchronize(pe[(c - 1) % 2]));
-                const int *prev = h_flag + ((c - 1) % 2) * (nsys + 1);
-                if (prev[0]) done = true;
-                else compact(prev + 1);
+                const int *prev = h_flag + ((c - 1) % 2) * nsys;
+                done = std::none_of(prev, prev + nsys, [](int l) { return l != 0; });
+                if (!done) compact(prev);
             }
         }
+        // the outcomes into the states
+        hipLaunchKernelGGL((k_bfold_done<T>), dim3((nsys + 255) / 256), dim3(256), 0, stream, nsys,
+                           (const BSlot<T> *)slot, st);
+        LAUNCH_CHECK();
         // final true residuals over every system (idrs.inc:304-310)
         bv = bv_all;
         gt = dim3(ntiles);
