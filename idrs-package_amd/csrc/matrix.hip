@@ -449,23 +449,32 @@ static void with_args(const Operator &op, F &&f) {
 
 // The row code serves the products that sum a row in stored order: DIA, and
 // CRS in the sliced layout (lanes per row sum in another order).
-const RowCode *op_rowcode(const Operator &op) {
+const RowCode *op_rowcode(const Operator &op, bool offsets) {
     const DevMatrix &K = *op.K;
     if (K.fmt == DevFmt::CRS && !(K.group == 1 && K.sell)) return nullptr;
     if (op.values32 && op.seed != std::complex<double>(0.0, 0.0)) return nullptr;   // refused by with_args
     if (op.seed.imag() != 0.0) return nullptr;
-    return (op.sval ? op.rowcode : K.rowcode).get();
+    if (const RowCode *rc = (op.sval ? op.rowcode : K.rowcode).get()) return rc;
+    if (!offsets || op.values32 || op.values_complex() || K.fmt != DevFmt::CRS) return nullptr;
+    const void *sliced = op.sval ? op.sl_sval : K.sell->sl_val;
+    return sliced ? K.offcode.get() : nullptr;
 }
 
 // the argument block of a row-coded product of op (x, xs, z, a, y to be set)
-static SpmvArgs<double, double> rowcode_args(const Operator &op, int epi, const EpiArgs<double> &E) {
+static SpmvArgs<double, double> rowcode_args(const Operator &op, const RowCode &rc, int epi,
+                                             const EpiArgs<double> &E) {
     const DevMatrix &K = *op.K;
     auto A = base_args<double, double>(K, nullptr);
     A.has_seed = op.seed != std::complex<double>(0.0, 0.0);
     A.sdiag = op.which_precon == 1 ? (const double *)op.pdiag : nullptr;
     A.seed = op.seed.real();
-    const size_t vecs = 4 + (epi == EPI_PDOT ? (size_t)E.prow : 0);
-    A.keep = vecs * sizeof(double) * (size_t)K.nrows <= KEEP_BYTES;
+    size_t b = (4 + (epi == EPI_PDOT ? (size_t)E.prow : 0)) * sizeof(double) * (size_t)K.nrows;
+    if (!rc.values) {
+        A.val = (const double *)(op.sval ? op.sl_sval : K.sell->sl_val);
+        A.sl_ptr = K.sell->sl_ptr;
+        b += sizeof(double) * (size_t)K.sell->nent;
+    }
+    A.keep = b <= KEEP_BYTES;
     return A;
 }
 
@@ -474,8 +483,8 @@ void op_spmv(const Operator &op, const T *x, T xs, const T *z, T a, T *y, int ep
              const int *info, hipStream_t st, const TileCtx *tc) {
     const DevMatrix &K = *op.K;
     if constexpr (std::is_same<T, double>::value) {
-        if (const RowCode *rc = tc ? nullptr : op_rowcode(op)) {
-            SpmvArgs<double, double> A = rowcode_args(op, epi, E);
+        if (const RowCode *rc = tc ? nullptr : op_rowcode(op, true)) {
+            SpmvArgs<double, double> A = rowcode_args(op, *rc, epi, E);
             A.x = x; A.xs = xs; A.z = z; A.a = a; A.y = y;
             return rowcode_spmv(K, *rc, op.values32, A, E, epi, info, st);
         }
@@ -507,8 +516,8 @@ void op_spmv_cols(const Operator &op, int nc, long ld, const T *x, T xs, const T
             return C;
         };
         if constexpr (std::is_same<T, double>::value) {
-            if (const RowCode *rc = op_rowcode(op)) {
-                SpmvArgs<double, double> A = rowcode_args(op, EPI_NONE, none);
+            if (const RowCode *rc = op_rowcode(op, false)) {
+                SpmvArgs<double, double> A = rowcode_args(op, *rc, EPI_NONE, none);
                 A.xs = xs;
                 rowcode_cols(K, *rc, op.values32, A, columns(), st);
                 continue;
@@ -1023,11 +1032,17 @@ static void prepare_rowcode(const Operator &op, hipStream_t st) {
     static std::mutex mu;
     const DevMatrix &K = *op.K;
     std::lock_guard<std::mutex> g(mu);
-    bool &tried = op.sval ? op.rowcode_tried : K.rowcode_tried;
-    if (tried || (op.sval && K.tperm)) return;
     if (K.fmt == DevFmt::CRS && !(K.group == 1 && K.sell)) return;   // not read in that layout
-    (op.sval ? op.rowcode : K.rowcode) = make_rowcode(op, st);
-    tried = true;
+    bool &tried = op.sval ? op.rowcode_tried : K.rowcode_tried;
+    std::shared_ptr<RowCode> &rc = op.sval ? op.rowcode : K.rowcode;
+    if (!tried && !(op.sval && K.tperm)) {
+        rc = make_rowcode(op, true, st);
+        tried = true;
+    }
+    if (!rc && !K.offcode_tried) {
+        K.offcode = make_rowcode(op, false, st);
+        K.offcode_tried = true;
+    }
 }
 
 void op_prepare(const Operator &op, hipStream_t st) {

@@ -101,6 +101,9 @@ struct DevMatrix {
     // looked for, or values that change too often to look
     mutable std::shared_ptr<RowCode> rowcode;
     mutable bool rowcode_tried = false;
+    // code of the column offsets alone (CRS in the sliced layout)
+    mutable std::shared_ptr<RowCode> offcode;
+    mutable bool offcode_tried = false;
     ~DevMatrix();
 };
 

@@ -21,8 +21,11 @@ struct alignas(16) RowEntry {
 
 // Distinct row p: len[p] entries ent[p * width + k], in stored order.  ent32:
 // the values rounded to float (the FP32-value products), held as double.
+// Without values (ent holds the offsets alone) the code stands for the column
+// indices of a sliced CRS matrix, whose values are read as before.
 struct RowCode {
     int npat = 0, width = 0;
+    bool values = true;
     unsigned char *code = nullptr;   // nrows
     RowEntry *ent = nullptr, *ent32 = nullptr;
     int *len = nullptr;
@@ -30,12 +33,14 @@ struct RowCode {
 };
 
 // The row code of K with the values of op (K's own without diagonal scaling),
-// or null when K is not of a coded form or has more than ROWCODE_MAX distinct
-// rows.  Two passes over the matrix.
-std::shared_ptr<RowCode> make_rowcode(const Operator &op, hipStream_t st);
+// or of K's column offsets alone; null when K is not of a coded form or has
+// more than ROWCODE_MAX distinct rows.  Two passes over the matrix.
+std::shared_ptr<RowCode> make_rowcode(const Operator &op, bool values, hipStream_t st);
 
-// The code that the products of op use, or null: built by op_prepare
-const RowCode *op_rowcode(const Operator &op);
+// The code that the products of op use, or null: built by op_prepare.  One of
+// offsets alone only with 'offsets' (block products and FP32 values have no
+// kernel for it).
+const RowCode *op_rowcode(const Operator &op, bool offsets);
 
 // y = xs (K' x - seed x/sdiag) + a z with the epilogue, as dispatch_epi
 void rowcode_spmv(const DevMatrix &K, const RowCode &rc, bool f32, const SpmvArgs<double, double> &A,

@@ -28,8 +28,10 @@ def _box(dims, rows):
 
 
 # 32^3 is the fewest rows coded; 1 kind has 27 distinct rows, 9 kinds 243, 10
-# kinds more than a byte holds (the product stays uncoded: still the same bits)
-@pytest.mark.parametrize("dims,kinds", [((32, 32, 32), 1), ((33, 31, 37), 2), ((41, 29, 35), 9), ((41, 29, 35), 10)])
+# kinds more than a byte holds (DIA stays uncoded and sliced CRS codes its
+# column offsets alone: still the same bits), 1000 as with variable coefficients
+@pytest.mark.parametrize("dims,kinds", [((32, 32, 32), 1), ((33, 31, 37), 2), ((41, 29, 35), 9), ((41, 29, 35), 10),
+                                        ((35, 33, 31), 1000)])
 @pytest.mark.parametrize("fmt", ["dia", "crs"])
 @pytest.mark.parametrize("scaled", [False, True])
 def test_coded_products_are_the_same_bits(gpu, dims, kinds, fmt, scaled):
