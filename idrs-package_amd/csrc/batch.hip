@@ -488,10 +488,12 @@ __global__ __launch_bounds__(BT) void k_bomega_fold(BV bv, const BSlot<T> *in, B
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
+// a device buffer from the solvers' caching pool
 struct DBuf {
     void *p = nullptr;
-    explicit DBuf(size_t bytes) { HIP_TRY(hipMalloc(&p, bytes ? bytes : 1)); }
-    ~DBuf() { (void)hipFree(p); }
+    size_t bytes;
+    explicit DBuf(size_t b) : bytes(b) { p = pool_alloc(b); }
+    ~DBuf() { pool_free(p, bytes); }
     DBuf(const DBuf &) = delete;
     DBuf &operator=(const DBuf &) = delete;
     template <class V> V *as() const { return (V *)p; }

@@ -57,17 +57,19 @@ static int guarded(F &&f) {
     }
 }
 
-// device copies of host vectors for the host-pointer entry points
+// device copies of host vectors for the host-pointer entry points, and the
+// products' scratch vectors, from the solvers' caching pool (a hipMalloc and
+// hipFree pair per vector and call waited for the device)
 template <class V>
 struct DVec {
     V *p = nullptr;
     size_t n = 0;
     DVec() = default;
-    explicit DVec(size_t cnt) : n(cnt) { HIP_TRY(hipMalloc(&p, sizeof(V) * (cnt ? cnt : 1))); }
+    explicit DVec(size_t cnt) : n(cnt) { p = (V *)pool_alloc(sizeof(V) * cnt); }
     DVec(const V *h, size_t cnt, hipStream_t st) : DVec(cnt) {
         if (h && cnt) HIP_TRY(hipMemcpyAsync(p, h, sizeof(V) * cnt, hipMemcpyHostToDevice, st));
     }
-    ~DVec() { (void)hipFree(p); }
+    ~DVec() { pool_free(p, sizeof(V) * n); }
     DVec(const DVec &) = delete;
     DVec &operator=(const DVec &) = delete;
     DVec &operator=(DVec &&o) noexcept {
