@@ -1,7 +1,8 @@
 // Batched IDR(s) on one GPU: the independent systems of a block-diagonal
 // operator advance together, one workgroup per tile (a row range inside one
-// system) for every streaming kernel and SpMV, one workgroup per system for
-// every reduction + scalar step.
+// system) for every streaming kernel and SpMV; the per-system sums and scalar
+// steps run at the start of the tile kernel that uses them.  Batches of small
+// systems run each system whole in one workgroup instead (block.hip).
 //
 // Each system follows MODULES/IDRS/idrs.inc:1-311 exactly as the
 // single-system solver does (same kernels' per-row arithmetic, same scalar

@@ -21,6 +21,8 @@
 //   fin_norm    : ||r||, iteration count, convergence test
 // and the omega step is: SpMV chain of A*r with the (r,r),(t,t),(t,r)
 // epilogue, fin_om, omega_update (r, x, ||r||^2 and the next P^T r), fin_cycle.
+// Up to 2^18 rows the fin kernels fold into the streaming kernel after them;
+// solves of up to 2560 rows run in one workgroup (block.hip).
 // Shadow spaces wider than PDOT_MAX rows take their P^T sums from a chunked
 // kernel (pdot.hpp) instead of the product epilogue and the update kernel.
 #include "idrs.hpp"
