@@ -811,12 +811,16 @@ void set_values(DevMatrix &K, const void *vals, bool device, hipStream_t st) {
     if (K.nrows) refresh_diag(K, st);
 }
 
-template <class T, class V>
-__global__ void k_pattern_grad(int n, const int *__restrict__ rp, const int *__restrict__ col,
-                               const T *__restrict__ lam, const T *__restrict__ x, T *__restrict__ grad) {
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
+// G lanes per row, so that the indices and the gradient stream coalesced (one
+// thread per row: 515 us for 1e6 rows of 17 random columns)
+template <class T, int G>
+__global__ __launch_bounds__(256) void k_pattern_grad(int n, const int *__restrict__ rp, const int *__restrict__ col,
+                                                      const T *__restrict__ lam, const T *__restrict__ x,
+                                                      T *__restrict__ grad) {
+    const int g = threadIdx.x % G;
+    for (long i = ((long)blockIdx.x * blockDim.x + threadIdx.x) / G; i < n; i += (long)gridDim.x * blockDim.x / G) {
         const T li = lam[i];
-        for (int k = rp[i]; k < rp[i + 1]; k++) grad[k] = -(li * x[col[k]]);
+        for (int k = rp[i] + g; k < rp[i + 1]; k += G) grad[k] = -(li * x[col[k]]);
     }
 }
 
@@ -825,8 +829,14 @@ void pattern_grad(const DevMatrix &K, const T *lambda, const T *x, T *grad, hipS
     if (K.fmt != DevFmt::CRS) throw std::invalid_argument("pattern gradient needs a CRS/COO matrix");
     if (K.orig_format == 3) throw std::invalid_argument("pattern gradient is in CRS entry order; use a CRS matrix");
     if (!K.nrows) return;
-    hipLaunchKernelGGL((k_pattern_grad<T, T>), dim3(vec_grid(K.nrows)), dim3(256), 0, st, K.nrows, K.row_ptr, K.col,
-                       lambda, x, grad);
+    const double avg = (double)K.nnz / K.nrows;
+    auto go = [&](auto kernel, long lanes) {
+        hipLaunchKernelGGL(kernel, dim3(vec_grid(lanes * K.nrows)), dim3(256), 0, st, K.nrows, K.row_ptr, K.col, lambda,
+                           x, grad);
+    };
+    if (avg <= 6) go(k_pattern_grad<T, 4>, 4);
+    else if (avg <= 24) go(k_pattern_grad<T, 16>, 16);
+    else go(k_pattern_grad<T, 64>, 64);
     LAUNCH_CHECK();
 }
 template void pattern_grad<double>(const DevMatrix &, const double *, const double *, double *, hipStream_t);
