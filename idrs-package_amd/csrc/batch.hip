@@ -536,7 +536,7 @@ void batch_idrs_solve(const Operator &A, int s, const T *b, T *x, const SolveOpt
 
     // Systems small enough each run whole in one workgroup, without waiting
     // for each other (block.hip).
-    if (block_fits<T>(A, nmax, s, o)) {
+    if (block_fits<T>(A, nmax, s, o, true)) {
         DBuf scratch(block_scratch<T>(A, ntot, s, o)), bres(sizeof(BlockResult) * nsys);
         DBuf bom(sizeof(T) * std::max(1, o.n_omega));
         T *omega_d = nullptr;

@@ -481,10 +481,10 @@ void launch(const Operator &A, BlkArgs<VT, T> &a, long nmax, int nsys, hipStream
 // and with Chebyshev(8) in DIA storage 74.8 -> 78.0); the vectors have to fit
 // LDS, and the form has to be one the kernel has.
 template <class T>
-bool block_fits(const Operator &A, long n, int s, const SolveOpts<T> &o) {
+bool block_fits(const Operator &A, long n, int s, const SolveOpts<T> &o, bool batch) {
     if constexpr (!std::is_same<T, double>::value && !std::is_same<T, c128>::value) return false;
     const DevMatrix &K = *A.K;
-    if (n > (K.part ? BLK_NMAX : BLK_SINGLE)) return false;
+    if (n > (batch ? BLK_NMAX : BLK_SINGLE)) return false;
     if (A.general() || A.values32 || s > BLK_S || A.degree > BLK_DEG) return false;
     if (K.nrows != K.ncols) return false;
     if (K.fmt == DevFmt::DIA ? K.ndiag > BLK_DIAG : K.max_row > BLK_WIDTH) return false;
@@ -513,8 +513,9 @@ void block_solve(const Operator &A, int nsys, const long *row0, long ntot, int s
                  const SolveOpts<T> &o, const T *m1, const T *omega, double *resvec, int rv_cap, T *H,
                  long max_cycles, void *scratch, BlockResult *out, hipStream_t st) {
     const DevMatrix &K = *A.K;
+    // without row0 the rows are one system, also those of a batch's matrix
     long nmax = ntot;
-    if (K.part) {
+    if (row0) {
         nmax = 0;
         for (int k = 0; k < nsys; k++) nmax = std::max(nmax, K.part->h_row0[k + 1] - K.part->h_row0[k]);
     }
@@ -586,7 +587,7 @@ void block_solve(const Operator &A, int nsys, const long *row0, long ntot, int s
 }
 
 #define IDRS_BLOCK(T)                                                                                            \
-    template bool block_fits<T>(const Operator &, long, int, const SolveOpts<T> &);                              \
+    template bool block_fits<T>(const Operator &, long, int, const SolveOpts<T> &, bool);                        \
     template size_t block_scratch<T>(const Operator &, long, int, const SolveOpts<T> &);                         \
     template void block_solve<T>(const Operator &, int, const long *, long, int, const T *, T *,                 \
                                  const SolveOpts<T> &, const T *, const T *, double *, int, T *, long, void *,   \

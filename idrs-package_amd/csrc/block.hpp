@@ -8,10 +8,10 @@
 
 namespace idrs {
 
-// true when the solve of every system of A (one, or the systems of a batch,
-// the largest of n rows) fits the one-workgroup kernel
+// true when the solve of A as one system of n rows, or (batch) of every system
+// of its partition, the largest of n rows, fits the one-workgroup kernel
 template <class T>
-bool block_fits(const Operator &A, long n, int s, const SolveOpts<T> &o);
+bool block_fits(const Operator &A, long n, int s, const SolveOpts<T> &o, bool batch);
 
 // The scratch memory of such a solve, in bytes, for ntot rows in all
 template <class T>
@@ -24,7 +24,7 @@ struct BlockResult {
 };
 
 // Enqueues the solves: nsys systems, rows [row0[k], row0[k+1]) each (device
-// array; nullptr: one system of ntot rows).  Pointers are device pointers;
+// array of A's partition; nullptr: one system of ntot rows).  Pointers are device pointers;
 // m1 the diagonal of M1 or nullptr, omega the user omegas, resvec of rv_cap
 // entries or nullptr, H as State::H.  max_cycles bounds every solve's cycles.
 template <class T>

@@ -1217,7 +1217,7 @@ int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOp
     SpmvTimer &tm = spmv_timer();
     if (ar && tm.enabled) throw std::invalid_argument("SpMV timing needs events: not in the allocation-free solve");
     if constexpr (std::is_same<T, double>::value || std::is_same<T, c128>::value) {
-        if (!tm.enabled && block_fits<T>(A, n, s, o)) {
+        if (!tm.enabled && block_fits<T>(A, n, s, o, false)) {
             solve_in_block<T>(A, n, s, b, x, o, out, cap_it, user_omega != 0, out_h, stream);
             return 0;
         }

@@ -86,3 +86,24 @@ def test_small_batches_match_oracle(gpu, sizes, s):
             assert r.flag[k] == o[1] == 0
             assert np.linalg.norm(c.matvec(r.x[at:at + c.n]) - bk) <= 1.01e-9 * np.linalg.norm(bk)
         at += c.n
+
+
+# One solve of a batch's whole matrix, each system of another size: the rows in
+# all, not a system's, decide the kernel (964 and 2560 rows: one workgroup).
+@pytest.mark.parametrize("sizes", [[64, 900], [900, 64], [60, 1500, 1000], [60, 1500, 1001], [1, 4000]])
+@pytest.mark.parametrize("entry", ["host", "ritz"])
+def test_single_solve_on_a_batch_matrix(gpu, sizes, entry):
+    systems = [_system(n, 11 + n)[0] for n in sizes]
+    KB = idrs_amd.batch_format([idrs_amd.crs_format(c.n, c.n, c.row_ptr, c.col_ind, rval=c.val) for c in systems])
+    at = np.concatenate([[0], np.cumsum(sizes)])
+    nz = np.concatenate([[0], np.cumsum([c.nnz for c in systems])])
+    whole = P.Crs(int(at[-1]), np.concatenate([[1]] + [c.row_ptr[1:] + nz[k] for k, c in enumerate(systems)]).astype(np.int32),
+                  np.concatenate([c.col_ind + at[k] for k, c in enumerate(systems)]).astype(np.int32),
+                  np.concatenate([c.val for c in systems]))
+    n, s = whole.n, 4
+    b = np.random.default_rng(7).uniform(-1, 1, n)
+    PT = P.gaussian_shadow(n, s, seed=2)
+    solve = idrs_amd.idrs if entry == "host" else idrs_amd.idrs_ritz
+    g = solve(idrs_amd.Matrix(KB), b, s, tolerance=0.0, maximum_iterations=10, PT_raw=PT)
+    o = orc.idrs(orc.OracleMatrix(orc.CRS, n, crs=whole), b, s, tolerance=0.0, maximum_iterations=10, PT_raw=PT)
+    assert (g.flag, g.iterations) == (o[1], o[3]) and rel(g.x, o[0]) < 1e-10
