@@ -32,112 +32,11 @@
 
 #include <cfloat>
 #include <chrono>
-#include <map>
 #include <mutex>
 #include <stdexcept>
 #include <vector>
 
 namespace idrs {
-
-// ---------------------------------------------------------------------------
-// small caching allocators (calls of equal size reuse workspaces; a free
-// would wait for the device): device buffers by (device, size), pinned host
-// buffers by (size, flags).  The device buffers kept for reuse stay within a
-// quarter of the device's memory (a buffer beyond it is freed), and all of
-// them are given back when an allocation fails.  Every user's work runs on
-// the library's stream, so a buffer taken again is written after its last
-// reader.
-// ---------------------------------------------------------------------------
-namespace {
-std::mutex g_pool_mu;
-std::multimap<std::pair<int, size_t>, void *> g_pool;
-std::map<int, size_t> g_pool_kept, g_pool_cap;   // bytes by device
-std::multimap<std::pair<size_t, unsigned>, void *> g_pinned;
-size_t pool_round(size_t bytes) {
-    bytes = (bytes + 255) & ~(size_t)255;
-    return bytes ? bytes : 256;
-}
-void pool_release(int dev) {
-    std::vector<void *> drop;
-    {
-        std::lock_guard<std::mutex> g(g_pool_mu);
-        for (auto it = g_pool.begin(); it != g_pool.end();) {
-            if (it->first.first == dev) {
-                drop.push_back(it->second);
-                it = g_pool.erase(it);
-            } else {
-                ++it;
-            }
-        }
-        g_pool_kept[dev] = 0;
-    }
-    for (void *p : drop) (void)hipFree(p);
-}
-}  // namespace
-
-void *pool_alloc(size_t bytes) {
-    bytes = pool_round(bytes);
-    int dev = 0;
-    HIP_TRY(hipGetDevice(&dev));
-    {
-        std::lock_guard<std::mutex> g(g_pool_mu);
-        auto it = g_pool.find({dev, bytes});
-        if (it != g_pool.end()) {
-            void *p = it->second;
-            g_pool.erase(it);
-            g_pool_kept[dev] -= bytes;
-            return p;
-        }
-    }
-    void *p = nullptr;
-    if (hipMalloc(&p, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        pool_release(dev);
-        HIP_TRY(hipMalloc(&p, bytes));
-    }
-    return p;
-}
-void pool_free(void *p, size_t bytes) {
-    if (!p) return;
-    bytes = pool_round(bytes);
-    int dev = 0;
-    if (hipPointerAttribute_t at{}; hipPointerGetAttributes(&at, p) == hipSuccess) dev = at.device;
-    {
-        std::lock_guard<std::mutex> g(g_pool_mu);
-        size_t &cap = g_pool_cap[dev];
-        if (!cap) {
-            size_t left = 0, total = 0;
-            cap = hipMemGetInfo(&left, &total) == hipSuccess ? total / 4 : size_t(1) << 30;
-        }
-        size_t &kept = g_pool_kept[dev];
-        if (kept + bytes <= cap) {
-            kept += bytes;
-            g_pool.emplace(std::make_pair(dev, bytes), p);
-            return;
-        }
-    }
-    (void)hipFree(p);
-}
-void *pinned_take(size_t bytes, unsigned flags) {
-    bytes = pool_round(bytes);
-    {
-        std::lock_guard<std::mutex> g(g_pool_mu);
-        auto it = g_pinned.find({bytes, flags});
-        if (it != g_pinned.end()) {
-            void *p = it->second;
-            g_pinned.erase(it);
-            return p;
-        }
-    }
-    void *p = nullptr;
-    HIP_TRY(hipHostMalloc(&p, bytes, flags));
-    return p;
-}
-void pinned_give(void *p, size_t bytes, unsigned flags) {
-    if (!p) return;
-    std::lock_guard<std::mutex> g(g_pool_mu);
-    g_pinned.emplace(std::make_pair(pool_round(bytes), flags), p);
-}
 
 namespace {
 // a device buffer from the caching pool, or (with an arena) a piece of the
