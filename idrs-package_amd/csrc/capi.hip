@@ -655,6 +655,13 @@ extern "C" {
 const char *idrs_last_error(void) { return g_err.c_str(); }
 int idrs_version(void) { return 100; }
 
+int idrs_release_pool(int64_t *bytes) {
+    return guarded([&] {
+        const size_t freed = pool_release();
+        if (bytes) *bytes = (int64_t)freed;
+    });
+}
+
 int idrs_device_count(void) {
     int c = 0;
     if (hipGetDeviceCount(&c) != hipSuccess) return 0;

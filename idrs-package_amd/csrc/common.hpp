@@ -32,6 +32,25 @@ struct HipError {
 #define LAUNCH_CHECK() HIP_TRY(hipGetLastError())
 
 // ---------------------------------------------------------------------------
+// device memory (pool.hip)
+// ---------------------------------------------------------------------------
+// hipMalloc for what outlives a call (matrices, operators): when the device
+// has no memory left its idle pool buffers are freed and it is tried again
+hipError_t dev_malloc_bytes(void **p, size_t bytes);
+template <class V>
+inline hipError_t dev_malloc(V **p, size_t bytes) { return dev_malloc_bytes((void **)p, bytes); }
+// Workspaces of the current device from its pool (throws when there is no
+// memory), and back; pinned host memory by size and flags.  Every user's work
+// runs on the library's stream, so a buffer taken again is written after its
+// last reader.
+void *pool_alloc(size_t bytes);
+void pool_free(void *p, size_t bytes);
+void *pinned_take(size_t bytes, unsigned flags);
+void pinned_give(void *p, size_t bytes, unsigned flags);
+// frees the idle buffers of every device; the bytes freed
+size_t pool_release();
+
+// ---------------------------------------------------------------------------
 // complex<double> / complex<float> value type (plain struct: trivially
 // copyable, passes as a kernel argument, 16-byte aligned loads).
 // ---------------------------------------------------------------------------

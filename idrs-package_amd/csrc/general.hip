@@ -448,9 +448,9 @@ void gen_make_deflation(Operator &op, const T *V, int nd, hipStream_t st) {
     (void)hipFree(op.dVtAV);
     op.dV = op.dAV = op.dVtAV = nullptr;
     op.ndefl = 0;
-    HIP_TRY(hipMalloc(&op.dV, sizeof(T) * n * nd));
-    HIP_TRY(hipMalloc(&op.dAV, sizeof(T) * n * nd));
-    HIP_TRY(hipMalloc(&op.dVtAV, sizeof(T) * nd * nd));
+    HIP_TRY(dev_malloc(&op.dV, sizeof(T) * n * nd));
+    HIP_TRY(dev_malloc(&op.dAV, sizeof(T) * n * nd));
+    HIP_TRY(dev_malloc(&op.dVtAV, sizeof(T) * nd * nd));
     op.defl_complex = Tr<T>::is_complex;
     HIP_TRY(hipMemcpyAsync(op.dV, V, sizeof(T) * n * nd, hipMemcpyDeviceToDevice, st));
     op.ndefl = nd;
@@ -557,7 +557,7 @@ void gen_prepare(const Operator &op) {
     (void)hipFree(op.gws);
     op.gws = nullptr;
     const long n = op.rows();
-    HIP_TRY(hipMalloc(&op.gws, sizeof(c128) * (8 * n + (long)MAX_DEFL * GEN_PARTS + MAX_DEFL)));
+    HIP_TRY(dev_malloc(&op.gws, sizeof(c128) * (8 * n + (long)MAX_DEFL * GEN_PARTS + MAX_DEFL)));
     op.gws_rows = n;
 }
 

@@ -2,7 +2,6 @@
 #pragma once
 
 #include "matrix.hpp"
-#include "pool.hpp"
 
 #include <stdexcept>
 

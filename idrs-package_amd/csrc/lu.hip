@@ -368,11 +368,11 @@ void build_typed(LuFactor &F, const DevMatrix &K, const DevMatrix *M, const DevM
             ~Free() { (void)hipFree(p); }
         } f1{tc}, f2{tm};
         if (C) {
-            HIP_TRY(hipMalloc(&tc, sizeof(FT) * cnt));
+            HIP_TRY(dev_malloc(&tc, sizeof(FT) * cnt));
             scatter<FT>(*C, dense, F.ld, F.hb, tc, st);
         }
         if (M) {
-            HIP_TRY(hipMalloc(&tm, sizeof(FT) * cnt));
+            HIP_TRY(dev_malloc(&tm, sizeof(FT) * cnt));
             scatter<FT>(*M, dense, F.ld, F.hb, tm, st);
         }
         if (M || C) {
@@ -390,7 +390,7 @@ void build_typed(LuFactor &F, const DevMatrix &K, const DevMatrix *M, const DevM
         HIP_TRY(hipStreamSynchronize(st));
     }
     int *info = nullptr;
-    HIP_TRY(hipMalloc(&info, sizeof(int)));
+    HIP_TRY(dev_malloc(&info, sizeof(int)));
     struct FreeI {
         int *p;
         ~FreeI() { (void)hipFree(p); }
@@ -459,7 +459,7 @@ std::shared_ptr<LuFactor> lu_build(int which, const DevMatrix &K, const DevMatri
     if (!shift) M = C = nullptr;       // without a shift the reference factors K alone (the band still
                                        // spans M and C, user_module.f90:1423-1425)
     const size_t es = cplx ? sizeof(c128) : sizeof(double);
-    HIP_TRY(hipMalloc(&F->lu, es * (size_t)F->n * F->ld));
+    HIP_TRY(dev_malloc(&F->lu, es * (size_t)F->n * F->ld));
     if (cplx) build_typed<c128>(*F, K, M, C, shift, st);
     else build_typed<double>(*F, K, M, C, shift, st);
     return F;

@@ -150,7 +150,7 @@ template <class V>
 static V *dev_upload(const V *h, size_t count) {
     V *d = nullptr;
     if (count == 0) count = 1;
-    HIP_TRY(hipMalloc(&d, sizeof(V) * count));
+    HIP_TRY(dev_malloc(&d, sizeof(V) * count));
     if (h) HIP_TRY(hipMemcpy(d, h, sizeof(V) * count, hipMemcpyHostToDevice));
     return d;
 }
@@ -636,10 +636,10 @@ DevMatrix *make_blockdiag(int nsys, const DevMatrix *const *Ks) {
     M->nnz = nnz;
     M->max_row = max_row;
     const size_t vsz = kind == ValKind::Complex ? sizeof(c128) : sizeof(double);
-    HIP_TRY(hipMalloc(&M->row_ptr, sizeof(int) * (nrows + 1)));
-    HIP_TRY(hipMalloc(&M->col, sizeof(int) * (nnz ? nnz : 1)));
-    HIP_TRY(hipMalloc(&M->val, vsz * (nnz ? nnz : 1)));
-    HIP_TRY(hipMalloc(&M->diag, vsz * nrows));
+    HIP_TRY(dev_malloc(&M->row_ptr, sizeof(int) * (nrows + 1)));
+    HIP_TRY(dev_malloc(&M->col, sizeof(int) * (nnz ? nnz : 1)));
+    HIP_TRY(dev_malloc(&M->val, vsz * (nnz ? nnz : 1)));
+    HIP_TRY(dev_malloc(&M->diag, vsz * nrows));
     std::unique_ptr<Partition> P(new Partition);
     P->nsys = nsys;
     P->h_row0.assign(nsys + 1, 0);
@@ -721,8 +721,8 @@ DevMatrix *make_transpose(const DevMatrix &K) {
     T->col = dev_upload(tcol.data(), (size_t)nnz);
     T->tperm = dev_upload(perm.data(), (size_t)nnz);
     const size_t vsz = K.kind == ValKind::Complex ? sizeof(c128) : sizeof(double);
-    HIP_TRY(hipMalloc(&T->val, vsz * (nnz ? nnz : 1)));
-    HIP_TRY(hipMalloc(&T->diag, vsz * (m ? m : 1)));
+    HIP_TRY(dev_malloc(&T->val, vsz * (nnz ? nnz : 1)));
+    HIP_TRY(dev_malloc(&T->diag, vsz * (m ? m : 1)));
     double avg = m > 0 ? (double)nnz / m : 1.0;
     int g = 2;
     while (g < 64 && g < avg) g *= 2;
@@ -984,7 +984,7 @@ __global__ void k_sell_gather(long nent, const int *__restrict__ perm, const V *
 
 static void *sliced_copy(const Sell &S, const void *src, bool cplx, hipStream_t st, void *dst) {
     const size_t vsz = cplx ? sizeof(c128) : sizeof(double);
-    if (!dst) HIP_TRY(hipMalloc(&dst, vsz * (S.nent ? S.nent : 1)));
+    if (!dst) HIP_TRY(dev_malloc(&dst, vsz * (S.nent ? S.nent : 1)));
     const int g = vec_grid(S.nent);
     if (cplx)
         hipLaunchKernelGGL((k_sell_gather<c128>), dim3(g), dim3(256), 0, st, S.nent, S.sl_perm, (const c128 *)src,
@@ -1019,7 +1019,7 @@ void build_sell(DevMatrix &K, hipStream_t st) {
     }
     S->sl_ptr = dev_upload(sp.data(), sp.size());
     S->sl_perm = dev_upload(perm.data(), perm.size());
-    HIP_TRY(hipMalloc(&S->sl_col, sizeof(int) * (S->nent ? S->nent : 1)));
+    HIP_TRY(dev_malloc(&S->sl_col, sizeof(int) * (S->nent ? S->nent : 1)));
     const int g = vec_grid(S->nent);
     hipLaunchKernelGGL((k_sell_gather<int>), dim3(g), dim3(256), 0, st, S->nent, S->sl_perm, (const int *)K.col,
                        S->sl_col);
@@ -1077,8 +1077,8 @@ int autotune_group(DevMatrix &K, int reps, hipStream_t st, std::vector<std::pair
     const bool cplx = K.kind == ValKind::Complex;
     const size_t vsz = cplx ? sizeof(c128) : sizeof(double);
     void *x = nullptr, *y = nullptr;
-    HIP_TRY(hipMalloc(&x, vsz * (K.ncols ? K.ncols : 1)));
-    HIP_TRY(hipMalloc(&y, vsz * K.nrows));
+    HIP_TRY(dev_malloc(&x, vsz * (K.ncols ? K.ncols : 1)));
+    HIP_TRY(dev_malloc(&y, vsz * K.nrows));
     HIP_TRY(hipMemsetAsync(x, 0, vsz * (K.ncols ? K.ncols : 1), st));
     hipEvent_t a, b;
     HIP_TRY(hipEventCreate(&a));
@@ -1234,7 +1234,7 @@ static void drop_unit_diagonal(Operator &op, bool cvals, hipStream_t st) {
     const size_t vsz = cvals ? sizeof(c128) : sizeof(double);
     const int g = std::min(vec_grid(n), 1024);
     int *bad = nullptr;
-    HIP_TRY(hipMalloc(&bad, sizeof(int) * g));
+    HIP_TRY(dev_malloc(&bad, sizeof(int) * g));
     std::vector<int> hb(g);
     try {
         if (cvals)
@@ -1253,7 +1253,7 @@ static void drop_unit_diagonal(Operator &op, bool cvals, hipStream_t st) {
     for (int v : hb)
         if (v) return;
     void *packed = nullptr;
-    HIP_TRY(hipMalloc(&packed, vsz * n * (K.ndiag - 1)));
+    HIP_TRY(dev_malloc(&packed, vsz * n * (K.ndiag - 1)));
     char *src = (char *)op.sval, *dst = (char *)packed;
     if (z0 > 0) HIP_TRY(hipMemcpyAsync(dst, src, vsz * n * z0, hipMemcpyDeviceToDevice, st));
     if (z0 < K.ndiag - 1)
@@ -1299,7 +1299,7 @@ void op_set_diag_precon(Operator &op, int which, const std::complex<double> *shi
     bool cdiag = (K.kind == ValKind::Complex) || (shift && shift->imag() != 0.0);
     op.pdiag_kind = cdiag ? ValKind::Complex : ValKind::Real;
     if (cdiag) {
-        HIP_TRY(hipMalloc(&op.pdiag, sizeof(c128) * (n ? n : 1)));
+        HIP_TRY(dev_malloc(&op.pdiag, sizeof(c128) * (n ? n : 1)));
         if (K.kind == ValKind::Complex)
             HIP_TRY(hipMemcpyAsync(op.pdiag, K.diag, sizeof(c128) * n, hipMemcpyDeviceToDevice, st));
         else {
@@ -1312,7 +1312,7 @@ void op_set_diag_precon(Operator &op, int which, const std::complex<double> *shi
             LAUNCH_CHECK();
         }
     } else {
-        HIP_TRY(hipMalloc(&op.pdiag, sizeof(double) * (n ? n : 1)));
+        HIP_TRY(dev_malloc(&op.pdiag, sizeof(double) * (n ? n : 1)));
         HIP_TRY(hipMemcpyAsync(op.pdiag, K.diag, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
         if (shift) {
             hipLaunchKernelGGL((k_add_scalar<double>), dim3(g), dim3(256), 0, st, n, (double *)op.pdiag, -shift->real());
@@ -1328,11 +1328,11 @@ static void op_scale_values(Operator &op, bool cdiag, hipStream_t st) {
     long cnt = K.fmt == DevFmt::CRS ? K.nnz : (long)K.ndiag * K.nrows;
     int gv = vec_grid(cnt);
     bool cvals = (K.kind == ValKind::Complex) || cdiag;
-    HIP_TRY(hipMalloc(&op.sval, (cvals ? sizeof(c128) : sizeof(double)) * (cnt ? cnt : 1)));
+    HIP_TRY(dev_malloc(&op.sval, (cvals ? sizeof(c128) : sizeof(double)) * (cnt ? cnt : 1)));
     void *src = K.val;
     void *tmpc = nullptr;
     if (cvals && K.kind != ValKind::Complex) {
-        HIP_TRY(hipMalloc(&tmpc, sizeof(c128) * (cnt ? cnt : 1)));
+        HIP_TRY(dev_malloc(&tmpc, sizeof(c128) * (cnt ? cnt : 1)));
         hipLaunchKernelGGL(k_real_to_cplx, dim3(gv), dim3(256), 0, st, cnt, (const double *)K.val, (c128 *)tmpc);
         LAUNCH_CHECK();
         src = tmpc;
@@ -1380,12 +1380,12 @@ void op_set_diag_values(Operator &op, const std::vector<std::complex<double>> &d
     if (cdiag) {
         std::vector<c128> h(n);
         for (long i = 0; i < n; i++) h[i] = c128(d[i].real(), d[i].imag());
-        HIP_TRY(hipMalloc(&op.pdiag, sizeof(c128) * (n ? n : 1)));
+        HIP_TRY(dev_malloc(&op.pdiag, sizeof(c128) * (n ? n : 1)));
         HIP_TRY(hipMemcpy(op.pdiag, h.data(), sizeof(c128) * n, hipMemcpyHostToDevice));
     } else {
         std::vector<double> h(n);
         for (long i = 0; i < n; i++) h[i] = d[i].real();
-        HIP_TRY(hipMalloc(&op.pdiag, sizeof(double) * (n ? n : 1)));
+        HIP_TRY(dev_malloc(&op.pdiag, sizeof(double) * (n ? n : 1)));
         HIP_TRY(hipMemcpy(op.pdiag, h.data(), sizeof(double) * n, hipMemcpyHostToDevice));
     }
     op_scale_values(op, cdiag, st);
@@ -1399,13 +1399,13 @@ void op_make_lowprec(Operator &op) {
     int gv = vec_grid(cnt);
     if (op.sval) {
         if (!op.sval32) {
-            HIP_TRY(hipMalloc(&op.sval32, sizeof(float) * (cnt ? cnt : 1)));
+            HIP_TRY(dev_malloc(&op.sval32, sizeof(float) * (cnt ? cnt : 1)));
             hipLaunchKernelGGL((k_convert<double, float>), dim3(gv), dim3(256), 0, st, cnt, (const double *)op.sval,
                                (float *)op.sval32);
             LAUNCH_CHECK();
         }
     } else if (!K.val32) {
-        HIP_TRY(hipMalloc(&K.val32, sizeof(float) * (cnt ? cnt : 1)));
+        HIP_TRY(dev_malloc(&K.val32, sizeof(float) * (cnt ? cnt : 1)));
         hipLaunchKernelGGL((k_convert<double, float>), dim3(gv), dim3(256), 0, st, cnt, (const double *)K.val,
                            (float *)K.val32);
         LAUNCH_CHECK();
@@ -1419,7 +1419,7 @@ void op_make_lowprec(Operator &op) {
         const void *src = op.sval ? op.sl_sval : K.sell->sl_val;
         if (!dst && src) {
             // (value, column) pairs, 8 bytes per entry (see sell_row)
-            HIP_TRY(hipMalloc(&dst, sizeof(unsigned long long) * (ne ? ne : 1)));
+            HIP_TRY(dev_malloc(&dst, sizeof(unsigned long long) * (ne ? ne : 1)));
             hipLaunchKernelGGL(k_pair32, dim3(gs), dim3(256), 0, st, ne, (const double *)src, K.sell->sl_col,
                                (unsigned long long *)dst);
             LAUNCH_CHECK();

@@ -11,11 +11,12 @@ namespace {
 
 // The idle buffers of a device stay within a quarter of its memory.  The
 // pools live until the process ends.
+std::mutex g_pools_mu;
+std::map<int, BufferPool *> g_pools;
+
 BufferPool &device_pool(int dev) {
-    static std::mutex mu;
-    static std::map<int, BufferPool *> pools;
-    std::lock_guard<std::mutex> g(mu);
-    BufferPool *&p = pools[dev];
+    std::lock_guard<std::mutex> g(g_pools_mu);
+    BufferPool *&p = g_pools[dev];
     if (!p) {
         size_t left = 0, total = 0;
         const size_t cap = hipMemGetInfo(&left, &total) == hipSuccess ? total / 4 : size_t(1) << 30;
@@ -40,6 +41,27 @@ std::mutex g_pinned_mu;
 std::multimap<std::pair<size_t, unsigned>, void *> g_pinned;
 
 }  // namespace
+
+hipError_t dev_malloc_bytes(void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
+    int dev = 0;
+    if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
+    *p = device_pool(dev).allocate(bytes);
+    return *p ? hipSuccess : hipErrorOutOfMemory;
+}
+
+size_t pool_release() {
+    std::vector<BufferPool *> all;
+    {
+        std::lock_guard<std::mutex> g(g_pools_mu);
+        for (auto &e : g_pools) all.push_back(e.second);
+    }
+    size_t freed = 0;
+    for (BufferPool *p : all) freed += p->trim();
+    return freed;
+}
 
 void *pool_alloc(size_t bytes) {
     bytes = pool_round(bytes);

@@ -1,6 +1,6 @@
-// Caching allocators of the library: a bounded pool of idle buffers (plain
-// host code over an allocate/free pair, so that its rules can be run without a
-// GPU) and the device and pinned-memory pools built on it (pool.hip).
+// A bounded pool of idle buffers: plain host code over an allocate/free pair,
+// so that its rules can be run without a GPU.  The device pools are in
+// pool.hip.
 #pragma once
 
 #include <cstddef>
@@ -101,14 +101,5 @@ private:
     std::map<size_t, std::list<std::list<Idle>::iterator>> by_size;   // in the same order
     size_t kept_ = 0;
 };
-
-// Device memory of the current device from its pool (throws when there is
-// none), and back; pinned host memory by size and flags.  Every user's work
-// runs on the library's stream, so a buffer taken again is written after its
-// last reader.
-void *pool_alloc(size_t bytes);
-void pool_free(void *p, size_t bytes);
-void *pinned_take(size_t bytes, unsigned flags);
-void pinned_give(void *p, size_t bytes, unsigned flags);
 
 }  // namespace idrs

@@ -307,10 +307,16 @@ void launch_pat(const DevMatrix &K, const RowCode &rc, bool f32, const SpmvArgs<
     LAUNCH_CHECK();
 }
 
+// null: no device memory left
 template <class V>
 V *dev_new(size_t count) {
     V *p = nullptr;
-    HIP_TRY(hipMalloc(&p, sizeof(V) * std::max<size_t>(1, count)));
+    const hipError_t e = dev_malloc(&p, sizeof(V) * std::max<size_t>(1, count));
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    HIP_TRY(e);
     return p;
 }
 
@@ -343,7 +349,9 @@ std::shared_ptr<RowCode> make_rowcode(const Operator &op, bool values, hipStream
         if (op.sval && op.unit_diag >= 0) S.ud = op.unit_diag;
     }
     if (width < 1 || width > ROWCODE_WIDTH) return nullptr;
+    // the code is optional: without memory for it the products stay uncoded
     Work *w = dev_new<Work>(1);
+    if (!w) return nullptr;
     std::shared_ptr<RowCode> rc;
     try {
         const int g = vec_grid(K.nrows);
@@ -376,6 +384,9 @@ std::shared_ptr<RowCode> make_rowcode(const Operator &op, bool values, hipStream
             rc->ent = dev_new<RowEntry>((size_t)count * width);
             rc->ent32 = dev_new<RowEntry>((size_t)count * width);
             rc->len = dev_new<int>(count);
+            if (!rc->code || !rc->ent || !rc->ent32 || !rc->len) rc.reset();
+        }
+        if (rc) {
             hipLaunchKernelGGL(k_row_table, dim3(1), dim3(256), 0, st, S, w, width, rc->ent, rc->ent32, rc->len);
             LAUNCH_CHECK();
             hipLaunchKernelGGL(k_code_rows, dim3(g), dim3(256), 0, st, S, w, width, rc->ent, rc->len, rc->code);

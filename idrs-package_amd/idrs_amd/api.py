@@ -1159,3 +1159,11 @@ def ms_scaleback(A, alpha_s, Y, out=None):
     f = lib.idrs_ms_scaleback_c128 if cplx else lib.idrs_ms_scaleback_f64
     check(f(A.handle, ns, d, a.ctypes.data, _ptr(Yc), _ptr(Xc), 0))
     return Xc.T
+
+
+def release_pool():
+    """Frees the device buffers the library keeps for reuse between calls, so
+    that another allocator (torch's) can have the memory; the bytes freed."""
+    n = ctypes.c_int64(0)
+    check(_lib.load().idrs_release_pool(ctypes.byref(n)))
+    return n.value

@@ -563,6 +563,11 @@ int idrs_make_p_c128(int n, int s, int method, const double *PT_raw, const doubl
 /* Number of HIP devices visible (0 without a GPU); never fails. */
 int idrs_device_count(void);
 
+/* Frees the device buffers that the library keeps for reuse between calls
+   (at most a quarter of each device's memory), for another allocator of the
+   process; *bytes (may be NULL): the bytes freed.  Waits for the device. */
+int idrs_release_pool(int64_t *bytes);
+
 #ifdef __cplusplus
 }
 #endif
