@@ -21,7 +21,7 @@
 //   fin_norm    : ||r||, iteration count, convergence test
 // and the omega step is: SpMV chain of A*r with the (r,r),(t,t),(t,r)
 // epilogue, fin_om, omega_update (r, x, ||r||^2 and the next P^T r), fin_cycle.
-// Up to 2^18 rows the fin kernels fold into the streaming kernel after them;
+// Up to 196 608 rows the fin kernels fold into the streaming kernel after them;
 // solves of up to 2560 rows run in one workgroup (block.hip).
 // Shadow spaces wider than PDOT_MAX rows take their P^T sums from a chunked
 // kernel (pdot.hpp) instead of the product epilogue and the update kernel.
@@ -517,10 +517,14 @@ __global__ __launch_bounds__(256) void k_omega_update(long n, const State<T> *st
 // ---------------------------------------------------------------------------
 template <class T>
 using Slot = State<T, FIN_S>;
-constexpr int FOLD_PARTS = 2048;   // most partials a workgroup sums per value
-// The line: 101x97x103 (1.0e6 rows) runs the same either way (33.9 ms), 128^3
-// loses (6.20 -> 6.55 ms), 61x47x53 gains 15 %.
-constexpr long FOLD_ROWS = 1L << 18;
+// The lines, folded against unfolded (ms): one-thread-per-row products, IDR(4),
+// 100 steps: 131 072 rows 1.93 / 2.14, 196 608 rows 2.31 / 2.35, 262 144 rows
+// 2.77 / 2.68 (IDR(16) 6.14 / 5.53: every workgroup sums 16 values of 1024
+// partials).  Products with lanes per row, twice the partials per row, 200
+// steps: 157 410 rows (1224 partials) IDR(4) 5.47 / 5.98, IDR(8) 7.18 / 7.37;
+// 178 200 rows (1392) IDR(4) 5.83 / 5.92, IDR(8) 7.64 / 7.24.
+constexpr int FOLD_PARTS = 1280;         // most partials a workgroup sums per value
+constexpr long FOLD_ROWS = 3L << 16;
 
 template <class T>
 __global__ void k_fold_init(const State<T> *st, Slot<T> *sl) {
@@ -555,12 +559,13 @@ __global__ void k_fold_init(const State<T> *st, Slot<T> *sl) {
 // the sums of reduce_partials, bit for bit, by 256 threads (nparts <=
 // FOLD_PARTS): a wavefront takes the shares of wavefronts wid, wid + 4, ... of
 // the 1024-thread kernel, four values at a time with all their loads in
-// flight.  scr: nv * 16 values.  No barrier at the end.
+// flight.  scr: nv * 16 values.  No barrier at the end.  A solve that has
+// finished (info >= 0, known by the time the first values are) skips the rest.
 template <class T>
-__device__ inline void fold_sums(const T *__restrict__ partials, int nparts, int nv, T *scr) {
+__device__ inline void fold_sums(const T *__restrict__ partials, int nparts, int nv, T *scr, int info) {
     constexpr int NW = FIN_THREADS / WAVE, NR = 256 / WAVE, V = NW / NR;
     const int lane = threadIdx.x % WAVE, wid = threadIdx.x / WAVE;
-    for (int q0 = 0; q0 < nv; q0 += 4) {
+    for (int q0 = 0; q0 < nv && (q0 == 0 || info < 0); q0 += 4) {
         T a[V][4];
 #pragma unroll
         for (int j = 0; j < V; j++)
@@ -624,7 +629,7 @@ __global__ __launch_bounds__(256) void k_form_u_fold(long n, int prow, const Slo
     __shared__ Slot<T> sl;
     __shared__ T scr[(FIN_S + 1) * (FIN_THREADS / WAVE)], red[FIN_S + 1];
     fold_load(in, &sl);
-    if (npin) fold_sums(pin, npin, 1 + prow, scr);
+    if (npin) fold_sums(pin, npin, 1 + prow, scr, in->info);
     __syncthreads();
     if (threadIdx.x < WAVE && npin && sl.info < 0) {
         if (threadIdx.x <= prow) red[threadIdx.x] = fold_value(scr, threadIdx.x);
@@ -679,8 +684,8 @@ __global__ __launch_bounds__(256) void k_orth_fold(long n, int k, int s, int pro
             ui[i] = want ? U[(long)i * n + q] : T(0);
         }
     }
-    fold_sums(pmu, npmu, prow, scr);
-    if (npn) fold_sums(pn, npn, 1, scr + prow * (FIN_THREADS / WAVE));
+    fold_sums(pmu, npmu, prow, scr, in->info);
+    if (npn) fold_sums(pn, npn, 1, scr + prow * (FIN_THREADS / WAVE), in->info);
     __syncthreads();
     if (threadIdx.x < WAVE && sl.info < 0) {
         if (blockIdx.x != 0 && threadIdx.x == 0) sl.H = nullptr;
@@ -774,8 +779,8 @@ __global__ __launch_bounds__(256) void k_omega_fold(long n, const Slot<T> *in, S
     __shared__ Slot<T> sl;
     __shared__ T scr[4 * (FIN_THREADS / WAVE)], red[4], lds[(NV + 1) * 4];
     fold_load(in, &sl);
-    fold_sums(pom, npom, 3, scr);
-    fold_sums(pn, npn, 1, scr + 3 * (FIN_THREADS / WAVE));
+    fold_sums(pom, npom, 3, scr, in->info);
+    fold_sums(pn, npn, 1, scr + 3 * (FIN_THREADS / WAVE), in->info);
     __syncthreads();
     if (threadIdx.x < WAVE && sl.info < 0) {
         if (threadIdx.x < 4) red[threadIdx.x] = fold_value(scr, threadIdx.x);
@@ -1248,21 +1253,27 @@ int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOp
         pn[0] = bpn.as<T>();
         pn[1] = pn[0] + gv;
         pc = bpc.as<T>();
-        hipLaunchKernelGGL((k_fold_init<T>), dim3(1), dim3(64), 0, stream, st, slot);
+        hipLaunchKernelGGL((k_fold_init<T>), dim3(1), dim3(64), 0, stream, st, slot + s + 1);
         LAUNCH_CHECK();
     }
     const int *info_p = fold ? &slot[0].info : info;   // what the host polls
+    // the end of a cycle (npin 0: of none, before the first) and U(:,0) of the next
+    auto fold_next = [&](int npin) {
+        hipLaunchKernelGGL((k_form_u_fold<T>), dim3(gv), dim3(256), 0, stream, n, prow, (const Slot<T> *)(slot + s + 1),
+                           slot, (const T *)pc, npin, (const T *)r, (const T *)G, U, m1, resvec);
+        LAUNCH_CHECK();
+    };
+    if (fold) fold_next(0);
     int fold_first = 1;
     auto enqueue_fold = [&]() {
         // slot i is read by the i-th streaming kernel of the cycle, which
-        // writes slot i + 1; the last writes slot 0.  The first cycle has no
-        // omega step behind it: its partials count is zero.
-        hipLaunchKernelGGL((k_form_u_fold<T>), dim3(gv), dim3(256), 0, stream, n, prow, (const Slot<T> *)slot, slot + 1,
-                           (const T *)pc, fold_first ? 0 : gv, (const T *)r, (const T *)G, U, m1, resvec);
-        LAUNCH_CHECK();
+        // writes slot i + 1; the last writes slot 0: a cycle ends with its
+        // outcome known, as the unfolded one does (judged by the next cycle's
+        // first kernel, a solve paid one more cycle of launches: IDR(4), DIA,
+        // 131 072 rows, 10 steps 448 -> 419 us)
         for (int k = 0; k < s; k++) {
-            const Slot<T> *in = slot + 1 + k;
-            Slot<T> *out = slot + 2 + k;
+            const Slot<T> *in = slot + k;
+            Slot<T> *out = slot + 1 + k;
             op_apply<T>(A, U + (long)k * n, G + (long)k * n, w1, w2, EPI_PDOT, epd, &in->info, stream);
             prereduce(prow);
             const T *pin = k > 0 ? pn[(k - 1) % 2] : nullptr;
@@ -1274,7 +1285,7 @@ int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOp
                                    enparts, pin, k > 0 ? gv : 0, G, U, r, x, m1, resvec, pn[k % 2]);
             LAUNCH_CHECK();
         }
-        const Slot<T> *in = slot + 1 + s;
+        const Slot<T> *in = slot + s;
         if (m1) {
             hipLaunchKernelGGL((k_form_v<T>), dim3(gv), dim3(256), 0, stream, n, &in->info, r, m1, v);
             LAUNCH_CHECK();
@@ -1282,7 +1293,7 @@ int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOp
         op_apply<T>(A, v, t, w1, w2, EPI_OMEGA, eom, &in->info, stream);
         prereduce(3);
 #define OF(NV)                                                                                                       \
-    hipLaunchKernelGGL((k_omega_fold<T, NV>), dim3(gv), dim3(256), 0, stream, n, in, slot, epart, enparts,           \
+    hipLaunchKernelGGL((k_omega_fold<T, NV>), dim3(gv), dim3(256), 0, stream, n, in, slot + s + 1, epart, enparts,   \
                        (const T *)pn[(s - 1) % 2], gv, (const T *)omega_d, (const T *)v, (const T *)t, r, x,         \
                        (const T *)P, prow, conjP, resvec, pc, gv)
         if (prow <= 1) OF(1);
@@ -1292,6 +1303,7 @@ int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOp
         else OF(16);
 #undef OF
         LAUNCH_CHECK();
+        fold_next(gv);
         fold_first = 0;
     };
 
@@ -1366,8 +1378,16 @@ int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOp
     try {
         for (long c = 0; c < max_cycles && !done; c++) {
             // the first folded cycle differs from the others in an argument:
-            // it runs as launches, while the host captures the others
-            if (use_graph && !gexec && (c > 0 || !fold)) capture();
+            // it runs as launches, while the host captures the others; a
+            // solve that has ended with it needs no second (IDR(4), DIA,
+            // 131 072 rows, 5 steps 373 -> 260 us)
+            if (use_graph && !gexec && (c > 0 || !fold)) {
+                capture();
+                if (c > 0) {
+                    HIP_TRY(hipEventSynchronize(pe[(c - 1) % 2]));
+                    if (h_info[(c - 1) % 2] >= 0) break;
+                }
+            }
             if (gexec) HIP_TRY(hipGraphLaunch(gexec, stream));
             else enqueue_cycle();
             if (ar) {
@@ -1383,11 +1403,8 @@ int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOp
                 if (h_info[(c - 1) % 2] >= 0) done = true;
             }
         }
-        if (fold) {   // the last omega step's norm, and the outcome into the state
-            hipLaunchKernelGGL((k_form_u_fold<T>), dim3(gv), dim3(256), 0, stream, n, prow, (const Slot<T> *)slot, slot + 1,
-                               (const T *)pc, gv, (const T *)r, (const T *)G, U, m1, resvec);
-            LAUNCH_CHECK();
-            hipLaunchKernelGGL((k_fold_done<T>), dim3(1), dim3(1), 0, stream, (const Slot<T> *)(slot + 1), st);
+        if (fold) {   // the outcome into the state
+            hipLaunchKernelGGL((k_fold_done<T>), dim3(1), dim3(1), 0, stream, (const Slot<T> *)slot, st);
             LAUNCH_CHECK();
         }
         // final true residual (idrs.inc:304-310)

@@ -1,5 +1,5 @@
 """The folded IDR(s) cycle (reductions and scalar steps inside the streaming
-kernels, up to 2^18 rows) against the allocation-free entry, which always runs
+kernels, up to 3 * 2^16 rows) against the allocation-free entry, which always runs
 them as kernels of their own: the same sums in the same order, so x, the flag,
 the count, relres and the residual history are the same bits -- for shadow
 spaces on both sides of the kernel's 4-column form, stops at every step of a
@@ -77,7 +77,7 @@ def test_folded_cycle_options(gpu):
     _same(P8, b, 6, 1e-10, 300)
 
 
-@pytest.mark.parametrize("n", [1 << 18, (1 << 18) + 1])
+@pytest.mark.parametrize("n", [3 << 16, (3 << 16) + 1, 1 << 18, (1 << 18) + 1])
 def test_largest_folded_system(gpu, n):
     crs, _, _ = P.toeplitz_1d(n)
     A = idrs_amd.Matrix(idrs_amd.crs_format(n, n, crs.row_ptr, crs.col_ind, rval=crs.val))
