@@ -537,6 +537,7 @@ void batch_idrs_solve(const Operator &A, int s, const T *b, T *x, const SolveOpt
     // Systems small enough each run whole in one workgroup, without waiting
     // for each other (block.hip).
     if (block_fits<T>(A, nmax, s, o, true)) {
+        last_solve_path() = IDRS_PATH_WORKGROUP;
         DBuf scratch(block_scratch<T>(A, ntot, s, o)), bres(sizeof(BlockResult) * nsys);
         DBuf bom(sizeof(T) * std::max(1, o.n_omega));
         T *omega_d = nullptr;
@@ -569,6 +570,7 @@ void batch_idrs_solve(const Operator &A, int s, const T *b, T *x, const SolveOpt
         return;
     }
 
+    last_solve_path() = IDRS_PATH_TILES;
     const size_t vb = sizeof(T) * (size_t)ntot;
     DBuf bG(vb * s), bU(vb * s), br(vb), bt(vb), bw1(vb), bw2(vb), btmp(vb), bP(vb * prow);
     DBuf bpart(sizeof(T) * (size_t)MAX_NV * ntiles), bst(sizeof(State<T>) * nsys), bflag(sizeof(int) * nsys);

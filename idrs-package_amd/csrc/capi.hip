@@ -8,6 +8,7 @@
 #include "mm.hpp"
 #include "ritz.hpp"
 #include "general.hpp"
+#include "rowcode.hpp"
 #include "lu.hpp"
 
 #include <cstdarg>
@@ -654,6 +655,22 @@ extern "C" {
 
 const char *idrs_last_error(void) { return g_err.c_str(); }
 int idrs_version(void) { return 100; }
+
+int idrs_last_solve_path(int *path) {
+    return guarded([&] {
+        need(path, "null argument");
+        *path = last_solve_path();
+    });
+}
+
+int idrs_matrix_rowcode(idrs_matrix_t A, int *kind, int *distinct) {
+    return guarded([&] {
+        need(A && kind && distinct, "null argument");
+        const RowCode *rc = op_rowcode(A->op, true);
+        *kind = !rc ? 0 : rc->values ? 1 : 2;
+        *distinct = rc ? rc->npat : 0;
+    });
+}
 
 int idrs_release_pool(int64_t *bytes) {
     return guarded([&] {

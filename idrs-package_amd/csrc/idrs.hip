@@ -1091,6 +1091,11 @@ static void solve_in_block(const Operator &A, long n, int s, const T *b, T *x, c
     out.spmv_launches = 0;
 }
 
+int &last_solve_path() {
+    static thread_local int path = IDRS_PATH_NONE;
+    return path;
+}
+
 template <class T>
 int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOpts<T> &o, SolveStats &out,
                hipStream_t stream) {
@@ -1122,6 +1127,7 @@ int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOp
     if (ar && tm.enabled) throw std::invalid_argument("SpMV timing needs events: not in the allocation-free solve");
     if constexpr (std::is_same<T, double>::value || std::is_same<T, c128>::value) {
         if (!tm.enabled && block_fits<T>(A, n, s, o, false)) {
+            last_solve_path() = IDRS_PATH_WORKGROUP;
             solve_in_block<T>(A, n, s, b, x, o, out, cap_it, user_omega != 0, out_h, stream);
             return 0;
         }
@@ -1241,6 +1247,7 @@ int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOp
     // The folded cycle while a workgroup's share of the partials stays small
     // (the allocation-free solve has no room for the slots)
     const bool fold = !ar && prow <= PDOT_MAX && s <= FIN_S && n <= FOLD_ROWS && enparts <= FOLD_PARTS && gv <= FOLD_PARTS;
+    last_solve_path() = fold ? IDRS_PATH_FOLDED : IDRS_PATH_LAUNCHES;
     // slots of the state, two norm buffers, and the omega step's partials
     Buf bslot, bpn, bpc;
     Slot<T> *slot = nullptr;

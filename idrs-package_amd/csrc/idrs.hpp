@@ -1,6 +1,7 @@
 // IDR(s) solver (RIDRS/CIDRS) on the device.
 #pragma once
 
+#include "idrs_capi.h"
 #include "matrix.hpp"
 
 #include <stdexcept>
@@ -68,6 +69,9 @@ struct SolveOpts {
     Arena *arena = nullptr;
     bool inner = false;              // the inner solve of another solver's iteration
 };
+
+// how the calling thread's last IDR(s) solve ran (IDRS_PATH_*)
+int &last_solve_path();
 
 template <class T>
 int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOpts<T> &o, SolveStats &st,

@@ -95,6 +95,8 @@ _PROTOS = {
     "idrs_last_error": (ctypes.c_char_p, []),
     "idrs_version": (c_int, []),
     "idrs_device_count": (c_int, []),
+    "idrs_last_solve_path": (c_int, [POINTER(c_int)]),
+    "idrs_matrix_rowcode": (c_int, [c_void_p, POINTER(c_int), POINTER(c_int)]),
     "idrs_release_pool": (c_int, [POINTER(c_int64)]),
     "idrs_crs_format_f64": (c_int, [c_int, c_int, c_void_p, c_void_p, c_void_p, POINTER(c_void_p)]),
     "idrs_crs_format_c128": (c_int, [c_int, c_int, c_void_p, c_void_p, c_void_p, POINTER(c_void_p)]),

@@ -266,6 +266,13 @@ class Matrix:
         check(_lib.load().idrs_matrix_stored_values(self._h, ctypes.byref(cnt), ctypes.byref(unit)))
         return cnt.value, bool(unit.value)
 
+    def rowcode(self):
+        """(kind, distinct rows) of the row code that products of real vectors
+        use now: kind None, "values" or "offsets"."""
+        k, d = ctypes.c_int(0), ctypes.c_int(0)
+        check(_lib.load().idrs_matrix_rowcode(self.handle, ctypes.byref(k), ctypes.byref(d)))
+        return (None, "values", "offsets")[k.value], d.value
+
     def set_seed(self, seed):
         self.seed = seed
         lib = _lib.load()
@@ -1159,6 +1166,14 @@ def ms_scaleback(A, alpha_s, Y, out=None):
     f = lib.idrs_ms_scaleback_c128 if cplx else lib.idrs_ms_scaleback_f64
     check(f(A.handle, ns, d, a.ctypes.data, _ptr(Yc), _ptr(Xc), 0))
     return Xc.T
+
+
+def last_solve_path():
+    """How the calling thread's last IDR(s) solve ran: "launches", "folded",
+    "workgroup" or "tiles" (None before the first)."""
+    p = ctypes.c_int(0)
+    check(_lib.load().idrs_last_solve_path(ctypes.byref(p)))
+    return (None, "launches", "folded", "workgroup", "tiles")[p.value]
 
 
 def release_pool():

@@ -563,6 +563,21 @@ int idrs_make_p_c128(int n, int s, int method, const double *PT_raw, const doubl
 /* Number of HIP devices visible (0 without a GPU); never fails. */
 int idrs_device_count(void);
 
+/* How the calling thread's last IDR(s) solve (single, batched or inner) ran:
+   a kernel per statement group, with the reductions folded into the kernels
+   that use them, whole in one workgroup (per system of a batch), or per tile
+   of a batch.  The library chooses by size and form. */
+#define IDRS_PATH_NONE 0
+#define IDRS_PATH_LAUNCHES 1
+#define IDRS_PATH_FOLDED 2
+#define IDRS_PATH_WORKGROUP 3
+#define IDRS_PATH_TILES 4
+int idrs_last_solve_path(int *path);
+
+/* The row code that A's products of real vectors use now: *kind 0 none, 1 the
+   rows' values and offsets, 2 the offsets alone; *distinct: its distinct rows. */
+int idrs_matrix_rowcode(idrs_matrix_t A, int *kind, int *distinct);
+
 /* Frees the device buffers that the library keeps for reuse between calls
    (at most a quarter of each device's memory), for another allocator of the
    process; *bytes (may be NULL): the bytes freed.  Waits for the device. */

@@ -63,6 +63,7 @@ def test_small_solves_match_oracle(gpu, n, s, form):
     k = min(10, n)
     g = idrs_amd.idrs(A, b, s, tolerance=0.0, maximum_iterations=k, PT_raw=PT, resvec=True, **kw)
     o = orc.idrs(Ao, b, s, tolerance=0.0, maximum_iterations=k, PT_raw=PT, **okw)
+    assert idrs_amd.last_solve_path() == ("workgroup" if n <= 2560 else "folded")
     assert g.iterations == o[3]
     if n > 2:   # one or two unknowns end in a breakdown on both sides
         assert g.flag == o[1] and rel(g.x, o[0]) < 1e-10
@@ -77,6 +78,7 @@ def test_small_batches_match_oracle(gpu, sizes, s):
     K = idrs_amd.batch_format([idrs_amd.crs_format(c.n, c.n, c.row_ptr, c.col_ind, rval=c.val) for c in systems])
     b = np.random.default_rng(5).uniform(-1, 1, sum(sizes))
     r = idrs_amd.idrs_batched(idrs_amd.Matrix(K), b, s, tolerance=1e-9, maximum_iterations=300)
+    assert idrs_amd.last_solve_path() == ("workgroup" if max(sizes) <= 4096 else "tiles")
     at = 0
     for k, c in enumerate(systems):
         bk = b[at:at + c.n]
@@ -105,5 +107,6 @@ def test_single_solve_on_a_batch_matrix(gpu, sizes, entry):
     PT = P.gaussian_shadow(n, s, seed=2)
     solve = idrs_amd.idrs if entry == "host" else idrs_amd.idrs_ritz
     g = solve(idrs_amd.Matrix(KB), b, s, tolerance=0.0, maximum_iterations=10, PT_raw=PT)
+    assert idrs_amd.last_solve_path() == ("workgroup" if n <= 2560 else "folded")
     o = orc.idrs(orc.OracleMatrix(orc.CRS, n, crs=whole), b, s, tolerance=0.0, maximum_iterations=10, PT_raw=PT)
     assert (g.flag, g.iterations) == (o[1], o[3]) and rel(g.x, o[0]) < 1e-10

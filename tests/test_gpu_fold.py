@@ -40,10 +40,12 @@ def _solve(f, A, b, s, tol, maxit, variant=1, M1=None, omega=None):
     return x.cpu().numpy(), st.flag, st.iterations, st.relres, rv[: st.iterations + 1]
 
 
-def _same(A, b, s, tol, maxit, **kw):
+def _same(A, b, s, tol, maxit, path="folded", **kw):
     lib = _lib.load()
     g = _solve(lib.idrs_idrs_f64, A, b, s, tol, maxit, **kw)
+    assert idrs_amd.last_solve_path() == path
     w = _solve(lib.idrs_idrs_f64_noalloc, A, b, s, tol, maxit, **kw)
+    assert idrs_amd.last_solve_path() == "launches"
     assert g[1:4] == w[1:4]
     assert np.array_equal(g[0], w[0]) and np.array_equal(g[4], w[4])
     return g
@@ -80,8 +82,18 @@ def test_folded_cycle_options(gpu):
 @pytest.mark.parametrize("n", [3 << 16, (3 << 16) + 1, 1 << 18, (1 << 18) + 1])
 def test_largest_folded_system(gpu, n):
     crs, _, _ = P.toeplitz_1d(n)
-    A = idrs_amd.Matrix(idrs_amd.crs_format(n, n, crs.row_ptr, crs.col_ind, rval=crs.val))
-    _same(A, _b(n, 3), 2, 0.0, 8)
+    K = idrs_amd.crs_format(n, n, crs.row_ptr, crs.col_ind, rval=crs.val)
+    K.set_group(1)          # one thread per row: a partial per 256 rows
+    _same(idrs_amd.Matrix(K), _b(n, 3), 2, 0.0, 8, path="folded" if n <= 3 << 16 else "launches")
+
+
+@pytest.mark.parametrize("n", [163840, 163841 + 1024])
+def test_largest_folded_product_grid(gpu, n):
+    """Eight lanes per row: 128 rows a partial, 1280 partials the most folded."""
+    crs, _, _ = P.toeplitz_1d(n)
+    K = idrs_amd.crs_format(n, n, crs.row_ptr, crs.col_ind, rval=crs.val)
+    K.set_group(8)
+    _same(idrs_amd.Matrix(K), _b(n, 4), 3, 0.0, 9, path="folded" if n <= 163840 else "launches")
 
 
 @pytest.mark.parametrize("k", [1, 5, 6, 23, 24, 70])
