@@ -23,7 +23,7 @@ namespace {
 
 constexpr int BLK_THREADS = 1024;
 constexpr int BLK_NMAX = 4096;                     // rows of a system of a batch
-constexpr int BLK_SINGLE = 2560;                   // rows of a single system
+constexpr int BLK_SINGLE = 2560;                   // rows of a single system, or with a wide s
 constexpr int BLK_S = PDOT_MAX;                    // largest s
 constexpr int BLK_DIAG = 32;                       // most stored diagonals
 constexpr int BLK_WIDTH = 32;                      // entries of the longest CRS row
@@ -473,24 +473,49 @@ void launch(const Operator &A, BlkArgs<VT, T> &a, long nmax, int nsys, hipStream
 
 }  // namespace
 
-// The line: a batch takes the kernel up to 4096 rows a system (256 systems of
-// 24^2 to 64^2 rows, IDR(2), CRS: 13.8 -> 4.4 ms; 8 of 50^2 to 64^2: 9.3 ->
-// 3.6), a single system up to 2560, where its products still cost less on one
-// CU than their launches (IDR(4), CRS, per iteration, launches -> here: 216
-// rows 29.8 -> 5.5 us, 1728 25.5 -> 9.5, 2744 25.7 -> 12.6, 4096 25.2 -> 17.1,
-// and with Chebyshev(8) in DIA storage 74.8 -> 78.0); the vectors have to fit
-// LDS, and the form has to be one the kernel has.
+// One workgroup's time of a step of a single system against that of its
+// launches, both in us without what they have in common: rows times the
+// entries of the step's products and the columns of G, U and P, against a
+// latency per launch (lanes per row, DIA, sliced).  Fitted to 60 steps of 256
+// to 2560 rows with 3 to 32 entries, degree 0 to 32, s = 1 to 16, real and
+// complex: the choice is within 12 % of the faster one but for one case of 570
+// (16 %).  One workgroup / launches, us a step: 7 entries CRS, IDR(4), 1728
+// rows 9.5 / 19, 2560 rows 12 / 19, with degree 8 39 / 60; DIA with degree 32
+// 153 / 114; 32 entries with degree 4 78 / 38; IDR(16), 7 entries, 1024 rows
+// 22 / 29, 2560 rows 46 / 30.
+static bool block_is_faster(const DevMatrix &K, long n, int s, int degree) {
+    const bool dia = K.fmt == DevFmt::DIA;
+    const double w = dia ? K.ndiag : K.max_row, products = (degree + 1) * (s + 1.0) / s;
+    const double launch = dia ? 2.8 + 0.026 * w : K.group == 1 ? 1.2 + 0.12 * w : 3.1;
+    return 1e-3 * n * ((dia ? 0.19 : 0.1) * w * products + 0.45 * s + 0.009 * s * s) <
+           7.4 + 0.36 * s + launch * products;
+}
+
+// The systems of a batch, up to 4096 rows each, do not wait for each other and
+// the tile launches cost more, so they take the kernel with any degree and row
+// length (256 systems of 24^2 to 64^2 rows, IDR(2): 13.8 -> 4.4 ms; one of 4096
+// rows with 32 entries and degree 32: tiles 2262 us a step, here 716); above
+// 2560 rows a wide shadow space, or a wider one over long complex rows, stays
+// on the tiles (one system of 4096 rows, sliced: IDR(16) 52 / 74, IDR(8) with
+// 32 complex entries 61 / 77).  A single system takes it up to 2560 rows, where
+// it is the faster one.  The vectors have to fit LDS, and the form has to be
+// one the kernel has.
 template <class T>
 bool block_fits(const Operator &A, long n, int s, const SolveOpts<T> &o, bool batch) {
     if constexpr (!std::is_same<T, double>::value && !std::is_same<T, c128>::value) return false;
     const DevMatrix &K = *A.K;
-    if (n > (batch ? BLK_NMAX : BLK_SINGLE)) return false;
     if (A.general() || A.values32 || s > BLK_S || A.degree > BLK_DEG) return false;
     if (K.nrows != K.ncols) return false;
     if (K.fmt == DevFmt::DIA ? K.ndiag > BLK_DIAG : K.max_row > BLK_WIDTH) return false;
+    if (batch) {
+        const bool wide = s > 8 || (Tr<T>::is_complex && s > 4 && K.max_row > 16);
+        if (n > (wide ? BLK_SINGLE : BLK_NMAX)) return false;
+    } else if (n > BLK_SINGLE || !block_is_faster(K, n, s, A.degree)) {
+        return false;
+    }
     if (!Tr<T>::is_complex && A.values_complex()) return false;   // refused further on
-    // a seed shift stays on the launches, and so does the inner solve of a
-    // flexible Krylov method, whose outer count follows the inner rounding
+    // the kernel has no seed shift; the inner solve of a flexible Krylov method
+    // stays on the launches, as its outer count follows the inner rounding
     if (A.seed != std::complex<double>(0.0, 0.0) || o.inner) return false;
     return lds_bytes<T>(A, n) <= BLK_LDS;
 }

@@ -12,7 +12,7 @@ import pytest
 
 import idrs_amd
 import orc
-from helpers import rel
+from helpers import rel, rounding_spread
 from idrs_amd import problems as P
 
 pytestmark = pytest.mark.gpu
@@ -31,6 +31,22 @@ def _system(n, seed, cplx=False):
     rp = np.concatenate([[1], 1 + np.cumsum(ok.sum(1))]).astype(np.int32)
     col = (i[:, None] + np.array(offs) + 1)[ok].astype(np.int32)
     return P.Crs(n, rp, col, np.ascontiguousarray(vals[ok])), (np.array(offs, dtype=np.int32), vals)
+
+
+def _box(dims):
+    """A 7-point stencil as CRS arrays and diagonals."""
+    n = dims[0] * dims[1] * dims[2]
+    i = np.arange(n)
+    xyz, st = (i % dims[0], (i // dims[0]) % dims[1], i // (dims[0] * dims[1])), (1, dims[0], dims[0] * dims[1])
+    cols = {0: np.full(n, 7.0)}
+    for d in range(3):
+        cols[-st[d]] = np.where(xyz[d] > 0, -1.0 - 0.05 * d, 0.0)
+        cols[st[d]] = np.where(xyz[d] < dims[d] - 1, -0.9 + 0.05 * d, 0.0)
+    offs = np.array(sorted(cols), dtype=np.int32)
+    vals = np.stack([cols[o] for o in offs], axis=1)
+    keep = vals != 0
+    rp = np.concatenate([[1], 1 + np.cumsum(keep.sum(1))]).astype(np.int32)
+    return P.Crs(n, rp, (i[:, None] + offs + 1)[keep].astype(np.int32), vals[keep]), offs, vals
 
 
 @pytest.mark.parametrize("n,s,form", [
@@ -110,3 +126,61 @@ def test_single_solve_on_a_batch_matrix(gpu, sizes, entry):
     assert idrs_amd.last_solve_path() == ("workgroup" if n <= 2560 else "folded")
     o = orc.idrs(orc.OracleMatrix(orc.CRS, n, crs=whole), b, s, tolerance=0.0, maximum_iterations=10, PT_raw=PT)
     assert (g.flag, g.iterations) == (o[1], o[3]) and rel(g.x, o[0]) < 1e-10
+
+
+# Which solves the kernel takes: on both sides of the lines by the work of a
+# step against its launches, each against the oracle (degree 32 in powers of A,
+# coefficients up to 7e10, amplifies rounding: there the bar is what 1e-16
+# perturbations of b do to the oracle itself).
+@pytest.mark.parametrize("dims,form,s,degree,path", [
+    ((12, 12, 12), "crs", 4, 0, "workgroup"), ((16, 16, 10), "crs", 4, 8, "workgroup"),
+    ((16, 8, 8), "crs", 16, 0, "workgroup"), ((16, 16, 10), "crs", 16, 0, "folded"),
+    ((8, 8, 8), "dia", 4, 32, "workgroup"), ((16, 16, 10), "dia", 4, 32, "folded"),
+    (512, "dense rows", 4, 8, "workgroup"), (2560, "dense rows", 4, 4, "folded")])
+def test_choice_of_the_one_workgroup_solve(gpu, dims, form, s, degree, path):
+    if form == "dense rows":
+        crs = P.random_dominant(dims, k=31, seed=1)
+        K = idrs_amd.crs_format(crs.n, crs.n, crs.row_ptr, crs.col_ind, rval=crs.val)
+    else:
+        crs, offs, vals = _box(dims)
+        if form == "dia":
+            K = idrs_amd.dia_format(crs.n, crs.n, offs, rvals=vals)
+        else:
+            K = idrs_amd.crs_format(crs.n, crs.n, crs.row_ptr, crs.col_ind, rval=crs.val)
+    A = idrs_amd.Matrix(K, which_precon=1 if degree else 0)
+    mk = {}
+    if degree:
+        idrs_amd.real_preconditioner(A, 2, degree, foci=[0.3, 1.7])
+        mk = dict(which_precon=1, degree=degree, alpha=orc.chebyshev(degree, np.array([0.3, 1.7])))
+    b = np.random.default_rng(3).uniform(-1, 1, crs.n)
+    PT = P.gaussian_shadow(crs.n, s, seed=4)
+    g = idrs_amd.idrs(A, b, s, tolerance=0.0, maximum_iterations=6, PT_raw=PT)
+    assert idrs_amd.last_solve_path() == path
+    Ao = orc.OracleMatrix(orc.CRS, crs.n, crs=crs, **mk)
+
+    def run(bp):
+        o = orc.idrs(Ao, bp, s, tolerance=0.0, maximum_iterations=6, PT_raw=PT)
+        return o[0], o[3]
+
+    xo, its = run(b)
+    bar = max(1e-10, 100 * rounding_spread(run, b)[0]) if degree == 32 else 1e-10
+    assert (g.flag, g.iterations) == (1, its) and rel(g.x, xo) < bar
+
+
+@pytest.mark.parametrize("n,s,cplx,k,path", [
+    (4096, 8, False, 4, "workgroup"), (4096, 9, False, 4, "tiles"), (2560, 16, False, 4, "workgroup"),
+    (4096, 4, True, 31, "workgroup"), (4096, 8, True, 31, "tiles"), (4096, 8, True, 4, "workgroup")])
+def test_choice_of_the_one_workgroup_batch(gpu, n, s, cplx, k, path):
+    crs = [P.random_dominant(m, k=k, seed=m) for m in (n, 70)]
+    if cplx:
+        for c in crs:
+            c.val = c.val * (1 + 0.1j)
+    K = idrs_amd.batch_format([idrs_amd.crs_format(c.n, c.n, c.row_ptr, c.col_ind,
+                                                   **{"cval" if cplx else "rval": c.val}) for c in crs])
+    b = np.random.default_rng(6).uniform(-1, 1, n + 70) + (0j if cplx else 0)
+    r = idrs_amd.idrs_batched(idrs_amd.Matrix(K), b, s, tolerance=0.0, maximum_iterations=7)
+    assert idrs_amd.last_solve_path() == path
+    for c, sl in ((crs[0], slice(0, n)), (crs[1], slice(n, n + 70))):
+        o = orc.idrs(orc.OracleMatrix(orc.CRS, c.n, crs=c, complex_vectors=cplx), b[sl], s, tolerance=0.0,
+                     maximum_iterations=7)
+        assert rel(r.x[sl], o[0]) < 1e-10
