@@ -94,7 +94,7 @@ static int idrs_entry(idrs_matrix_t A, int n, const double *b, int s, const idrs
     return guarded([&] {
         need(A && b && x, "null argument");
         hipStream_t st = lib_stream();
-        op_prepare(A->op, st);
+        op_prepare_solve<T>(A->op, st);
         idrs_opts_t o{};
         if (opts) o = *opts;
         SolveOpts<T> so;
@@ -169,7 +169,7 @@ static int ritz_entry(idrs_matrix_t A, int n, const double *b, int s, const idrs
         need((n_omega == 0 || omega) && (dim_u0 == 0 || U0) && ((h_rows == 0 && h_cols == 0) || H),
              "output array missing");
         hipStream_t st = lib_stream();
-        op_prepare(A->op, st);
+        op_prepare_solve<T>(A->op, st);
         idrs_opts_t o{};
         if (opts) o = *opts;
         need(!o.U0 && !o.omega && !o.H, "IDRS_RITZ returns U0, omega and H; it takes none of them");
@@ -324,7 +324,7 @@ static int krylov_entry(Kry kind, idrs_matrix_t A, int n, const double *b, int n
         need(A && b && X, "null argument");
         need(kind == Kry::QMRIDR || (sigma && ns >= 1), "sigma must hold at least one shift");
         hipStream_t st = lib_stream();
-        op_prepare(A->op, st);
+        op_prepare_solve<T>(A->op, st);
         idrs_krylov_opts_t o{};
         if (opts) o = *opts;
         KrylovOpts<T> ko;
@@ -504,7 +504,7 @@ static int mixed_entry(idrs_matrix_t A, int n, const double *b, int s, const idr
         need(A && b && x, "null argument");
         need(s >= 1 && s <= SMAX, "s must be in 1..64");
         hipStream_t st = lib_stream();
-        op_prepare(A->op, st);
+        op_prepare_solve<T>(A->op, st);
         idrs_opts_t o{};
         if (opts) o = *opts;
         need(!o.has_M1 && !o.U0 && !o.resvec && !o.omega && !o.H, "M1, U0, omega, resvec and H are not offered here");

@@ -44,6 +44,7 @@ inline hipError_t dev_malloc(V **p, size_t bytes) { return dev_malloc_bytes((voi
 // runs on the library's stream, so a buffer taken again is written after its
 // last reader.
 void *pool_alloc(size_t bytes);
+void *pool_try_alloc(size_t bytes);   // null: no memory
 void pool_free(void *p, size_t bytes);
 void *pinned_take(size_t bytes, unsigned flags);
 void pinned_give(void *p, size_t bytes, unsigned flags);

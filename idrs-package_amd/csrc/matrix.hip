@@ -454,7 +454,7 @@ const RowCode *op_rowcode(const Operator &op, bool offsets) {
     if (K.fmt == DevFmt::CRS && !(K.group == 1 && K.sell)) return nullptr;
     if (op.values32 && op.seed != std::complex<double>(0.0, 0.0)) return nullptr;   // refused by with_args
     if (op.seed.imag() != 0.0) return nullptr;
-    if (const RowCode *rc = (op.sval ? op.rowcode : K.rowcode).get()) return rc;
+    if (const RowCode *rc = op.sval ? op.rowcode.get() : K.rowcode.get()) return rc;
     if (!offsets || op.values32 || op.values_complex() || K.fmt != DevFmt::CRS) return nullptr;
     const void *sliced = op.sval ? op.sl_sval : K.sell->sl_val;
     return sliced ? K.offcode.get() : nullptr;
@@ -769,8 +769,8 @@ static void *sliced_copy(const Sell &S, const void *src, bool cplx, hipStream_t 
 // buffer (a free would synchronize the device on every refresh); the FP32
 // copy is dropped and rebuilt when next needed
 static void refresh_sliced(DevMatrix &K, hipStream_t st) {
-    K.rowcode.reset();
-    K.rowcode_tried = true;
+    K.rowcode.drop(true);
+    K.values_set = true;
     if (!K.sell) return;
     if (K.sell->sl_val32) {
         (void)hipFree(K.sell->sl_val32);
@@ -1035,28 +1035,24 @@ bool op_prepared(const Operator &op) {
     return sliced && (!op.general() || (op.gws && op.gws_rows == op.rows()));
 }
 
-// Looks for the row code of the values that op's products read, once per
-// matrix (scaled values: per operator).  With fresh values every few solves
-// (set_values, transposes) it is not looked for.
 static void prepare_rowcode(const Operator &op, hipStream_t st) {
-    static std::mutex mu;
     const DevMatrix &K = *op.K;
-    std::lock_guard<std::mutex> g(mu);
+    std::lock_guard<std::mutex> g(K.code_mu);
     if (K.fmt == DevFmt::CRS && !(K.group == 1 && K.sell)) return;   // not read in that layout
-    bool &tried = op.sval ? op.rowcode_tried : K.rowcode_tried;
-    std::shared_ptr<RowCode> &rc = op.sval ? op.rowcode : K.rowcode;
-    if (!tried && !(op.sval && K.tperm)) {
-        rc = make_rowcode(op, true, st);
-        tried = true;
-    }
-    if (!rc && !K.offcode_tried) {
-        K.offcode = make_rowcode(op, false, st);
-        K.offcode_tried = true;
-    }
+    CodeSlot &slot = op.sval ? op.rowcode : K.rowcode;
+    if (!slot.tried && !(op.sval && K.tperm) && !K.values_set) slot.set(make_rowcode(op, true, st));
+    if (!slot.get() && !K.offcode.tried) K.offcode.set(make_rowcode(op, false, st));
 }
 
+template <class T>
+void op_prepare_solve(const Operator &op, hipStream_t st) {
+    op_prepare(op, st);
+    if constexpr (std::is_same<T, double>::value) prepare_rowcode(op, st);
+}
+template void op_prepare_solve<double>(const Operator &, hipStream_t);
+template void op_prepare_solve<c128>(const Operator &, hipStream_t);
+
 void op_prepare(const Operator &op, hipStream_t st) {
-    prepare_rowcode(op, st);
     if (op_prepared(op)) return;
     const DevMatrix &K = *op.K;
     if (!(K.fmt != DevFmt::CRS || !K.sell || !op.sval || op.sl_sval))
@@ -1260,8 +1256,7 @@ static void drop_unit_diagonal(Operator &op, bool cvals, hipStream_t st) {
         HIP_TRY(hipMemcpyAsync(dst + vsz * n * z0, src + vsz * n * (z0 + 1), vsz * n * (K.ndiag - 1 - z0),
                                hipMemcpyDeviceToDevice, st));
     HIP_TRY(hipStreamSynchronize(st));
-    op.rowcode.reset();
-    op.rowcode_tried = false;
+    op.rowcode.drop(false);
     (void)hipFree(op.sval);
     op.sval = packed;
     op.unit_diag = z0;
@@ -1287,8 +1282,7 @@ void op_set_diag_precon(Operator &op, int which, const std::complex<double> *shi
     (void)hipFree(op.sl_sval);
     (void)hipFree(op.sl_sval32);
     op.pdiag = op.sval = op.sval32 = nullptr;
-    op.rowcode.reset();
-    op.rowcode_tried = false;
+    op.rowcode.drop(false);
     op.sl_sval = op.sl_sval32 = nullptr;
     op.unit_diag = -1;
     op.which_precon = which;
@@ -1371,8 +1365,7 @@ void op_set_diag_values(Operator &op, const std::vector<std::complex<double>> &d
     (void)hipFree(op.sl_sval);
     (void)hipFree(op.sl_sval32);
     op.pdiag = op.sval = op.sval32 = nullptr;
-    op.rowcode.reset();
-    op.rowcode_tried = false;
+    op.rowcode.drop(false);
     op.sl_sval = op.sl_sval32 = nullptr;
     op.unit_diag = -1;
     op.which_precon = 1;

@@ -5,8 +5,10 @@
 
 #include "common.hpp"
 
+#include <atomic>
 #include <complex>
 #include <memory>
+#include <mutex>
 #include <vector>
 
 namespace idrs {
@@ -68,6 +70,28 @@ struct Sell {
 
 struct RowCode;
 
+// A matrix's or an operator's row code (rowcode.hpp).  Looked for once, by the
+// thread that holds the matrix's code_mu; a reader sees none or a whole one.
+struct CodeSlot {
+    bool tried = false;
+    const RowCode *get() const { return now.load(std::memory_order_acquire); }
+    void set(std::shared_ptr<RowCode> rc) {
+        tried = true;
+        own = std::move(rc);
+        now.store(own.get(), std::memory_order_release);
+    }
+    // forgets it; searched: and is not looked for again
+    void drop(bool searched) {
+        now.store(nullptr, std::memory_order_release);
+        own.reset();
+        tried = searched;
+    }
+
+private:
+    std::shared_ptr<RowCode> own;
+    std::atomic<const RowCode *> now{nullptr};
+};
+
 struct DevMatrix {
     int orig_format = 0;     // user_module matrix_format: 2 CRS, 3 COO, 4 CDS, 5 DIA
     DevFmt fmt = DevFmt::CRS;
@@ -97,13 +121,13 @@ struct DevMatrix {
     std::unique_ptr<Partition> part;
     // set for transposes (make_transpose): val[p] = source val[tperm[p]]
     int *tperm = nullptr;
-    // row code of K's own values (rowcode.hpp), made by op_prepare; tried:
-    // looked for, or values that change too often to look
-    mutable std::shared_ptr<RowCode> rowcode;
-    mutable bool rowcode_tried = false;
-    // code of the column offsets alone (CRS in the sliced layout)
-    mutable std::shared_ptr<RowCode> offcode;
-    mutable bool offcode_tried = false;
+    // row codes of K's own values, and of the column offsets alone (CRS in
+    // the sliced layout), made by op_prepare_solve
+    mutable CodeSlot rowcode, offcode;
+    mutable std::mutex code_mu;
+    // the values have been replaced since the upload: more will follow, and
+    // the values are not coded any more (scaled ones neither)
+    bool values_set = false;
     ~DevMatrix();
 };
 
@@ -152,9 +176,7 @@ struct Operator {
     std::shared_ptr<LuFactor> lu;
     bool shift_invert = false;
     std::complex<double> si_shift{0.0, 0.0};
-    // row code of the scaled values, made by op_prepare
-    mutable std::shared_ptr<RowCode> rowcode;
-    mutable bool rowcode_tried = false;
+    mutable CodeSlot rowcode;        // row code of the scaled values
     mutable void *gws = nullptr;     // workspace of the general path (gen_prepare)
     mutable long gws_rows = 0;
     bool general() const { return Mm || Cm || block || ndefl > 0 || lu || shift_invert; }
@@ -268,6 +290,11 @@ void build_sell(DevMatrix &K, hipStream_t st);
 void op_prepare(const Operator &op, hipStream_t st);
 // true when op_prepare has nothing left to build for op
 bool op_prepared(const Operator &op);
+// op_prepare, and for a solve's products of real vectors the row code of the
+// values they read, looked for once per matrix (scaled values: per operator).
+// A single product does not look: the search takes as long as several.
+template <class T>
+void op_prepare_solve(const Operator &op, hipStream_t st);
 // block-diagonal CRS matrix of nsys square CRS systems (copies), with its
 // Partition
 DevMatrix *make_blockdiag(int nsys, const DevMatrix *const *Ks);

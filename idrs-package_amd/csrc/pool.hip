@@ -63,11 +63,14 @@ size_t pool_release() {
     return freed;
 }
 
-void *pool_alloc(size_t bytes) {
-    bytes = pool_round(bytes);
+void *pool_try_alloc(size_t bytes) {
     int dev = 0;
     HIP_TRY(hipGetDevice(&dev));
-    void *p = device_pool(dev).take(bytes);
+    return device_pool(dev).take(pool_round(bytes));
+}
+
+void *pool_alloc(size_t bytes) {
+    void *p = pool_try_alloc(bytes);
     if (!p) {
         set_last_error("no device memory for %zu bytes", bytes);
         throw HipError{hipErrorOutOfMemory};

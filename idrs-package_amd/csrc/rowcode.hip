@@ -67,8 +67,8 @@ struct Work {
     int count, bad;
 };
 
-// Puts the hashes of the rows q * step into the table; more than ROWCODE_MAX
-// of them: bad, and later rows are skipped.  Ordinary loads see nearly every
+// Puts the hashes of one row in each 'step' rows into the table; more than
+// ROWCODE_MAX of them: bad, and later rows are skipped.  Ordinary loads see nearly every
 // row's hash already there; a line read before its key was written only costs
 // an atomic that finds the key.  A quarter-filled table has no probe sequence
 // of PROBES, so one that long means an overfull table.
@@ -76,7 +76,10 @@ constexpr int PROBES = 64;
 __global__ __launch_bounds__(256) void k_find_rows(RowSrc S, long rows, long step, Work *w) {
     for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < rows; q += (long)gridDim.x * blockDim.x) {
         if (w->bad) return;
-        const int row = (int)(q * step);
+        // not always the first of them: on a box of 64 rows a side every 64th row
+        // is a boundary row, and a kind of row that the sample misses costs an
+        // atomic per row in the next pass (search at 64^3 690 us, so 230)
+        const int row = (int)min(q * step + (long)((unsigned long)q * 2654435761UL % (unsigned long)step), S.nrows - 1L);
         const unsigned long long h = S.hash(row);
         unsigned s = (unsigned)h % HSLOTS;
         int probe = 0;
@@ -96,12 +99,18 @@ __global__ __launch_bounds__(256) void k_find_rows(RowSrc S, long rows, long ste
     }
 }
 
-// numbers the distinct rows and writes the table
+// numbers the distinct rows and writes the table; too many of them, or too
+// large a table: bad
 __global__ __launch_bounds__(256) void k_row_table(RowSrc S, Work *w, int width, RowEntry *ent, RowEntry *ent32,
                                                    int *len) {
-    __shared__ int next;
-    if (threadIdx.x == 0) next = 0;
+    __shared__ int next, skip;
+    if (threadIdx.x == 0) {
+        next = 0;
+        skip = w->bad || w->count > ROWCODE_MAX || w->count * width > ROWCODE_ENTRIES;
+        if (skip) w->bad = 1;
+    }
     __syncthreads();
+    if (skip) return;
     for (int s = threadIdx.x; s < HSLOTS; s += blockDim.x)
         if (w->key[s]) {
             const int p = atomicAdd(&next, 1);
@@ -121,7 +130,9 @@ __global__ __launch_bounds__(256) void k_row_table(RowSrc S, Work *w, int width,
 // differs from the one of its hash)
 __global__ __launch_bounds__(256) void k_code_rows(RowSrc S, Work *w, int width, const RowEntry *ent, const int *len,
                                                    unsigned char *code) {
-    for (int row = blockIdx.x * blockDim.x + threadIdx.x; row < S.nrows; row += gridDim.x * blockDim.x) {
+    for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < S.nrows; q += (long)gridDim.x * blockDim.x) {
+        if (w->bad) return;
+        const int row = (int)q;
         const unsigned long long h = S.hash(row);
         unsigned s = (unsigned)h % HSLOTS;
         int probe = 0;
@@ -307,31 +318,19 @@ void launch_pat(const DevMatrix &K, const RowCode &rc, bool f32, const SpmvArgs<
     LAUNCH_CHECK();
 }
 
-// null: no device memory left
-template <class V>
-V *dev_new(size_t count) {
-    V *p = nullptr;
-    const hipError_t e = dev_malloc(&p, sizeof(V) * std::max<size_t>(1, count));
-    if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    HIP_TRY(e);
-    return p;
-}
-
 }  // namespace
 
-RowCode::~RowCode() {
-    (void)hipFree(code);
-    (void)hipFree(ent);
-    (void)hipFree(ent32);
-    (void)hipFree(len);
-}
+RowCode::~RowCode() { pool_free(mem, bytes); }
 
+// Zeroing, the sample, all rows, the table and the codes are enqueued at once
+// and waited for once; the first that finds too many distinct rows ends the
+// rest at their start.  Buffers come from the pool: a program that builds a
+// matrix per solve pays no allocation for it.
 std::shared_ptr<RowCode> make_rowcode(const Operator &op, bool values, hipStream_t st) {
     const DevMatrix &K = *op.K;
-    if (K.kind == ValKind::Complex || (values && op.values_complex()) || (!values && K.fmt != DevFmt::CRS) || K.part || K.nrows != K.ncols || K.nrows < ROWCODE_MIN_ROWS) return nullptr;
+    if (K.kind == ValKind::Complex || (values && op.values_complex())) return nullptr;
+    if (!values && K.fmt != DevFmt::CRS) return nullptr;
+    if (K.part || K.nrows != K.ncols || K.nrows < ROWCODE_MIN_ROWS) return nullptr;
     RowSrc S{};
     S.nrows = K.nrows;
     S.ncols = K.ncols;
@@ -349,56 +348,37 @@ std::shared_ptr<RowCode> make_rowcode(const Operator &op, bool values, hipStream
         if (op.sval && op.unit_diag >= 0) S.ud = op.unit_diag;
     }
     if (width < 1 || width > ROWCODE_WIDTH) return nullptr;
-    // the code is optional: without memory for it the products stay uncoded
-    Work *w = dev_new<Work>(1);
-    if (!w) return nullptr;
-    std::shared_ptr<RowCode> rc;
-    try {
-        const int g = vec_grid(K.nrows);
-        auto counts = [&](int &count, int &bad) {
-            int c[2];
-            HIP_TRY(hipMemcpyAsync(c, &w->count, sizeof c, hipMemcpyDeviceToHost, st));
-            HIP_TRY(hipStreamSynchronize(st));
-            count = c[0];
-            bad = c[1];
-        };
-        hipLaunchKernelGGL(k_zero_work, dim3(1), dim3(256), 0, st, w);
-        LAUNCH_CHECK();
-        // a sample of 4096 rows turns away most matrices that do not repeat
-        const long rows = K.nrows, step = std::max<long>(1, rows / 4096);
-        int count = 0, bad = 0;
-        hipLaunchKernelGGL(k_find_rows, dim3(16), dim3(256), 0, st, S, (rows + step - 1) / step, step, w);
-        LAUNCH_CHECK();
-        counts(count, bad);
-        if (!bad) {
-            hipLaunchKernelGGL(k_find_rows, dim3(g), dim3(256), 0, st, S, rows, 1L, w);
-            LAUNCH_CHECK();
-            counts(count, bad);
-        }
-        if (!bad && count <= ROWCODE_MAX && count * width <= ROWCODE_ENTRIES) {
-            rc = std::make_shared<RowCode>();
-            rc->npat = count;
-            rc->values = values;
-            rc->width = width;
-            rc->code = dev_new<unsigned char>(K.nrows);
-            rc->ent = dev_new<RowEntry>((size_t)count * width);
-            rc->ent32 = dev_new<RowEntry>((size_t)count * width);
-            rc->len = dev_new<int>(count);
-            if (!rc->code || !rc->ent || !rc->ent32 || !rc->len) rc.reset();
-        }
-        if (rc) {
-            hipLaunchKernelGGL(k_row_table, dim3(1), dim3(256), 0, st, S, w, width, rc->ent, rc->ent32, rc->len);
-            LAUNCH_CHECK();
-            hipLaunchKernelGGL(k_code_rows, dim3(g), dim3(256), 0, st, S, w, width, rc->ent, rc->len, rc->code);
-            LAUNCH_CHECK();
-            counts(count, bad);
-            if (bad) rc.reset();
-        }
-    } catch (...) {
-        (void)hipFree(w);
-        throw;
-    }
-    (void)hipFree(w);
+    auto rc = std::make_shared<RowCode>();
+    const size_t ent_bytes = sizeof(RowEntry) * ROWCODE_ENTRIES, len_bytes = sizeof(int) * ROWCODE_MAX;
+    rc->bytes = 2 * ent_bytes + len_bytes + sizeof(Work) + (size_t)K.nrows;
+    rc->mem = pool_try_alloc(rc->bytes);
+    if (!rc->mem) return nullptr;   // optional: without memory for it the products stay uncoded
+    char *p = (char *)rc->mem;
+    rc->ent = (RowEntry *)p;
+    rc->ent32 = (RowEntry *)(p += ent_bytes);
+    Work *w = (Work *)(p += ent_bytes);
+    rc->len = (int *)(p += sizeof(Work));
+    rc->code = (unsigned char *)(p + len_bytes);
+    rc->values = values;
+    rc->width = width;
+    const int g = vec_grid(K.nrows);
+    hipLaunchKernelGGL(k_zero_work, dim3(1), dim3(256), 0, st, w);
+    LAUNCH_CHECK();
+    // a sample of 4096 rows turns away most matrices that do not repeat
+    const long rows = K.nrows, step = std::max<long>(1, rows / 4096);
+    hipLaunchKernelGGL(k_find_rows, dim3(16), dim3(256), 0, st, S, (rows + step - 1) / step, step, w);
+    LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_find_rows, dim3(g), dim3(256), 0, st, S, rows, 1L, w);
+    LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_row_table, dim3(1), dim3(256), 0, st, S, w, width, rc->ent, rc->ent32, rc->len);
+    LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_code_rows, dim3(g), dim3(256), 0, st, S, w, width, rc->ent, rc->len, rc->code);
+    LAUNCH_CHECK();
+    int found[2];   // count, bad
+    HIP_TRY(hipMemcpyAsync(found, &w->count, sizeof found, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    if (found[1]) return nullptr;
+    rc->npat = found[0];
     return rc;
 }
 

@@ -29,15 +29,21 @@ struct RowCode {
     unsigned char *code = nullptr;   // nrows
     RowEntry *ent = nullptr, *ent32 = nullptr;
     int *len = nullptr;
+    void *mem = nullptr;   // holds them all, from the pool
+    size_t bytes = 0;
+    RowCode() = default;
+    RowCode(const RowCode &) = delete;
+    RowCode &operator=(const RowCode &) = delete;
     ~RowCode();
 };
 
 // The row code of K with the values of op (K's own without diagonal scaling),
 // or of K's column offsets alone; null when K is not of a coded form or has
-// more than ROWCODE_MAX distinct rows.  Two passes over the matrix.
+// more than ROWCODE_MAX distinct rows, or without memory for it.  Two passes
+// over the matrix and one wait.
 std::shared_ptr<RowCode> make_rowcode(const Operator &op, bool values, hipStream_t st);
 
-// The code that the products of op use, or null: built by op_prepare.  One of
+// The code that the products of op use, or null: built by op_prepare_solve.  One of
 // offsets alone only with 'offsets' (block products and FP32 values have no
 // kernel for it).
 const RowCode *op_rowcode(const Operator &op, bool offsets);
