@@ -804,7 +804,7 @@ int idrs_user_matrix_set_group(idrs_user_matrix_t K, int group) {
         DevMatrix &M = *K->M;
         if (M.fmt != DevFmt::CRS) return;
         if (group == 1 && !M.sell) build_sell(M, lib_stream());
-        if (group != 1) M.sell.reset();
+        if (group != 1) drop_sell(M);
         M.group = group;
     });
 }

@@ -1029,6 +1029,12 @@ void build_sell(DevMatrix &K, hipStream_t st) {
     K.sell = std::move(S);
 }
 
+void drop_sell(DevMatrix &K) {
+    K.sell.reset();
+    K.rowcode.drop(K.values_set);
+    K.offcode.drop(false);
+}
+
 bool op_prepared(const Operator &op) {
     const DevMatrix &K = *op.K;
     const bool sliced = K.fmt != DevFmt::CRS || !K.sell || !op.sval || op.sl_sval;
@@ -1125,7 +1131,7 @@ int autotune_group(DevMatrix &K, int reps, hipStream_t st, std::vector<std::pair
                 }
             }
             K.group = best;
-            if (best != 1) K.sell.reset();
+            if (best != 1) drop_sell(K);
         }
         // row slabs of a one-thread-per-row product
         if (K.fmt != DevFmt::CRS || K.group == 1) {

@@ -283,8 +283,9 @@ DevMatrix *make_dia(int nrows, int ncols, int ndiag, const int *offsets, const v
 // for one-thread-per-row products (DIA, the sliced copy) then the row-slab
 // count.  Returns the group; times: (group or -slabs, ms per product)
 int autotune_group(DevMatrix &K, int reps, hipStream_t st, std::vector<std::pair<int, float>> *times);
-// builds / drops K's sliced copy (group 1)
+// builds / drops K's sliced copy (group 1), with the row codes of its products
 void build_sell(DevMatrix &K, hipStream_t st);
+void drop_sell(DevMatrix &K);
 // makes the operator's sliced scaled values when K has a sliced copy; call
 // before products are captured into a graph
 void op_prepare(const Operator &op, hipStream_t st);

@@ -192,3 +192,20 @@ def test_complex_vectors_look_for_no_code(gpu):
     A = idrs_amd.Matrix(_matrix(n, offs, vals, "dia"))
     idrs_amd.idrs(A, _b(n, 3) + 0j, 4, maximum_iterations=3)
     assert A.rowcode()[0] is None
+
+
+def test_lanes_per_row_keep_no_code(gpu):
+    """A layout whose products cannot use the codes gives their memory back,
+    and going back to the sliced copy finds them again."""
+    n, offs, vals = _stencil((64, 33, 32), "star")
+    K = _matrix(n, offs, vals, "crs")
+    A = idrs_amd.Matrix(K)
+    b = _b(n, 3)
+    idrs_amd.idrs(A, b, 2, maximum_iterations=3)
+    assert A.rowcode() == ("values", 27)
+    idrs_amd.release_pool()
+    K.set_group(4)
+    assert A.rowcode() == (None, 0) and idrs_amd.release_pool() >= n     # a byte a row
+    K.set_group(1)
+    idrs_amd.idrs(A, b, 2, maximum_iterations=3)
+    assert A.rowcode() == ("values", 27)
