@@ -42,6 +42,16 @@ def _batch(systems, diag_precon=False, poly=None):
     return A, b
 
 
+# Batches whose systems all have at most 4096 rows run each in one workgroup;
+# with one larger system every system runs on the tile kernels.
+LARGER = [(65, 20.0, 0.9)]
+PATHS = pytest.mark.parametrize("path", ["workgroup", "tiles"])
+
+
+def _more(specs, path):
+    return specs + (LARGER if path == "tiles" else [])
+
+
 SPECS = [(5, 1.0, 0.3), (9, 30.0, 1.1), (17, 5.0, 2.0), (33, 80.0, 4.0), (40, 12.0, 5.5), (12, 60.0, 0.7)]
 
 
@@ -58,12 +68,14 @@ def test_batch_partition(gpu):
         assert np.allclose(w[row0[k]:row0[k + 1]], c.matvec(v[row0[k]:row0[k + 1]]), rtol=1e-13, atol=1e-10)
 
 
+@PATHS
 @pytest.mark.parametrize("s,variant", [(2, 1), (4, 1), (1, 2)])
-def test_batch_matches_single_solves(gpu, s, variant):
-    systems = _systems(SPECS)
+def test_batch_matches_single_solves(gpu, s, variant, path):
+    systems = _systems(_more(SPECS, path))
     A, b = _batch(systems)
     _, row0 = idrs_amd.batch_info(A.K)
     r = idrs_amd.idrs_batched(A, b, s, tolerance=1e-8, maximum_iterations=3000, variant=variant)
+    assert idrs_amd.last_solve_path() == path
     for k, (c, bb) in enumerate(systems):
         Ao = oracle_crs(c)
         xo, fo, ro, io, _ = orc.idrs(Ao, bb, s, tolerance=1e-8, maximum_iterations=3000, variant=variant)
@@ -95,14 +107,16 @@ def test_batch_matches_single_solves(gpu, s, variant):
             assert d < max(1e-10, 100 * dx), (k, d, dx)
 
 
-def test_batch_chebyshev_and_scaling(gpu):
+@PATHS
+def test_batch_chebyshev_and_scaling(gpu, path):
     """Diagonal scaling and a Chebyshev polynomial on every system (the
     pp_idrs operator), against the oracle's per-system operator."""
-    systems = _systems(SPECS[:4], seed=3)
+    systems = _systems(_more(SPECS[:4], path), seed=3)
     poly = (2, 4, (0.15, 1.85))
     A, b = _batch(systems, diag_precon=True, poly=poly)
     _, row0 = idrs_amd.batch_info(A.K)
     g = idrs_amd.idrs_batched(A, b, 4, tolerance=0.0, maximum_iterations=10)
+    assert idrs_amd.last_solve_path() == path
     for k, (c, bb) in enumerate(systems):
         Ao = oracle_crs(c, diag_precon=True, poly=poly)
 
@@ -119,16 +133,18 @@ def test_batch_chebyshev_and_scaling(gpu):
             assert d < max(1e-10, 100 * dx), (k, d, dx)
 
 
-def test_batch_x0_pt_raw_and_device(gpu):
+@PATHS
+def test_batch_x0_pt_raw_and_device(gpu, path):
     import torch
 
-    systems = _systems(SPECS[:3], seed=5)
+    systems = _systems(_more(SPECS[:3], path), seed=5)
     A, b = _batch(systems)
     _, row0 = idrs_amd.batch_info(A.K)
     rng = np.random.default_rng(6)
     x0 = rng.standard_normal(row0[-1])
     PT = rng.standard_normal((row0[-1], 2))
     h = idrs_amd.idrs_batched(A, b, 2, tolerance=0.0, maximum_iterations=9, x0=x0, PT_raw=PT)
+    assert idrs_amd.last_solve_path() == path
     for k, (c, bb) in enumerate(systems):
         sl = slice(row0[k], row0[k + 1])
         xo = orc.idrs(oracle_crs(c), bb, 2, tolerance=0.0, maximum_iterations=9, x0=x0[sl], PT_raw=PT[sl])[0]
@@ -139,13 +155,15 @@ def test_batch_x0_pt_raw_and_device(gpu):
     assert rel(d.x.cpu().numpy(), h.x) < 1e-14
 
 
-def test_batch_frozen_systems(gpu):
+@PATHS
+def test_batch_frozen_systems(gpu, path):
     """One easy and one hard system: the easy one stops at its own count and
     its solution stays what its own solve returns."""
-    systems = _systems([(6, 0.0, 0.0), (48, 90.0, 0.4)], seed=8)
+    systems = _systems([(6, 0.0, 0.0), (48 if path == "workgroup" else 66, 90.0, 0.4)], seed=8)
     A, b = _batch(systems)
     _, row0 = idrs_amd.batch_info(A.K)
     r = idrs_amd.idrs_batched(A, b, 2, tolerance=1e-10, maximum_iterations=4000)
+    assert idrs_amd.last_solve_path() == path
     its = []
     for k, (c, bb) in enumerate(systems):
         xo, fo, ro, io, _ = orc.idrs(oracle_crs(c), bb, 2, tolerance=1e-10, maximum_iterations=4000)
@@ -168,6 +186,7 @@ def test_batch_graph_replay_is_bit_identical(gpu, poly):
     kw = dict(tolerance=1e-9, maximum_iterations=3000)
     e = idrs_amd.idrs_batched(A, b, 2, graph=False, **kw)
     g = idrs_amd.idrs_batched(A, b, 2, graph=True, **kw)
+    assert idrs_amd.last_solve_path() == "tiles"
     print("iterations", sorted(set(e.iterations.tolist())))
     assert len(set(e.iterations.tolist())) >= 8
     assert np.array_equal(e.iterations, g.iterations) and np.array_equal(e.flag, g.flag)
@@ -177,14 +196,16 @@ def test_batch_graph_replay_is_bit_identical(gpu, poly):
     assert np.array_equal(e.x, g.x, equal_nan=True)
 
 
-def test_batch_sliced_copy(gpu):
+@PATHS
+def test_batch_sliced_copy(gpu, path):
     """The batch's tile product on the sliced-ELL copy (group 1; tiles start
     mid-slice at system boundaries) against each system's oracle solve."""
-    systems = _systems(SPECS)
+    systems = _systems(_more(SPECS, path))
     A, b = _batch(systems)
     A.K.set_group(1)
     _, row0 = idrs_amd.batch_info(A.K)
     r = idrs_amd.idrs_batched(A, b, 2, tolerance=1e-8, maximum_iterations=3000)
+    assert idrs_amd.last_solve_path() == path
     for k, (c, bb) in enumerate(systems):
         xo, fo, ro, io, _ = orc.idrs(oracle_crs(c), bb, 2, tolerance=1e-8, maximum_iterations=3000)
         assert r.flag[k] == fo == 0 and abs(r.iterations[k] - io) <= 2, (k, r.iterations[k], io)

@@ -52,7 +52,8 @@ def _box(dims):
 @pytest.mark.parametrize("n,s,form", [
     (1, 1, "crs"), (2, 1, "crs"), (63, 2, "dia"), (64, 4, "crs"), (65, 5, "crs"), (1023, 4, "dia"), (1024, 3, "crs"),
     (1025, 16, "crs"), (2047, 4, "complex"), (2049, 8, "dia"), (2560, 4, "crs"), (2561, 4, "crs"),
-    (1500, 4, "poly"), (1500, 4, "m1"), (700, 2, "x0"), (700, 1, "variant2"), (700, 1, "variant4")])
+    (1500, 4, "poly"), (1500, 4, "m1"), (700, 2, "x0"), (700, 1, "variant2"), (700, 1, "variant4"),
+    (700, 4, "variant3"), (700, 4, "variant4")])
 def test_small_solves_match_oracle(gpu, n, s, form):
     cplx = form == "complex"
     crs, (offs, vals) = _system(n, 3 + n, cplx)

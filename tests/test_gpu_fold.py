@@ -11,6 +11,8 @@ import numpy as np
 import pytest
 
 import idrs_amd
+import orc
+from helpers import gpu_crs, oracle_crs, rel
 from idrs_amd import _lib
 from idrs_amd import problems as P
 
@@ -94,6 +96,38 @@ def test_largest_folded_product_grid(gpu, n):
     K = idrs_amd.crs_format(n, n, crs.row_ptr, crs.col_ind, rval=crs.val)
     K.set_group(8)
     _same(idrs_amd.Matrix(K), _b(n, 4), 3, 0.0, 9, path="folded" if n <= 163840 else "launches")
+
+
+# complex vectors in each form of the solve, every shadow space and option,
+# against the oracle at a fixed count (1e-10, the bar of the other solves; the
+# Hessenberg matrix 1e-9 of its largest entry)
+@pytest.mark.parametrize("m,path", [(10, "workgroup"), (16, "folded"), (60, "launches")])
+@pytest.mark.parametrize("s,variant,extra", [(4, 1, "x0 U0"), (8, 1, "H"), (4, 1, "M1 omega"), (1, 2, "M1"), (1, 3, ""),
+                                             (1, 4, "x0"), (16, 1, "")])
+def test_complex_solves_match_oracle(gpu, m, path, s, variant, extra):
+    crs, _ = P.convection_diffusion_3d(m, 10.0, reaction=1.0)
+    crs.val = crs.val * (1.0 + 0.2j)
+    n, rng = crs.n, np.random.default_rng(s)
+    rand = lambda *shape: rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
+    A, Ao, b = gpu_crs(crs), oracle_crs(crs), rand(n)
+    kw = dict(tolerance=0.0, maximum_iterations=14, variant=variant)
+    okw = dict(kw)
+    if "x0" in extra:
+        kw["x0"] = okw["x0"] = rand(n)
+    if "U0" in extra:
+        kw["U0"] = okw["U0"] = rand(n, s)
+    if "omega" in extra:
+        kw["omega"] = okw["omega"] = np.array([0.9 + 0.1j, 1.1 - 0.2j])
+    if "M1" in extra:
+        kw["M1"], okw["M1"] = gpu_crs(crs, diag_precon=True), oracle_crs(crs, diag_precon=True)
+    if "H" in extra:
+        kw["H"] = okw["H_nritz"] = 13
+    g = idrs_amd.idrs(A, b, s, **kw)
+    assert idrs_amd.last_solve_path() == path
+    o = orc.idrs(Ao, b, s, **okw)
+    assert (g.flag, g.iterations) == (o[1], o[3]) and rel(g.x, o[0]) < 1e-10
+    if "H" in extra:
+        assert np.abs(g.H - o[5]).max() <= 1e-9 * np.abs(o[5]).max()
 
 
 @pytest.mark.parametrize("k", [1, 5, 6, 23, 24, 70])

@@ -134,8 +134,13 @@ def test_flags_forced_from_host(gpu):
     assert rc == idrs_amd._lib.IDRS_ERR_ARG
 
 
-def test_initial_search_space_and_x0(gpu):
-    crs, _ = P.convection_diffusion_3d(10, 5.0)
+# 10^3 rows: one workgroup, 16^3: the folded cycle
+SIDES = pytest.mark.parametrize("m,path", [(10, "workgroup"), (16, "folded")])
+
+
+@SIDES
+def test_initial_search_space_and_x0(gpu, m, path):
+    crs, _ = P.convection_diffusion_3d(m, 5.0)
     rng = np.random.default_rng(3)
     b = rng.standard_normal(crs.n)
     A, Ao = _pair(crs)
@@ -143,6 +148,7 @@ def test_initial_search_space_and_x0(gpu):
     x0 = rng.standard_normal(crs.n)
     PT = P.gaussian_shadow(crs.n, 3, seed=1)
     r = idrs_amd.idrs(A, b, 3, tolerance=1e-9, U0=U0, x0=x0, PT_raw=PT)
+    assert idrs_amd.last_solve_path() == path
     xo, fo, ro, io, _ = orc.idrs(Ao, b, 3, tolerance=1e-9, U0=U0, x0=x0, PT_raw=PT)
     assert r.flag == fo == 0 and abs(r.iterations - io) <= 2
     g = idrs_amd.idrs(A, b, 3, tolerance=0.0, maximum_iterations=15, U0=U0, x0=x0, PT_raw=PT)
@@ -150,15 +156,17 @@ def test_initial_search_space_and_x0(gpu):
     assert rel(g.x, o[0]) < 1e-10
 
 
-def test_m1_diagonal_preconditioner(gpu):
+@SIDES
+def test_m1_diagonal_preconditioner(gpu, m, path):
     """M1 present with a diagonal: t = om*(v/M1) branches (idrs.inc:169-190, 266-267)."""
-    crs, _ = P.convection_diffusion_3d(10, 20.0, reaction=2.0)
+    crs, _ = P.convection_diffusion_3d(m, 20.0, reaction=2.0)
     b = np.random.default_rng(4).standard_normal(crs.n)
     A, Ao = _pair(crs)
     M1 = gpu_crs(crs, diag_precon=True)
     M1o = oracle_crs(crs, diag_precon=True)
     PT = P.gaussian_shadow(crs.n, 2, seed=2)
     r = idrs_amd.idrs(A, b, 2, M1=M1, tolerance=1e-9, PT_raw=PT)
+    assert idrs_amd.last_solve_path() == path
     xo, fo, ro, io, _ = orc.idrs(Ao, b, 2, M1=M1o, tolerance=1e-9, PT_raw=PT)
     assert r.flag == fo == 0 and abs(r.iterations - io) <= 2
     g = idrs_amd.idrs(A, b, 2, M1=M1, tolerance=0.0, maximum_iterations=20, PT_raw=PT)

@@ -43,14 +43,17 @@ def _cosines(U, V):
     return np.linalg.svd(np.conj(Qu).T @ Qv)[1]
 
 
+# 8^3 and 10^3 rows: one workgroup, 15^3: the folded cycle (s > 16: launches)
+@pytest.mark.parametrize("side", [8, 15])
 @pytest.mark.parametrize("cplx", [False, True])
 @pytest.mark.parametrize("s,m", [(1, 12), (4, 23), (8, 30), (20, 50)])
-def test_hessenberg_matches_oracle(gpu, cplx, s, m):
-    crs = _cd3(cplx=cplx)
+def test_hessenberg_matches_oracle(gpu, cplx, s, m, side):
+    crs = _cd3(side, cplx=cplx)
     b = _rhs(crs.n, cplx, seed=s)
     nritz = (m // (s + 1)) * s + m % (s + 1)
     print(f"H s={s} its={m} nritz={nritz} complex={cplx}", flush=True)
     g = idrs_amd.idrs(gpu_crs(crs), b, s, tolerance=0.0, maximum_iterations=m, H=nritz + 3)
+    assert idrs_amd.last_solve_path() == ("launches" if s > 16 else "workgroup" if side == 8 else "folded")
     o = orc.idrs(oracle_crs(crs), b, s, tolerance=0.0, maximum_iterations=m, H_nritz=nritz + 3)
     assert g.iterations == o[3] == m
     assert rel(g.x, o[0]) < 1e-10
@@ -85,10 +88,11 @@ def test_hessenberg_finite_termination(gpu, cplx):
         assert np.min(np.abs(ritzv - v)) < 1e-7
 
 
+@pytest.mark.parametrize("side", [10, 15])
 @pytest.mark.parametrize("cplx", [False, True])
 @pytest.mark.parametrize("with_m", [False, True])
-def test_idrs_ritz_matches_oracle(gpu, cplx, with_m):
-    crs = _cd3(m=10, cplx=cplx)
+def test_idrs_ritz_matches_oracle(gpu, cplx, with_m, side):
+    crs = _cd3(m=side, cplx=cplx)
     n, s = crs.n, 4
     b = _rhs(n, cplx, seed=3)
     A, Ao = gpu_crs(crs), oracle_crs(crs)
@@ -157,13 +161,14 @@ def test_preconditioner_from_ritz_values(gpu, kind):
     assert abs(r.iterations - ro[3]) <= max(2, 0.05 * ro[3])
 
 
+@pytest.mark.parametrize("side", [10, 15])
 @pytest.mark.parametrize("cplx", [False, True])
-def test_recycle_space_solve(gpu, cplx):
+def test_recycle_space_solve(gpu, cplx, side):
     """PP_IDRS/recycle.inc: IDRS_RITZ returns U0(n, s); the next solve starts
     its first cycle from that search space (idrs.inc:55-65, 183-190).  The
     GPU's U0 drives both the GPU and the oracle solve (equal at a fixed
     count), and the recycled solve converges."""
-    crs = _cd3(m=10, cplx=cplx)
+    crs = _cd3(m=side, cplx=cplx)
     n, s = crs.n, 4
     A, Ao = gpu_crs(crs), oracle_crs(crs)
     g = idrs_amd.idrs_ritz(A, _rhs(n, cplx, seed=4), s, tolerance=1e-8, maximum_iterations=400, dim_u0=s)

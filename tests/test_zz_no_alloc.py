@@ -1,9 +1,10 @@
 """The allocation-free IDRS entry point (idrs_idrs_f64_noalloc) against the
 ordinary one (idrs_idrs_f64 with device pointers), through the C ABI.
 
-Both run the same kernels in the same order on the same grids, so their
-results must be bit-identical: x, the flag, the iteration count, relres and
-the residual history.  Two calls in a row share the scratch region, the
+Both do the same operations in the same order (the ordinary solve of a mid-size
+system runs the reductions and scalar steps inside the streaming kernels), so
+their results must be bit-identical: x, the flag, the iteration count, relres
+and the residual history.  Two calls in a row share the scratch region, the
 second with a smaller system, so what the first left behind must not leak
 into the second.  A system whose workspace exceeds the region is refused
 with an argument error before anything runs.
