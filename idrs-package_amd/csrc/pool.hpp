@@ -26,15 +26,15 @@ public:
     BufferPool(const BufferPool &) = delete;
     BufferPool &operator=(const BufferPool &) = delete;
 
-    // a buffer of exactly 'bytes', an idle one (the last given back) or a new
-    // one; null: out of memory
+    // a buffer of exactly 'bytes', an idle one (the longest idle of that size)
+    // or a new one; null: out of memory
     void *take(size_t bytes) {
         {
             std::lock_guard<std::mutex> g(mu);
             auto it = by_size.find(bytes);
             if (it != by_size.end()) {
-                std::list<Idle>::iterator e = it->second.back();
-                it->second.pop_back();
+                std::list<Idle>::iterator e = it->second.front();
+                it->second.pop_front();
                 if (it->second.empty()) by_size.erase(it);
                 void *p = e->p;
                 kept_ -= bytes;

@@ -38,12 +38,12 @@ static void put(void *p) {
     } while (0)
 
 int main() {
-    {   // a size comes back, the one given last first; never more than the cap
+    {   // a size comes back, the one given first first; never more than the cap
         BufferPool p({get, put}, 1000);
         void *a = p.take(100), *b = p.take(100);
         p.give(a, 100);
         p.give(b, 100);
-        CHECK(p.take(100) == b && p.take(100) == a && g_allocs == 2);
+        CHECK(p.take(100) == a && p.take(100) == b && g_allocs == 2);
         p.give(a, 100);
         p.give(b, 100);
         void *big = p.take(1001);
