@@ -559,13 +559,12 @@ __global__ void k_fold_init(const State<T> *st, Slot<T> *sl) {
 // the sums of reduce_partials, bit for bit, by 256 threads (nparts <=
 // FOLD_PARTS): a wavefront takes the shares of wavefronts wid, wid + 4, ... of
 // the 1024-thread kernel, four values at a time with all their loads in
-// flight.  scr: nv * 16 values.  No barrier at the end.  A solve that has
-// finished (info >= 0, known by the time the first values are) skips the rest.
+// flight.  scr: nv * 16 values.  No barrier at the end.
 template <class T>
-__device__ inline void fold_sums(const T *__restrict__ partials, int nparts, int nv, T *scr, int info) {
+__device__ inline void fold_sums(const T *__restrict__ partials, int nparts, int nv, T *scr) {
     constexpr int NW = FIN_THREADS / WAVE, NR = 256 / WAVE, V = NW / NR;
     const int lane = threadIdx.x % WAVE, wid = threadIdx.x / WAVE;
-    for (int q0 = 0; q0 < nv && (q0 == 0 || info < 0); q0 += 4) {
+    for (int q0 = 0; q0 < nv; q0 += 4) {
         T a[V][4];
 #pragma unroll
         for (int j = 0; j < V; j++)
@@ -629,7 +628,7 @@ __global__ __launch_bounds__(256) void k_form_u_fold(long n, int prow, const Slo
     __shared__ Slot<T> sl;
     __shared__ T scr[(FIN_S + 1) * (FIN_THREADS / WAVE)], red[FIN_S + 1];
     fold_load(in, &sl);
-    if (npin) fold_sums(pin, npin, 1 + prow, scr, in->info);
+    if (npin) fold_sums(pin, npin, 1 + prow, scr);
     __syncthreads();
     if (threadIdx.x < WAVE && npin && sl.info < 0) {
         if (threadIdx.x <= prow) red[threadIdx.x] = fold_value(scr, threadIdx.x);
@@ -684,8 +683,8 @@ __global__ __launch_bounds__(256) void k_orth_fold(long n, int k, int s, int pro
             ui[i] = want ? U[(long)i * n + q] : T(0);
         }
     }
-    fold_sums(pmu, npmu, prow, scr, in->info);
-    if (npn) fold_sums(pn, npn, 1, scr + prow * (FIN_THREADS / WAVE), in->info);
+    fold_sums(pmu, npmu, prow, scr);
+    if (npn) fold_sums(pn, npn, 1, scr + prow * (FIN_THREADS / WAVE));
     __syncthreads();
     if (threadIdx.x < WAVE && sl.info < 0) {
         if (blockIdx.x != 0 && threadIdx.x == 0) sl.H = nullptr;
@@ -779,8 +778,8 @@ __global__ __launch_bounds__(256) void k_omega_fold(long n, const Slot<T> *in, S
     __shared__ Slot<T> sl;
     __shared__ T scr[4 * (FIN_THREADS / WAVE)], red[4], lds[(NV + 1) * 4];
     fold_load(in, &sl);
-    fold_sums(pom, npom, 3, scr, in->info);
-    fold_sums(pn, npn, 1, scr + 3 * (FIN_THREADS / WAVE), in->info);
+    fold_sums(pom, npom, 3, scr);
+    fold_sums(pn, npn, 1, scr + 3 * (FIN_THREADS / WAVE));
     __syncthreads();
     if (threadIdx.x < WAVE && sl.info < 0) {
         if (threadIdx.x < 4) red[threadIdx.x] = fold_value(scr, threadIdx.x);
@@ -1359,7 +1358,10 @@ int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOp
     int h_local[2] = {-1, -1};
     int *h_info = ar ? h_local : lres.r.h_info;
     hipEvent_t pe[2] = {lres.r.pe[0], lres.r.pe[1]};
-    long max_cycles = cap_it / (s + 1) + 2;
+    // a cycle is s + 1 steps, so a limit on the steps is one on the cycles (the
+    // device stops at it): none is launched beyond (131 072 rows, DIA, IDR(4):
+    // 5 steps 373 -> 248 us, 20 steps 633 -> 527)
+    const long max_cycles = maxit > 0 ? (cap_it + s) / (s + 1) : cap_it / (s + 1) + 2;
     // Small systems are bound by the host's launch rate (~55 launches per
     // cycle): capture one cycle in a HIP graph and replay it -- the same
     // kernels with the same arguments in the same order.  Not while timing
@@ -1385,14 +1387,15 @@ int idrs_solve(const Operator &A, long n, int s, const T *b, T *x, const SolveOp
     try {
         for (long c = 0; c < max_cycles && !done; c++) {
             // the first folded cycle differs from the others in an argument:
-            // it runs as launches, while the host captures the others; a
-            // solve that has ended with it needs no second (IDR(4), DIA,
-            // 131 072 rows, 5 steps 373 -> 260 us)
+            // it runs as launches, while the host captures the others; one
+            // that has ended the solve meanwhile needs no second
             if (use_graph && !gexec && (c > 0 || !fold)) {
                 capture();
                 if (c > 0) {
-                    HIP_TRY(hipEventSynchronize(pe[(c - 1) % 2]));
-                    if (h_info[(c - 1) % 2] >= 0) break;
+                    const hipError_t q = hipEventQuery(pe[(c - 1) % 2]);
+                    if (q == hipSuccess && h_info[(c - 1) % 2] >= 0) break;
+                    if (q == hipErrorNotReady) (void)hipGetLastError();
+                    else HIP_TRY(q);
                 }
             }
             if (gexec) HIP_TRY(hipGraphLaunch(gexec, stream));
