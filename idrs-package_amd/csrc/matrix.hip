@@ -366,7 +366,9 @@ static SpmvArgs<VT, T> base_args(const DevMatrix &K, const VT *val) {
 // is read non-temporally, so that it does not push out the gathered vector.
 // A chain of DIA products per step, cached against non-temporal: 100^3
 // 11.6 / 14.8 us, 128^3 21.1 / 26.5, 160^3 (295 MB) 45.6 / 49.6, 200^3
-// (576 MB) 116 / 96.
+// (576 MB) 116 / 96.  The count takes a sliced copy with its padding, which is
+// not read, and the rows of P of the product at hand, so near the line the
+// P^T y product of a matrix can stream what its omega product keeps.
 constexpr size_t KEEP_BYTES = size_t(240) << 20;
 template <class VT, class T>
 static void set_keep(const Operator &op, SpmvArgs<VT, T> &A, int epi, const EpiArgs<T> &E) {

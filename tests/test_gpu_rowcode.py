@@ -123,15 +123,16 @@ def _matrix(n, offs, vals, fmt):
 
 
 # every width the kernels are compiled for (3, 5, 7 and any: 9, 27), every
-# shadow width of the P^T y epilogue, with and without a seed shift
+# shadow width of the P^T y epilogue, with and without a seed shift (s = 8:
+# scaled values, whose shift is divided by the diagonal)
 @pytest.mark.parametrize("shape,reach", [((40000,), "star"), ((211, 190), "star"), ((34, 33, 32), "star"),
                                          ((211, 190), "box"), ((34, 33, 32), "box")])
 @pytest.mark.parametrize("fmt", ["dia", "crs"])
-@pytest.mark.parametrize("s,variant,seed", [(1, 1, 0.0), (2, 1, 0.0), (4, 1, 0.3), (8, 1, 0.0), (16, 1, 0.0),
-                                            (1, 2, 0.0)])
+@pytest.mark.parametrize("s,variant,seed", [(1, 1, 0.0), (2, 1, 0.0), (4, 1, 0.3), (8, 1, 0.0), (8, 1, 0.3),
+                                            (16, 1, 0.0), (1, 2, 0.0)])
 def test_coded_solves_are_the_same_bits(gpu, shape, reach, fmt, s, variant, seed):
     n, offs, vals = _stencil(shape, reach)
-    A = idrs_amd.Matrix(_matrix(n, offs, vals, fmt))
+    A = idrs_amd.Matrix(_matrix(n, offs, vals, fmt), which_precon=1 if s == 8 else 0)
     if seed:
         A.set_seed(seed)
     b, v = _b(n, 3), np.random.default_rng(2).uniform(-1, 1, n)
