@@ -798,11 +798,13 @@ def main():
         results = [step(True)]
         print(f"# {fmt} event-timed solve: spmv={results[0].spmv_ms:.1f} ms / {results[0].spmv_launches} launches",
               file=sys.stderr, flush=True)
-        # roofline of the SpMV kernel over the timed launches.  This
-        # workload's rows repeat (27 distinct ones), so a product that sums
-        # rows in stored order reads one byte a row for the matrix
-        coded = n >= 1 << 15 and (fmt == "dia" or group == 1)
-        mat_bytes = n if coded else 8 * nvals if fmt == "dia" else 12 * nnz + 4 * (n + 1)
+        # roofline of the SpMV kernel over the timed launches.  A coded
+        # product reads one byte a row for the matrix (values) or for its
+        # column indices (offsets)
+        code, distinct = A.rowcode()
+        coded = code is not None
+        mat_bytes = (n if code == "values" else 8 * nnz + n if code == "offsets"
+                     else 8 * nvals if fmt == "dia" else 12 * nnz + 4 * (n + 1))
         tot_bytes, launches = solve_spmv_bytes(n, nnz, s, d, last.iterations, s)
         tot_bytes = tot_bytes - launches * (12 * nnz + 4 * (n + 1)) + launches * mat_bytes
         spmv_ms = sum(r.spmv_ms for r in results) / len(results)
@@ -819,11 +821,12 @@ def main():
                 "peak": HBM_PEAK_GBS,
                 "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 4),
-                "traffic": None if coded else read_traffic(fmt),
+                # the committed counters are of the row-coded product
+                "traffic": read_traffic(fmt) if code == "values" else None,
                 "kernel": "k_spmv_pat" if coded else f"k_spmv_{fmt}",
                 "bytes_per_launch": round(tot_bytes / launches),
                 "stored_values": nvals, "implicit_unit_diagonal": unit, "lanes_per_row": group,
-                "row_slabs": row_slabs,
+                "row_slabs": row_slabs, "row_code": code, "distinct_rows": distinct,
                 "avg_launch_us": round(spmv_ms * 1e3 / launches, 2),
             },
             "solve_gbs_model": round(solve_gbs, 1),
