@@ -1048,7 +1048,7 @@ static void prepare_rowcode(const Operator &op, hipStream_t st) {
     std::lock_guard<std::mutex> g(K.code_mu);
     if (K.fmt == DevFmt::CRS && !(K.group == 1 && K.sell)) return;   // not read in that layout
     CodeSlot &slot = op.sval ? op.rowcode : K.rowcode;
-    if (!slot.tried && !(op.sval && K.tperm) && !K.values_set) slot.set(make_rowcode(op, true, st));
+    if (!slot.tried && !(op.sval && K.tperm)) slot.set(make_rowcode(op, true, st));
     if (!slot.get() && !K.offcode.tried) K.offcode.set(make_rowcode(op, false, st));
 }
 
@@ -1281,6 +1281,13 @@ long Operator::stored_values() const {
 // the product.
 static void op_scale_values(Operator &op, bool cdiag, hipStream_t st);
 
+// New scaled values: the code of the old ones goes, and the next solve looks
+// for another -- not where K's values were replaced and the last search found
+// none, as every refresh would then pay for one.
+static void drop_scaled_code(Operator &op) {
+    op.rowcode.drop(op.K->values_set && op.rowcode.tried && !op.rowcode.get());
+}
+
 void op_set_diag_precon(Operator &op, int which, const std::complex<double> *shift) {
     hipStream_t st = lib_stream();
     DevMatrix &K = *op.K;
@@ -1290,7 +1297,7 @@ void op_set_diag_precon(Operator &op, int which, const std::complex<double> *shi
     (void)hipFree(op.sl_sval);
     (void)hipFree(op.sl_sval32);
     op.pdiag = op.sval = op.sval32 = nullptr;
-    op.rowcode.drop(false);
+    drop_scaled_code(op);
     op.sl_sval = op.sl_sval32 = nullptr;
     op.unit_diag = -1;
     op.which_precon = which;
@@ -1373,7 +1380,7 @@ void op_set_diag_values(Operator &op, const std::vector<std::complex<double>> &d
     (void)hipFree(op.sl_sval);
     (void)hipFree(op.sl_sval32);
     op.pdiag = op.sval = op.sval32 = nullptr;
-    op.rowcode.drop(false);
+    drop_scaled_code(op);
     op.sl_sval = op.sl_sval32 = nullptr;
     op.unit_diag = -1;
     op.which_precon = 1;

@@ -126,7 +126,7 @@ struct DevMatrix {
     mutable CodeSlot rowcode, offcode;
     mutable std::mutex code_mu;
     // the values have been replaced since the upload: more will follow, and
-    // the values are not coded any more (scaled ones neither)
+    // K's own are not coded any more (scaled ones: drop_scaled_code)
     bool values_set = false;
     ~DevMatrix();
 };

@@ -167,22 +167,38 @@ def test_new_values_drop_the_code(gpu, scaled):
     if scaled:
         A.set_precon(1)
     x = idrs_amd.idrs(A, b, 4, tolerance=0.0, maximum_iterations=5).x
-    assert A.rowcode() == ("offsets", 27)
+    # a scaled operator looks again while it finds a code
+    assert A.rowcode() == ("values" if scaled else "offsets", 27)
     R = idrs_amd.Matrix(_matrix(n, offs, 2.0 * vals, "crs"), which_precon=1 if scaled else 0)
     assert np.array_equal(idrs_amd.idrs(R, b, 4, tolerance=0.0, maximum_iterations=5).x.cpu(), x.cpu())
     assert R.rowcode() == ("values", 27) and np.array_equal(A * v, R * v)
+    # values that do not repeat, and then constant ones again: no more searches
+    varied = vals * np.random.default_rng(5).uniform(1, 2, n)[:, None]
+    for new in (varied, vals):
+        _set_values(K, new[vals != 0])
+        if scaled:
+            A.set_precon(1)
+        x = idrs_amd.idrs(A, b, 4, tolerance=0.0, maximum_iterations=5).x
+        assert A.rowcode() == ("offsets", 27)
+        R = idrs_amd.Matrix(_matrix(n, offs, new, "crs"), which_precon=1 if scaled else 0)
+        assert np.array_equal(idrs_amd.idrs(R, b, 4, tolerance=0.0, maximum_iterations=5).x.cpu(), x.cpu())
 
 
 @pytest.mark.parametrize("scaled", [False, True])
 def test_coded_single_precision_values(gpu, scaled):
-    """The mixed solve's FP32-value products: coded, against a matrix whose
-    values were set once more (not coded in single precision)."""
+    """The mixed solve's FP32-value products: coded, against a matrix that
+    holds the same values after others in which no code was found (its
+    offsets, coded, serve FP64 values only)."""
     n, offs, vals = _stencil((34, 33, 32), "star")
     vals = vals / 3.0
     K, K1 = _matrix(n, offs, vals, "crs"), _matrix(n, offs, vals, "crs")
-    _set_values(K1, vals[vals != 0])
     b = np.random.default_rng(4).uniform(-1, 1, n)
     A, A1 = (idrs_amd.Matrix(k, which_precon=1 if scaled else 0) for k in (K, K1))
+    for new in (vals * np.random.default_rng(5).uniform(1, 2, n)[:, None], vals):
+        _set_values(K1, new[vals != 0])
+        if scaled:
+            A1.set_precon(1)
+        idrs_amd.idrs(A1, b, 4, maximum_iterations=1)
     x, x1 = (idrs_amd.idrs_mixed(a, b, 4, tolerance=1e-9) for a in (A, A1))
     assert A.rowcode() == ("values", 27) and A1.rowcode() == ("offsets", 27)
     assert x.flag == 0 and (x.iterations, x.outer) == (x1.iterations, x1.outer) and np.array_equal(x.x, x1.x)
