@@ -553,7 +553,7 @@ static int matvec_entry(idrs_matrix_t A, const double *v, double *w, int what) {
     return guarded([&] {
         need(A && v && w, "null argument");
         hipStream_t st = lib_stream();
-        op_prepare(A->op, st);
+        op_prepare_products<T>(A->op, what == 1 ? 0 : A->op.degree + 1L, st);
         long n = A->op.rows();
         DVec<T> dv((const T *)v, n, st), dw(n), w1(n), w2(n), w3(n);
         EpiArgs<T> none{};
@@ -572,7 +572,7 @@ static int matvec_block_entry(idrs_matrix_t A, int ncols, const double *V, doubl
         need(A->op.K->nrows == A->op.K->ncols, "block products need a square matrix");
         const long rows = A->op.rows();
         hipStream_t st = lib_stream();
-        op_prepare(A->op, st);
+        op_prepare_products<T>(A->op, ncols * (A->op.degree + 1L), st);
         const size_t cnt = (size_t)rows * ncols;
         DVec<T> dv((const T *)V, cnt, st), dw(cnt), w1(cnt), w2(cnt);
         op_apply_cols<T>(A->op, ncols, rows, dv.p, dw.p, w1.p, w2.p, st);
@@ -587,7 +587,7 @@ static int ms_scaleback_entry(idrs_matrix_t A, int ns, int degree, const double 
         need(A && alpha_s && Y && X, "null argument");
         need(ns >= 1 && degree >= 0, "bad arguments");
         hipStream_t st = lib_stream();
-        op_prepare(A->op, st);
+        op_prepare_products<T>(A->op, (long)ns * degree, st);
         const long n = A->op.rows();
         // blocks of up to 8 shifts share each product's read of the matrix
         const int nb = std::min(ns, SPMV_COLS);

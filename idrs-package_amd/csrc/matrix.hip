@@ -1060,6 +1060,14 @@ void op_prepare_solve(const Operator &op, hipStream_t st) {
 template void op_prepare_solve<double>(const Operator &, hipStream_t);
 template void op_prepare_solve<c128>(const Operator &, hipStream_t);
 
+template <class T>
+void op_prepare_products(const Operator &op, long products, hipStream_t st) {
+    if (std::is_same<T, double>::value && (op.K->products += products) >= 64) op_prepare_solve<T>(op, st);
+    else op_prepare(op, st);
+}
+template void op_prepare_products<double>(const Operator &, long, hipStream_t);
+template void op_prepare_products<c128>(const Operator &, long, hipStream_t);
+
 void op_prepare(const Operator &op, hipStream_t st) {
     if (op_prepared(op)) return;
     const DevMatrix &K = *op.K;

@@ -125,6 +125,7 @@ struct DevMatrix {
     // the sliced layout), made by op_prepare_solve
     mutable CodeSlot rowcode, offcode;
     mutable std::mutex code_mu;
+    mutable std::atomic<long> products{0};   // asked for outside solves
     // the values have been replaced since the upload: more will follow, and
     // K's own are not coded any more (scaled ones: drop_scaled_code)
     bool values_set = false;
@@ -293,9 +294,12 @@ void op_prepare(const Operator &op, hipStream_t st);
 bool op_prepared(const Operator &op);
 // op_prepare, and for a solve's products of real vectors the row code of the
 // values they read, looked for once per matrix (scaled values: per operator).
-// A single product does not look: the search takes as long as several.
+// A single product does not look, as the search takes as long as several; the
+// product entries count theirs and look at the 64th of a matrix.
 template <class T>
 void op_prepare_solve(const Operator &op, hipStream_t st);
+template <class T>
+void op_prepare_products(const Operator &op, long products, hipStream_t st);
 // block-diagonal CRS matrix of nsys square CRS systems (copies), with its
 // Partition
 DevMatrix *make_blockdiag(int nsys, const DevMatrix *const *Ks);

@@ -3,7 +3,7 @@ against the uncoded products of the same matrices, bit for bit: the same
 operations on the same values in the same order.  A solve looks for the code,
 a product alone does not, so that an operator's products before its first
 solve, and the allocation-free solve, which builds nothing, are the uncoded
-ones.
+ones (many products look too).
 """
 import ctypes
 
@@ -202,6 +202,17 @@ def test_coded_single_precision_values(gpu, scaled):
     x, x1 = (idrs_amd.idrs_mixed(a, b, 4, tolerance=1e-9) for a in (A, A1))
     assert A.rowcode() == ("values", 27) and A1.rowcode() == ("offsets", 27)
     assert x.flag == 0 and (x.iterations, x.outer) == (x1.iterations, x1.outer) and np.array_equal(x.x, x1.x)
+
+
+def test_many_products_look_for_a_code(gpu):
+    n, offs, vals = _stencil((34, 33, 32), "star")
+    A = idrs_amd.Matrix(_matrix(n, offs, vals, "dia"))
+    V = np.random.default_rng(2).uniform(-1, 1, (n, 21))
+    before = A * V
+    for _ in range(2):
+        assert np.array_equal(A * V, before) and A.rowcode()[0] is None      # 42, 63 products
+    assert np.array_equal(A * V[:, 0], before[:, 0]) and A.rowcode() == ("values", 27)
+    assert np.array_equal(A * V, before)
 
 
 def test_complex_vectors_look_for_no_code(gpu):
